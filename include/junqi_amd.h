@@ -348,21 +348,18 @@ int jq_history_snapshot(jq_history *hist, jq_env *env, const int8_t *acting, int
  * the observer seat as mask_words (device int32 (batch, 521)) and/or mask_bool
  * (device uint8 (batch, 16641)); any output may be NULL. Rows outside
  * [0, num_steps * num_envs) are rebuilt from the empty terminated state.
- * (DeviceRolloutHistory::reconstruct, rollout_history.cu:289-523.) Internal
- * scratch of `batch` rows is kept between calls (grown when needed), so calls
- * on one history must not overlap on different streams. */
+ * (DeviceRolloutHistory::reconstruct, rollout_history.cu:289-523.) The rows are
+ * read in place: no scratch, no allocation. */
 int jq_history_reconstruct(jq_history *hist, const int64_t *flat, const int8_t *observer, int32_t batch, int32_t fmt,
                            void *spatial, void *aux, float *global, int32_t *mask_words, uint8_t *mask_bool,
                            void *stream);
 
-/* The same rebuild with no device allocation: for callers that cannot allocate
- * (code under HIP graph capture, serving loops, harnesses that forbid
- * hipMalloc). No counterpart in the reference. The rebuilt rows live in one
- * file-scope device array of the library, JQ_NOALLOC_MAX_ROWS rows (21.45 MB,
- * held on each device the library runs on until the process ends), shared by
- * every call on that device: calls that overlap on one device race, so keep
- * them on one stream or serialise them. batch > JQ_NOALLOC_MAX_ROWS returns
- * JQ_E_ARG; split larger minibatches. Outputs equal jq_history_reconstruct's. */
+/* The same rebuild for callers that cannot allocate (code under HIP graph
+ * capture, serving loops, harnesses that forbid hipMalloc), at most
+ * JQ_NOALLOC_MAX_ROWS rows a call. No counterpart in the reference. Neither
+ * rebuild allocates or keeps device memory, so calls may overlap on different
+ * streams. batch > JQ_NOALLOC_MAX_ROWS returns JQ_E_ARG; split larger
+ * minibatches. Outputs equal jq_history_reconstruct's. */
 #define JQ_NOALLOC_MAX_ROWS 1024
 int jq_history_reconstruct_noalloc(jq_history *hist, const int64_t *flat, const int8_t *observer, int32_t batch,
                                    int32_t fmt, void *spatial, void *aux, float *global, int32_t *mask_words,

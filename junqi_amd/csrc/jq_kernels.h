@@ -896,10 +896,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) void
 }
 
 // ------------------------------------------------------------------ reset
-// Empty, terminated state of one env (no pieces, empty board, zero beliefs),
-// written by threads t of nt.
-__device__ __forceinline__ void clear_env(const State &S, int env, int t, int nt)
+// Empty, terminated state of every env (no pieces, empty board, zero beliefs),
+// before the first reset.
+__global__ __launch_bounds__(64) void k_clear(State S)
 {
+    const int env = blockIdx.x, t = threadIdx.x, nt = 64;
+    if (env >= S.n) return;
     for (int f = t; f < CELL_STRIDE; f += nt) S.cell[(size_t)env * CELL_STRIDE + f] = -1;
     PieceRec r;
     r.pos = r.zero = r.dstep = r.dloc = -1;
@@ -912,7 +914,7 @@ __device__ __forceinline__ void clear_env(const State &S, int env, int t, int nt
     for (int p = t; p < PID_STRIDE; p += nt) {
         S.piece[pc_idx(env, p)] = r;
         for (int o = 0; o < 4; ++o) {
-            if (S.cm) S.cm[cm_idx(env, o, p)] = c;   // a rebuild-only state keeps no full records
+            S.cm[cm_idx(env, o, p)] = c;
             S.cme[cm_idx(env, o, p)] = ce;
             S.cmk[cm_idx(env, o, p)] = 0;
             S.cmv[cm_idx(env, o, p)] = cv;
@@ -929,14 +931,6 @@ __device__ __forceinline__ void clear_env(const State &S, int env, int t, int nt
         S.lg[env].n = 0;
         S.lg[env].seat = 0;
     }
-}
-
-// Empty, terminated state for every env (before the first reset).
-__global__ __launch_bounds__(64) void k_clear(State S)
-{
-    const int env = blockIdx.x, l = threadIdx.x;
-    if (env >= S.n) return;
-    clear_env(S, env, l, 64);
 }
 
 // Start an env from a lineup (GameState.new_game, state.py:490-620; beliefs,
@@ -1095,7 +1089,10 @@ __global__ __launch_bounds__(64) void k_finalize(State S, int beliefs, const uin
 // ltype when given, else from the piece records.
 // lscr: LSCR_WORDS words of the wave's LDS, the compact source cells of the
 // movable pieces (words 0-2) and the engineers' rail destinations (3-11).
-__device__ __forceinline__ void legal_body(const State &S, int env, int l, int seat, bool off, const int8_t *cell, uint32_t *bits,
+// The masks go to row `row` (the env's own index, or the row of a minibatch
+// rebuilt from a history); REC: the legal record of the CSR pass is written.
+template <bool REC = true>
+__device__ __forceinline__ void legal_body(const State &S, int env, int row, int l, int seat, bool off, const int8_t *cell, uint32_t *bits,
                            const uint8_t *rotl, const int16_t *lpos, const int8_t *ltype, uint64_t *lscr,
                            int32_t *__restrict__ counts, int32_t *__restrict__ mask_words, uint8_t *__restrict__ mask_bool)
 {
@@ -1169,7 +1166,7 @@ __device__ __forceinline__ void legal_body(const State &S, int env, int l, int s
     }
     const int nmov = __popcll(__ballot(lead));
     const int total = wave_sum(lead ? cnt : 0);
-    if (lead) {
+    if (REC && lead) {
         LegalRec &G = S.lg[env];
         G.src[rank] = (int16_t)src;
         G.mask[rank][0] = m0; G.mask[rank][1] = m1; G.mask[rank][2] = m2;
@@ -1190,44 +1187,58 @@ __device__ __forceinline__ void legal_body(const State &S, int env, int l, int s
             }
         }
     }
-    if (l == 0) {
+    if (REC && l == 0) {
         S.lg[env].n = nmov;
         S.lg[env].seat = seat;
         if (counts) counts[env] = total;
     }
     wave_sync();
     if (mask_words)
-        for (int w = l; w < JQ_MASK_WORDS; w += 64) mask_words[(size_t)env * JQ_MASK_WORDS + w] = (int32_t)bits[w];
+        for (int w = l; w < JQ_MASK_WORDS; w += 64) mask_words[(size_t)row * JQ_MASK_WORDS + w] = (int32_t)bits[w];
     if (mask_bool) {
         __builtin_amdgcn_s_setprio(0);
-        uint8_t *row = mask_bool + (size_t)env * JQ_ACTION_DIM;
+        uint8_t *out = mask_bool + (size_t)row * JQ_ACTION_DIM;
         // bytes until the first 16-byte boundary, then whole 16-byte chunks, then the tail
-        const int mis = (int)((uintptr_t)row & 15);
+        const int mis = (int)((uintptr_t)out & 15);
         const int head = mis ? 16 - mis : 0;
-        for (int i = l; i < head; i += 64) row[i] = (bits[i >> 5] >> (i & 31)) & 1;
+        for (int i = l; i < head; i += 64) out[i] = (bits[i >> 5] >> (i & 31)) & 1;
         const int nchunks = (JQ_ACTION_DIM - head) / 16;
         for (int q = l; q < nchunks; q += 64) {
             const int i0 = head + q * 16;   // bits i0 .. i0 + 15 (word (i0 >> 5) + 1 <= 520)
             const uint32_t v = __builtin_amdgcn_alignbit(bits[(i0 >> 5) + 1], bits[i0 >> 5], i0 & 31);
-            *reinterpret_cast<uint4 *>(row + i0) =
+            *reinterpret_cast<uint4 *>(out + i0) =
                 make_uint4(nib_to_bytes(v), nib_to_bytes(v >> 4), nib_to_bytes(v >> 8), nib_to_bytes(v >> 12));
         }
-        for (int i = head + nchunks * 16 + l; i < JQ_ACTION_DIM; i += 64) row[i] = (bits[i >> 5] >> (i & 31)) & 1;
-    }}
+        for (int i = head + nchunks * 16 + l; i < JQ_ACTION_DIM; i += 64) out[i] = (bits[i >> 5] >> (i & 31)) & 1;
+    }
+}
 
+// HIST: block r takes row flat[r] of a rollout history (S = history_state) for
+// seat acting[r], and writes its masks as row r of the minibatch; flat values
+// outside [0, S.n) have no legal action. No counts or legal records then.
+template <bool HIST = false>
 __global__ __launch_bounds__(64) void k_legal(State S, const int8_t *__restrict__ acting,
                                               int32_t *__restrict__ counts, int32_t *__restrict__ mask_words,
-                                              uint8_t *__restrict__ mask_bool)
+                                              uint8_t *__restrict__ mask_bool,
+                                              const int64_t *__restrict__ flat = nullptr)
 {
-    const int env = blockIdx.x, l = threadIdx.x;
-    if (env >= S.n) return;
+    const int row = blockIdx.x, l = threadIdx.x;
+    int env = row;
+    bool stored = true;
+    if constexpr (HIST) {
+        const int64_t f = flat[row];
+        stored = f >= 0 && f < (int64_t)S.n;
+        env = stored ? (int)f : 0;
+    } else if (env >= S.n) {
+        return;
+    }
     __shared__ int8_t cell[CELL_STRIDE];
     __shared__ uint32_t bits[JQ_MASK_WORDS_PAD];
     __shared__ uint8_t rotl[NONB + 3];   // world compact -> canonical compact of the acting seat
     __shared__ uint64_t lscr[LSCR_WORDS];
     const EnvRec &E = S.env[env];
-    const int seat = acting ? acting[env] : E.turn;
-    const bool off = E.term || seat < 0 || seat > 3 || ((E.sdead >> (seat & 3)) & 1);
+    const int seat = acting ? acting[row] : E.turn;
+    const bool off = !stored || E.term || seat < 0 || seat > 3 || ((E.sdead >> (seat & 3)) & 1);
     for (int f = l; f < CELL_STRIDE; f += 64) cell[f] = f < NC ? S.cell[(size_t)env * CELL_STRIDE + f] : -1;
     // wave issue priority 2 through the legal pass, 0 for the bool rows'
     // stores (legal_body lowers it): a wave still computing gets issue slots
@@ -1240,7 +1251,7 @@ __global__ __launch_bounds__(64) void k_legal(State S, const int8_t *__restrict_
         for (int c = l; c < NONB; c += 64) rotl[c] = cT.rotc[s4][c];
     }
     __syncthreads();
-    legal_body(S, env, l, seat, off, cell, bits, rotl, nullptr, nullptr, lscr, counts, mask_words, mask_bool);
+    legal_body<!HIST>(S, env, row, l, seat, off, cell, bits, rotl, nullptr, nullptr, lscr, counts, mask_words, mask_bool);
 }
 
 // Exclusive scan of counts into offsets (N+1); one 1024-thread block walks the
@@ -1655,7 +1666,7 @@ __device__ __forceinline__ void env_step_wave(const State &S, int env, int l, co
         for (int c = l; c < NONB; c += 64) E.rotl[c] = cT.rotc[seat & 3][c];
     }
     wave_sync();
-    legal_body(S, env, l, seat, off, E.cell, E.bits, E.rotl, E.pos, E.ptype, E.lscr, A.counts, A.mask_words,
+    legal_body(S, env, env, l, seat, off, E.cell, E.bits, E.rotl, E.pos, E.ptype, E.lscr, A.counts, A.mask_words,
                nullptr);
     if (l == 0) write_step_res(A.O, env, E.res);   // the step's reports go out last
 }

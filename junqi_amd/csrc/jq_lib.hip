@@ -45,13 +45,12 @@ struct jq_env {
 // Rollout history: per-step copies of every per-env state block.
 struct jq_history {
     int device = 0;
-    int32_t show_mode = 0, max_moves = 0;
+    int32_t show_mode = 0;
     HistState H{};
     std::vector<void *> allocs;
     float *rlut = nullptr;           // recency table copied from the snapshotted handle
     bool rlut_ready = false;
-    jq_env *replay = nullptr;        // scratch state of the rebuilt rows
-    int32_t replay_cap = 0;
+    int obs_f32_pad = -1;            // as jq_env's, for the rebuilding kernel
 };
 
 namespace {
@@ -286,28 +285,29 @@ int obs_u8_grid(jq_env *e)
 // rounds up (a pad that left only 0.9 % of slack under the third was rounded
 // past it: 2 blocks per CU, 3.06 ms). 0 when the occupancy query does not
 // confirm exactly 3.
-int obs_f32_pad(jq_env *e, int &pad)
+template <class Kernel>
+int obs_f32_pad(Kernel kernel, int device, int &cache, int &pad)
 {
-    if (e->obs_f32_pad < 0) {
+    if (cache < 0) {
         hipFuncAttributes fa{};
         int lds_cu = 0, per_cu = 0;
-        HIP_TRY(hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(&k_observe<0, false>)));
-        HIP_TRY(hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, e->device));
+        HIP_TRY(hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(kernel)));
+        HIP_TRY(hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, device));
         int p = (lds_cu / 3 + lds_cu / 4) / 2 - (int)fa.sharedSizeBytes;
         if (p > 0) {
-            HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_observe<0, false>, OBS_THREADS, p));
+            HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, OBS_THREADS, p));
             if (per_cu != 3) p = 0;
         } else {
             p = 0;
         }
-        e->obs_f32_pad = p;
+        cache = p;
     }
-    pad = e->obs_f32_pad;
+    pad = cache;
     return JQ_OK;
 }
 
 // The checks of an observation request (format, buffers, tables it needs).
-int obs_args(const jq_env *e, int32_t fmt, const void *spatial, const void *aux, const float *global)
+int obs_args(bool rlut_ready, bool ext_on, int32_t fmt, const void *spatial, const void *aux, const float *global)
 {
     if (!spatial) return fail(JQ_E_ARG, "null spatial output");
     if (fmt < JQ_OBS_F32 || fmt > JQ_OBS_U8) return fail(JQ_E_ARG, "bad observation format %d", fmt);
@@ -316,8 +316,8 @@ int obs_args(const jq_env *e, int32_t fmt, const void *spatial, const void *aux,
         return fail(JQ_E_ARG, "observation buffers must be aligned to their element size");
     if (aux && fmt != JQ_OBS_U8) return fail(JQ_E_ARG, "aux rows belong to the u8 format only");
     if (aux && (uintptr_t)aux % 16) return fail(JQ_E_ARG, "u8 aux rows must be 16-byte aligned");
-    if ((fmt != JQ_OBS_U8 || aux) && !e->rlut_ready) return fail(JQ_E_STATE, "recency table not uploaded");
-    if (e->ext_on && fmt == JQ_OBS_U8)
+    if ((fmt != JQ_OBS_U8 || aux) && !rlut_ready) return fail(JQ_E_STATE, "recency table not uploaded");
+    if (ext_on && fmt == JQ_OBS_U8)
         return fail(JQ_E_STATE, "uploaded beliefs are arbitrary floats: observe them as JQ_OBS_F32 or JQ_OBS_BF16");
     return JQ_OK;
 }
@@ -558,7 +558,8 @@ int jq_legal(jq_env *e, const int8_t *acting, int32_t *counts, int32_t *offsets,
     if ((offsets || values) && !counts) return fail(JQ_E_ARG, "offsets/values need counts");
     if (values && !offsets) return fail(JQ_E_ARG, "values need offsets");
     if (values && values_capacity < 0) return fail(JQ_E_ARG, "negative values capacity");
-    hipLaunchKernelGGL(k_legal, dim3(e->S.n), dim3(64), 0, strm(stream), e->S, acting, counts, mask_words, mask_bool);
+    hipLaunchKernelGGL(k_legal<>, dim3(e->S.n), dim3(64), 0, strm(stream), e->S, acting, counts, mask_words, mask_bool,
+                       nullptr);
     if ((rc = launch_check("k_legal")) != 0) return rc;
     if (offsets) {
         hipLaunchKernelGGL(k_scan, dim3(1), dim3(SCAN_THREADS), 0, strm(stream), counts, offsets, e->S.n);
@@ -579,7 +580,8 @@ int jq_legal_slots(jq_env *e, const int8_t *acting, uint8_t *slots, void *stream
     if (rc) return rc;
     if (!slots) return fail(JQ_E_ARG, "null slot mask");
     if ((uintptr_t)slots % 16) return fail(JQ_E_ARG, "slot mask must be 16-byte aligned");
-    hipLaunchKernelGGL(k_legal, dim3(e->S.n), dim3(64), 0, strm(stream), e->S, acting, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL(k_legal<>, dim3(e->S.n), dim3(64), 0, strm(stream), e->S, acting, nullptr, nullptr, nullptr,
+                       nullptr);
     if ((rc = launch_check("k_legal")) != 0) return rc;
     hipLaunchKernelGGL(k_slots, dim3(e->S.n), dim3(64), 0, strm(stream), e->S, slots);
     return launch_check("k_slots");
@@ -590,28 +592,28 @@ int jq_observe(jq_env *e, const int8_t *observer, int32_t fmt, int32_t all_seats
 {
     int rc = check_env(e);
     if (rc) return rc;
-    if ((rc = obs_args(e, fmt, spatial, aux, global)) != 0) return rc;
+    if ((rc = obs_args(e->rlut_ready, e->ext_on, fmt, spatial, aux, global)) != 0) return rc;
     const int nrows = all_seats ? e->S.n * 4 : e->S.n;
     const dim3 grid(nrows), block(OBS_THREADS);
     const float *x = e->ext_bel;
     if (fmt == JQ_OBS_U8 && (rc = obs_u8_grid(e)) != 0) return rc;
     int f32_pad = 0;
-    if (fmt == JQ_OBS_F32 && !e->ext_on && (rc = obs_f32_pad(e, f32_pad)) != 0) return rc;
+    if (fmt == JQ_OBS_F32 && !e->ext_on && (rc = obs_f32_pad(k_observe<0>, e->device, e->obs_f32_pad, f32_pad)) != 0) return rc;
     hipEvent_t t_end = e->obs_t_end;   // begin already recorded by jq_env_step
     e->obs_t_end = nullptr;
     if (!t_end && (rc = obs_timing_begin(e, stream, &t_end)) != 0) return rc;
     switch (fmt) {
     case JQ_OBS_F32:
         if (e->ext_on)
-            hipLaunchKernelGGL((k_observe<0, true>), grid, block, 0, strm(stream), e->S, observer, all_seats, spatial, aux, global, nrows, x);
+            hipLaunchKernelGGL((k_observe<0, true>), grid, block, 0, strm(stream), e->S, observer, all_seats, spatial, aux, global, nrows, x, nullptr);
         else
-            hipLaunchKernelGGL((k_observe<0, false>), grid, block, f32_pad, strm(stream), e->S, observer, all_seats, spatial, aux, global, nrows, nullptr);
+            hipLaunchKernelGGL((k_observe<0, false>), grid, block, f32_pad, strm(stream), e->S, observer, all_seats, spatial, aux, global, nrows, nullptr, nullptr);
         break;
     case JQ_OBS_BF16:
         if (e->ext_on)
-            hipLaunchKernelGGL((k_observe<1, true>), grid, block, 0, strm(stream), e->S, observer, all_seats, spatial, aux, global, nrows, x);
+            hipLaunchKernelGGL((k_observe<1, true>), grid, block, 0, strm(stream), e->S, observer, all_seats, spatial, aux, global, nrows, x, nullptr);
         else
-            hipLaunchKernelGGL((k_observe<1, false>), grid, block, 0, strm(stream), e->S, observer, all_seats, spatial, aux, global, nrows, nullptr);
+            hipLaunchKernelGGL((k_observe<1, false>), grid, block, 0, strm(stream), e->S, observer, all_seats, spatial, aux, global, nrows, nullptr, nullptr);
         break;
     default:
         hipLaunchKernelGGL(k_observe_u8_persist, dim3(std::min(nrows, e->obs_blocks)), dim3(OBS_THREADS), 0,
@@ -724,7 +726,7 @@ int jq_env_step(jq_env *e, const int32_t *actions, int32_t sampler, uint64_t sam
     if (sampler != JQ_SAMPLE_UNIFORM && sampler != JQ_SAMPLE_LOGITS) return fail(JQ_E_ARG, "bad sampler %d", sampler);
     if (!e->zob_ready) return fail(JQ_E_STATE, "upload the Zobrist tables before stepping");
     // the observation's arguments are checked before anything is launched
-    if (spatial && (rc = obs_args(e, obs_fmt, spatial, aux, global)) != 0) return rc;
+    if (spatial && (rc = obs_args(e->rlut_ready, e->ext_on, obs_fmt, spatial, aux, global)) != 0) return rc;
     EnvStepArgs A = {};
     A.actions = actions; A.sampler = sampler; A.sample_seed = sample_seed; A.ply = ply; A.offsets = offsets;
     A.values = values; A.values_cap = values_capacity;
@@ -917,7 +919,7 @@ int jq_history_destroy(jq_history *h)
 {
     if (!h) return JQ_OK;
     (void)hipSetDevice(h->device);
-    if (h->replay) jq_destroy(h->replay);
+    (void)hipDeviceSynchronize();   // kernels of any stream may still read the history
     for (void *p : h->allocs) (void)hipFree(p);
     delete h;
     return JQ_OK;
@@ -942,21 +944,44 @@ int jq_history_snapshot(jq_history *h, jq_env *e, const int8_t *acting, int32_t 
     if (!e->rlut_ready) return fail(JQ_E_STATE, "recency table not uploaded to the state handle");
     HIP_TRY(hipSetDevice(h->device));
     hipStream_t s = strm(stream);
-    const size_t n = (size_t)H.n, r0 = (size_t)step * n;
-    const State &S = e->S;
-    HIP_TRY(hipMemcpyAsync(H.cell + r0 * CELL_STRIDE, S.cell, n * CELL_STRIDE, hipMemcpyDeviceToDevice, s));
-    HIP_TRY(hipMemcpyAsync(H.piece + r0 * PID_STRIDE, S.piece, n * PID_STRIDE * sizeof(PieceRec), hipMemcpyDeviceToDevice, s));
-    HIP_TRY(hipMemcpyAsync(H.cm + r0 * 4 * PID_STRIDE, S.cm, n * 4 * PID_STRIDE * sizeof(CmRec), hipMemcpyDeviceToDevice, s));
-    HIP_TRY(hipMemcpyAsync(H.cme + r0 * 4 * PID_STRIDE, S.cme, n * 4 * PID_STRIDE * sizeof(CmEat), hipMemcpyDeviceToDevice, s));
-    HIP_TRY(hipMemcpyAsync(H.bcode + r0 * 4 * PID_STRIDE, S.bcode, n * 4 * PID_STRIDE, hipMemcpyDeviceToDevice, s));
-    HIP_TRY(hipMemcpyAsync(H.rem + r0 * 4 * 48, S.rem, n * 4 * 48, hipMemcpyDeviceToDevice, s));
-    HIP_TRY(hipMemcpyAsync(H.env + r0, S.env, n * sizeof(EnvRec), hipMemcpyDeviceToDevice, s));
-    HIP_TRY(hipMemcpyAsync(H.hist + r0 * HIST_LEN, S.hist, n * HIST_LEN * sizeof(int32_t), hipMemcpyDeviceToDevice, s));
+    hipLaunchKernelGGL(k_history_snapshot, dim3(H.n), dim3(256), 0, s, e->S, H, step);
+    int rc = launch_check("k_history_snapshot");
+    if (rc) return rc;
     if (!h->rlut_ready) {
-        HIP_TRY(hipMemcpyAsync(h->rlut, S.rlut, 4 * 4096 * sizeof(float), hipMemcpyDeviceToDevice, s));
+        HIP_TRY(hipMemcpyAsync(h->rlut, e->S.rlut, 4 * 4096 * sizeof(float), hipMemcpyDeviceToDevice, s));
         h->rlut_ready = true;
     }
-    h->max_moves = S.max_moves;
+    return JQ_OK;
+}
+
+// Observations and masks of `batch` history rows, straight from the history's
+// arrays: no scratch state, no allocation.
+static int history_rebuild(jq_history *h, const int64_t *flat, const int8_t *observer, int32_t batch, int32_t fmt,
+                           void *spatial, void *aux, float *global, int32_t *mask_words, uint8_t *mask_bool,
+                           void *stream)
+{
+    if (!flat || !observer) return fail(JQ_E_ARG, "history reconstruction received a null device pointer");
+    if (!h->rlut_ready) return fail(JQ_E_STATE, "history has no snapshot yet");
+    HIP_TRY(hipSetDevice(h->device));
+    int rc;
+    const State S = history_state(h->H, h->rlut, h->show_mode);
+    if (spatial || aux || global) {
+        if (!spatial || !global) return fail(JQ_E_ARG, "spatial and global outputs go together");
+        if ((rc = obs_args(true, false, fmt, spatial, aux, global)) != 0) return rc;
+        int pad = 0;
+        if (fmt == JQ_OBS_F32 &&
+            (rc = obs_f32_pad(k_observe<0, false, true>, h->device, h->obs_f32_pad, pad)) != 0) return rc;
+        auto *kernel = fmt == JQ_OBS_F32 ? &k_observe<0, false, true>
+                                         : fmt == JQ_OBS_BF16 ? &k_observe<1, false, true> : &k_observe<2, false, true>;
+        hipLaunchKernelGGL(kernel, dim3(batch), dim3(OBS_THREADS), pad, strm(stream), S, observer, 0, spatial, aux,
+                           global, batch, nullptr, flat);
+        if ((rc = launch_check("k_observe")) != 0) return rc;
+    }
+    if (mask_words || mask_bool) {
+        hipLaunchKernelGGL(k_legal<true>, dim3(batch), dim3(64), 0, strm(stream), S, observer, nullptr, mask_words,
+                           mask_bool, flat);
+        if ((rc = launch_check("k_legal")) != 0) return rc;
+    }
     return JQ_OK;
 }
 
@@ -966,128 +991,19 @@ int jq_history_reconstruct(jq_history *h, const int64_t *flat, const int8_t *obs
 {
     if (!h) return fail(JQ_E_ARG, "null history");
     if (batch <= 0) return fail(JQ_E_ARG, "cannot reconstruct an empty history minibatch");
-    if (!flat || !observer) return fail(JQ_E_ARG, "history reconstruction received a null device pointer");
-    if (!h->rlut_ready) return fail(JQ_E_STATE, "history has no snapshot yet");
-    HIP_TRY(hipSetDevice(h->device));
-    int rc;
-    if (h->replay_cap < batch) {   // scratch rows, grown to the largest batch seen
-        if (h->replay) { jq_destroy(h->replay); h->replay = nullptr; h->replay_cap = 0; }
-        if ((rc = jq_create(&h->replay, batch, std::max(1, h->max_moves), h->show_mode, h->device)) != 0) return rc;
-        h->replay_cap = batch;
-    }
-    jq_env *R = h->replay;
-    R->S.n = batch;
-    R->S.rlut = h->rlut;
-    R->rlut_ready = true;
-    hipLaunchKernelGGL(k_history_gather, dim3(batch), dim3(256), 0, strm(stream), h->H, flat, batch, R->S);
-    if ((rc = launch_check("k_history_gather")) != 0) return rc;
-    if (spatial || aux || global) {
-        if (!spatial || !global) return fail(JQ_E_ARG, "spatial and global outputs go together");
-        if ((rc = jq_observe(R, observer, fmt, 0, spatial, aux, global, stream)) != 0) return rc;
-    }
-    if (mask_words || mask_bool)
-        if ((rc = jq_legal(R, observer, nullptr, nullptr, nullptr, 0, mask_words, mask_bool, stream)) != 0) return rc;
-    return JQ_OK;
+    return history_rebuild(h, flat, observer, batch, fmt, spatial, aux, global, mask_words, mask_bool, stream);
 }
 
-// ------------------------------------------------ history rebuild without allocation
-// Rebuild-only state for jq_history_reconstruct_noalloc: the arrays the gather,
-// the observation and the legal masks touch, for at most JQ_NOALLOC_MAX_ROWS
-// rows, carved from one file-scope device array (no full combat-memory
-// records: the rebuild reads only their summaries, views and eaten-by sets).
-// 20,948 bytes per row, 21.45 MB in all on each device the library runs on.
-namespace {
-constexpr size_t NA_ROWS = JQ_NOALLOC_MAX_ROWS;
-constexpr size_t na_up(size_t x) { return (x + 255) & ~size_t(255); }
-constexpr size_t NA_CELL = 0;
-constexpr size_t NA_PIECE = NA_CELL + na_up(NA_ROWS * CELL_STRIDE);
-constexpr size_t NA_CME = NA_PIECE + na_up(NA_ROWS * PID_STRIDE * sizeof(PieceRec));
-constexpr size_t NA_CMK = NA_CME + na_up(NA_ROWS * 4 * PID_STRIDE * sizeof(CmEat));
-constexpr size_t NA_CMV = NA_CMK + na_up(NA_ROWS * 4 * PID_STRIDE);
-constexpr size_t NA_BCODE = NA_CMV + na_up(NA_ROWS * 4 * PID_STRIDE * sizeof(CmView));
-constexpr size_t NA_REM = NA_BCODE + na_up(NA_ROWS * 4 * PID_STRIDE);
-constexpr size_t NA_ENV = NA_REM + na_up(NA_ROWS * 4 * 48);
-constexpr size_t NA_HIST = NA_ENV + na_up(NA_ROWS * sizeof(EnvRec));
-constexpr size_t NA_LG = NA_HIST + na_up(NA_ROWS * HIST_LEN * sizeof(int32_t));
-constexpr size_t NA_BYTES = NA_LG + na_up(NA_ROWS * sizeof(LegalRec));
-}  // namespace
-
-static __device__ __align__(256) uint8_t scratch[NA_BYTES];
-
-namespace {
-std::mutex g_na_mu;
-uint8_t *g_na_ptr[64] = {};    // device address of `scratch` on each device
-jq_env g_na_env[64];           // host view of each device's rebuild state
-
-// Per device, once: the device address of `scratch` (the array's name is a
-// host-side stand-in and must never reach a kernel) and the state over it.
-int noalloc_state(int device, jq_env *&out)
-{
-    std::lock_guard<std::mutex> lk(g_na_mu);
-    if (device < 0 || device >= 64) return fail(JQ_E_ARG, "device %d out of range", device);
-    if (!g_na_ptr[device]) {
-        int rc = ensure_device_tables(device);
-        if (rc) return rc;
-        void *p = nullptr;
-        const hipError_t err = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (err != hipSuccess || !p)
-            return fail(JQ_E_HIP, "hipGetSymbolAddress(scratch) on device %d: %s", device, hipGetErrorString(err));
-        uint8_t *b = static_cast<uint8_t *>(p);
-        jq_env &e = g_na_env[device];
-        e.device = device;
-        State &S = e.S;
-        S.cell = reinterpret_cast<int8_t *>(b + NA_CELL);
-        S.piece = reinterpret_cast<PieceRec *>(b + NA_PIECE);
-        S.cm = nullptr;
-        S.cme = reinterpret_cast<CmEat *>(b + NA_CME);
-        S.cmk = b + NA_CMK;
-        S.cmv = reinterpret_cast<CmView *>(b + NA_CMV);
-        S.bcode = b + NA_BCODE;
-        S.rem = reinterpret_cast<int8_t *>(b + NA_REM);
-        S.env = reinterpret_cast<EnvRec *>(b + NA_ENV);
-        S.hist = reinterpret_cast<int32_t *>(b + NA_HIST);
-        S.lg = reinterpret_cast<LegalRec *>(b + NA_LG);
-        S.ztab = nullptr;
-        S.pool = nullptr;
-        S.pool_size = 0;
-        g_na_ptr[device] = b;
-    }
-    out = &g_na_env[device];
-    return JQ_OK;
-}
-}  // namespace
-
-extern "C" int jq_history_reconstruct_noalloc(jq_history *h, const int64_t *flat, const int8_t *observer,
-                                              int32_t batch, int32_t fmt, void *spatial, void *aux, float *global,
-                                              int32_t *mask_words, uint8_t *mask_bool, void *stream)
+int jq_history_reconstruct_noalloc(jq_history *h, const int64_t *flat, const int8_t *observer, int32_t batch,
+                                   int32_t fmt, void *spatial, void *aux, float *global, int32_t *mask_words,
+                                   uint8_t *mask_bool, void *stream)
 {
     if (!h) return fail(JQ_E_ARG, "null history");
     if (batch <= 0) return fail(JQ_E_ARG, "cannot reconstruct an empty history minibatch");
     if (batch > JQ_NOALLOC_MAX_ROWS)
         return fail(JQ_E_ARG, "batch %d exceeds the %d rows jq_history_reconstruct_noalloc holds", batch,
                     JQ_NOALLOC_MAX_ROWS);
-    if (!flat || !observer) return fail(JQ_E_ARG, "history reconstruction received a null device pointer");
-    if (!h->rlut_ready) return fail(JQ_E_STATE, "history has no snapshot yet");
-    HIP_TRY(hipSetDevice(h->device));
-    jq_env *R = nullptr;
-    int rc = noalloc_state(h->device, R);
-    if (rc) return rc;
-    R->S.n = batch;
-    R->S.max_moves = std::max(1, h->max_moves);
-    R->S.show_mode = h->show_mode;
-    R->S.rlut = h->rlut;
-    R->rlut_ready = true;
-    R->zob_ready = false;
-    R->ext_on = false;
-    hipLaunchKernelGGL(k_history_gather, dim3(batch), dim3(256), 0, strm(stream), h->H, flat, batch, R->S);
-    if ((rc = launch_check("k_history_gather")) != 0) return rc;
-    if (spatial || aux || global) {
-        if (!spatial || !global) return fail(JQ_E_ARG, "spatial and global outputs go together");
-        if ((rc = jq_observe(R, observer, fmt, 0, spatial, aux, global, stream)) != 0) return rc;
-    }
-    if (mask_words || mask_bool)
-        if ((rc = jq_legal(R, observer, nullptr, nullptr, nullptr, 0, mask_words, mask_bool, stream)) != 0) return rc;
-    return JQ_OK;
+    return history_rebuild(h, flat, observer, batch, fmt, spatial, aux, global, mask_words, mask_bool, stream);
 }
 
 // ---------------------------------------------------------------- masks

@@ -163,6 +163,10 @@ struct PieceIn {
     int lsum, rsum;                // left / right enemies' memory of an own piece (cm_summary)
 };
 
+// HIST: the state is a rollout history's arrays (history_state), which keep the
+// combat-memory records but not the views and summary bytes derived from them;
+// those are derived here, from the one or two records the pid needs.
+template <bool HIST = false>
 __device__ __forceinline__ void piece_load(const State &S, int env, int obs, int pid, PieceIn &P)
 {
     const int le = (obs + 1) & 3, re = (obs + 3) & 3, s = pid / 30;
@@ -176,14 +180,26 @@ __device__ __forceinline__ void piece_load(const State &S, int env, int obs, int
     P.ldir = P.lchain = P.fstep = -1;
     P.lsum = P.rsum = 0;
     if ((s & 1) != (obs & 1)) {
-        const CmView v = S.cmv[cm_idx(env, obs, pid)];
+        CmView v;
+        if constexpr (HIST) {
+            const CmRec c = S.cm[cm_idx(env, obs, pid)];
+            v = cm_view(c, obs);
+        } else {
+            v = S.cmv[cm_idx(env, obs, pid)];
+        }
         P.kmask = v.kmask; P.types = v.types; P.cnts = v.cnts;
         P.ldir = v.ldir; P.lchain = v.lchain; P.fstep = v.fstep;
     } else if (s == obs) {
         const CmEat e = S.cme[cm_idx(env, obs, pid)];
         P.elo = e.elo; P.ehi = e.ehi;
-        P.lsum = S.cmk[cm_idx(env, le, pid)];
-        P.rsum = S.cmk[cm_idx(env, re, pid)];
+        if constexpr (HIST) {
+            const CmRec cl = S.cm[cm_idx(env, le, pid)], cr = S.cm[cm_idx(env, re, pid)];
+            P.lsum = cm_summary(cl);
+            P.rsum = cm_summary(cr);
+        } else {
+            P.lsum = S.cmk[cm_idx(env, le, pid)];
+            P.rsum = S.cmk[cm_idx(env, re, pid)];
+        }
     }
 }
 
@@ -405,6 +421,7 @@ struct RowIn {
 // Thread roles: 0..127 one pid each (piece_of_thread) or, for the 8 spare
 // threads, one padding recency slot; 128..159 one move-history ring slot each,
 // 160..166 the whole-plane seat flags; 0..27 also write the 28 globals.
+template <bool HIST = false>
 __device__ __forceinline__ void row_fetch(const State &S, int env, int obs, int t, RowIn &R)
 {
     const int l = t & 63;
@@ -413,12 +430,26 @@ __device__ __forceinline__ void row_fetch(const State &S, int env, int obs, int 
     R.hist = 0;
     R.rem = 0;
     const int pid = t < PID_STRIDE ? piece_of_thread(t, obs) : -1;
-    if (pid >= 0) piece_load(S, env, obs, pid, R.P);
+    if (pid >= 0) piece_load<HIST>(S, env, obs, pid, R.P);
     else if (t >= T_HIST && t < T_FLAGS) R.hist = S.hist[(size_t)env * HIST_LEN + (t - T_HIST)];
     if (t < 24) {
         const int seat = t < 12 ? (obs + 1) & 3 : (obs + 3) & 3;
         R.rem = S.rem[((size_t)env * 4 + obs) * 48 + seat * 12 + t % 12];
     }
+}
+
+// The inputs of an empty, terminated game (k_clear), for a history row that
+// does not exist.
+__device__ __forceinline__ void row_empty(RowIn &R)
+{
+    R.ew = 0;
+    R.own_tp = 15;   // no piece (-1 & 15)
+    R.hist = R.rem = 0;
+    PieceIn &P = R.P;
+    P.pos = P.tp = P.dstep = P.dreason = P.dloc = P.zero = P.ldir = P.lchain = P.fstep = -1;
+    P.mcount = P.aeat = P.psurv = P.bcode = P.lsum = P.rsum = 0;
+    P.kmask = P.types = P.cnts = 0;
+    P.elo = P.ehi = 0;
 }
 
 // The observer of `row` (row_obs) as a per-lane vector load: lane 0 holds it,
@@ -795,12 +826,18 @@ __device__ __forceinline__ void obs_emit_u8(const ObsLds &L, uint8_t *row, int m
 // nrows = N (one row per env, observer given or the acting seat) or 4N
 // (all_seats: row = env * 4 + observer). One 256-thread block per row. EXT
 // (f32 / bf16): belief planes from ext, (N, 4, 12, 289) float32 world-cell
-// beliefs per (env, observer).
-template <int FMT, bool EXT = false>
+// beliefs per (env, observer). HIST: row i is row flat[i] of a rollout history
+// (S = history_state) seen by observer[i]; flat values outside [0, S.n) give
+// the empty terminated game. The block reads the ~8 KB of its history row that
+// its observer uses; a gather of the whole 36 KB row into a scratch state,
+// observed from there, took 69 us more at 4,096 bf16 rows (291.8 us a minibatch
+// with it).
+template <int FMT, bool EXT = false, bool HIST = false>
 __global__ __launch_bounds__(OBS_THREADS) void k_observe(State S, const int8_t *__restrict__ observer, int all_seats,
                                                          void *__restrict__ spatial, void *__restrict__ aux,
                                                          float *__restrict__ glob, int nrows,
-                                                         const float *__restrict__ ext = nullptr)
+                                                         const float *__restrict__ ext = nullptr,
+                                                         const int64_t *__restrict__ flat = nullptr)
 {
     __shared__ ObsLds L;
     ExtLds *X = nullptr;
@@ -811,7 +848,17 @@ __global__ __launch_bounds__(OBS_THREADS) void k_observe(State S, const int8_t *
     constexpr int ES = FMT == 0 ? 4 : FMT == 1 ? 2 : 1;
     const int t = threadIdx.x, row = blockIdx.x;
     if (row >= nrows) return;
-    const int env = row_env(row, all_seats), obs = row_obs(S, observer, all_seats, row);
+    int env, obs;
+    bool stored = true;   // the row exists (always, but for HIST)
+    if constexpr (HIST) {
+        const int64_t f = flat[row];
+        stored = f >= 0 && f < (int64_t)S.n;
+        env = stored ? (int)f : 0;
+        obs = observer[row] & 3;
+    } else {
+        env = row_env(row, all_seats);
+        obs = row_obs(S, observer, all_seats, row);
+    }
     uint8_t *rowp = reinterpret_cast<uint8_t *>(spatial) + (size_t)row * OBS_ROW * ES;
     const int m = (int)(((uintptr_t)rowp / ES) & (16 / ES - 1));
     // Wave issue priority 2 from the block's start through its fill, 0 while
@@ -826,7 +873,8 @@ __global__ __launch_bounds__(OBS_THREADS) void k_observe(State S, const int8_t *
     if (EXT && t < PID_STRIDE) X->rel[t] = 0;
     lds_barrier();
     RowIn R;
-    row_fetch(S, env, obs, t, R);
+    if (stored) row_fetch<HIST>(S, env, obs, t, R);
+    else row_empty(R);
     row_fill<EXT, FMT == 2>(S, obs, m, t, R, L, glob ? glob + (size_t)row * 28 : nullptr,
                             EXT ? ext + ((size_t)env * 4 + obs) * 12 * NC : nullptr, X);
     __builtin_amdgcn_s_setprio(0);

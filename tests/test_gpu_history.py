@@ -113,3 +113,51 @@ def test_history_rejects_a_mismatched_state(jq):
     hist.close()
     other.close()
     ro.close()
+
+
+@pytest.mark.parametrize("n,show", [(1, 0), (67, 1), (256, 2)])
+def test_history_rows_equal_the_live_state(jq, n, show):
+    """Rows rebuilt in place equal the live games' own observations and masks
+    (which read the derived views, not the records) for every seat and format,
+    after enough play for combat memory, deaths and restarts; rows outside the
+    history equal an empty batch's."""
+    from junqi_amd import _lib as L
+    print(f"[history] live n={n} show={show}", flush=True)
+    b = jq.JunqiBatch(n, show_mode=show, max_num_moves=500)
+    b.reset(9)
+    b.legal()
+    for k in range(420):
+        b.env_step(sampler="logits", sample_seed=3, ply=k, reset_seed=k)
+    dev, steps = b.device, 3
+    hist = jq.GpuRolloutHistory(num_steps=steps, num_envs=n, show_mode=show)
+    for t in (2, 0, 1):   # the last snapshot is the live state
+        hist.snapshot(b, torch.zeros(n, dtype=torch.int8, device=dev), t)
+        if t != 1:
+            b.env_step(sampler="logits", sample_seed=3, ply=1000 + t, reset_seed=t)
+    empty = jq.JunqiBatch(1, show_mode=show)
+    for fmt, dt in (("f32", torch.float32), ("bf16", torch.bfloat16), ("u8", torch.uint8)):
+        code = {"f32": L.OBS_F32, "bf16": L.OBS_BF16, "u8": L.OBS_U8}[fmt]
+        for seat in range(4):
+            seats = torch.full((n,), seat, dtype=torch.int8, device=dev)
+            live = b.observe(seats, fmt=fmt)
+            legal = b.legal(seats, mask_bool=True)
+            none = empty.observe(seats[:1], fmt=fmt)
+            flat = torch.cat([torch.arange(n, device=dev) + n, torch.tensor([-1, steps * n, 1 << 40], device=dev)])
+            rows, obs = n + 3, torch.full((n + 3,), seat, dtype=torch.int8, device=dev)
+            sp = torch.empty((rows, 317, 17, 17), dtype=dt, device=dev)
+            gl = torch.empty((rows, 28), dtype=torch.float32, device=dev)
+            aux = torch.empty((rows, L.AUX_BYTES), dtype=torch.uint8, device=dev) if fmt == "u8" else None
+            words = torch.empty((rows, 521), dtype=torch.int32, device=dev)
+            mask = torch.empty((rows, 16641), dtype=torch.bool, device=dev)
+            L.check(L.lib.jq_history_reconstruct(hist._h, flat.data_ptr(), obs.data_ptr(), rows, code, sp.data_ptr(),
+                                                 None if aux is None else aux.data_ptr(), gl.data_ptr(),
+                                                 words.data_ptr(), mask.data_ptr(),
+                                                 torch.cuda.current_stream().cuda_stream))
+            got = [sp, gl] + ([aux] if fmt == "u8" else [])
+            for g, w, e in zip(got, live, none):
+                assert torch.equal(g[:n], w) and torch.equal(g[n:], e.expand_as(g[n:])), (fmt, seat)
+            assert torch.equal(words[:n], legal["mask_words"]) and torch.equal(mask[:n], legal["mask_bool"])
+            assert not words[n:].any() and not mask[n:].any()
+    hist.close()
+    b.close()
+    empty.close()
