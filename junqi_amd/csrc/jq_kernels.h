@@ -21,8 +21,6 @@
 namespace jq {
 
 __constant__ Tables cT;
-__constant__ uint8_t cBVAL[BC_COUNT][12];   // belief code x type -> obs value code
-__constant__ float cDECODE[256];             // obs value code -> float
 constexpr int JQ_MASK_WORDS_PAD = 528;
 constexpr int LSCR_WORDS = 12;   // legal_body's per-wave LDS scratch (u64 words)
 

@@ -28,7 +28,7 @@ struct jq_env {
     std::vector<void *> allocs;
     bool zob_ready = false, rlut_ready = false;
     int obs_blocks = 0;              // resident u8 observation blocks on the device
-    int obs_f32_pad = -1;            // dynamic LDS bytes that hold the f32 observation at 3 blocks per CU
+    int cus = 0;                     // compute units of the device
     float *ext_bel = nullptr;        // uploaded (N, 4, 12, 289) beliefs, allocated on first upload
     bool ext_on = false;             // observations read the uploaded beliefs
     int8_t *pool = nullptr;          // setup pool buffer (reused while uploads fit)
@@ -50,7 +50,7 @@ struct jq_history {
     std::vector<void *> allocs;
     float *rlut = nullptr;           // recency table copied from the snapshotted handle
     bool rlut_ready = false;
-    int obs_f32_pad = -1;            // as jq_env's, for the rebuilding kernel
+    int cus = 0;                     // compute units of the device
 };
 
 namespace {
@@ -126,6 +126,26 @@ void build_host_tables()
     g_host_tables = true;
 }
 
+// The observation blocks' row-independent LDS content (ObsConsts).
+ObsConsts build_obs_consts()
+{
+    ObsConsts k{};
+    for (int i = 0; i < NC; ++i)
+        for (int b = 0; b < 6; ++b)
+            if ((g_tables.statics[i] >> b) & 1) {
+                const int e = (58 + b) * NC + i;
+                k.stat[(e >> 5) - STAT_Q0 * 4] |= 1u << (e & 31);
+            }
+    for (int i = 0; i < 17; ++i) {
+        uint32_t u;
+        k.dec[i] = g_decode[i];
+        std::memcpy(&u, &g_decode[i], 4);
+        k.decb[i] = (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);   // bf16, round to nearest even
+    }
+    std::memcpy(k.bval, g_bval, sizeof g_bval);
+    return k;
+}
+
 int ensure_device_tables(int device)
 {
     std::lock_guard<std::mutex> lk(g_tab_mu);
@@ -133,8 +153,8 @@ int ensure_device_tables(int device)
     if (device < 0 || device >= 64) return fail(JQ_E_ARG, "device %d out of range", device);
     if (g_tab_done[device]) return JQ_OK;
     HIP_TRY(hipMemcpyToSymbol(HIP_SYMBOL(cT), &g_tables, sizeof g_tables));
-    HIP_TRY(hipMemcpyToSymbol(HIP_SYMBOL(cBVAL), g_bval, sizeof g_bval));
-    HIP_TRY(hipMemcpyToSymbol(HIP_SYMBOL(cDECODE), g_decode, sizeof g_decode));
+    const ObsConsts oc = build_obs_consts();
+    HIP_TRY(hipMemcpyToSymbol(HIP_SYMBOL(cOBS), &oc, sizeof oc));
     g_tab_done[device] = true;
     return JQ_OK;
 }
@@ -264,46 +284,69 @@ int launch_check(const char *what)
     return JQ_OK;
 }
 
+int device_cus(int device, int &cus)
+{
+    if (cus > 0) return JQ_OK;
+    int n = 0;
+    HIP_TRY(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device));
+    cus = std::max(1, n);
+    return JQ_OK;
+}
+
 // Persistent grid of the u8 observation kernel: every block the device can
 // hold at once.
 int obs_u8_grid(jq_env *e)
 {
     if (e->obs_blocks > 0) return JQ_OK;
-    int per_cu = 0, cus = 0;
+    int per_cu = 0;
     HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_observe_u8_persist, OBS_THREADS, 0));
-    HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, e->device));
-    e->obs_blocks = std::max(1, per_cu) * std::max(1, cus);
+    int rc = device_cus(e->device, e->cus);
+    if (rc) return rc;
+    e->obs_blocks = std::max(1, per_cu) * e->cus;
     return JQ_OK;
 }
 
-// The f32 observation (one block per 366,452-byte row) writes faster with at
-// most 3 blocks per CU than at the 4 its LDS and registers allow (fewer rows
-// streaming at once: 2.377 -> 2.272 ms per launch at 32,768 rows; bf16 rows,
-// half as long, are slower at 3). Each block asks for unused dynamic LDS that
-// brings it to the midpoint between a third and a quarter of the CU's LDS, so
-// a fourth block does not fit and a third still does after the allocation
-// rounds up (a pad that left only 0.9 % of slack under the third was rounded
-// past it: 2 blocks per CU, 3.06 ms). 0 when the occupancy query does not
-// confirm exactly 3.
-template <class Kernel>
-int obs_f32_pad(Kernel kernel, int device, int &cache, int &pad)
+// u8 rows (one per env) go through the persistent kernel from more than four
+// rows per resident block on: its prefetch of the next row's inputs hides their
+// loads, which come from memory after a step's gigabytes of stores, and its tail
+// takes the CSR pass. Below that k_observe, with the CSR pass in line, is
+// faster (us per fused u8 step, persistent -> k_observe: 64 games 50.6 -> 40.3,
+// 1,024 65.4 -> 57.4, 4,096 118.4 -> 116.2, 16,384 364 -> 381, 32,768
+// 709 -> 751).
+bool obs_persists(const jq_env *e) { return e->S.n > 4 * e->obs_blocks; }
+
+// How k_observe runs `nrows` rows of format `fmt` on a device with `cus` CUs:
+// blocks per row, and streaming or ordinary stores.
+//
+// Few rows: as many blocks per row as keep the grid near T blocks per CU (f32 4,
+// u8 4, bf16 2.75), at most 16 (u8 rows, a quarter as long, 4). us per launch,
+// 512-thread blocks, P = 1 -> the rule's: f32 24 rows 28.8 -> 10.9, 96 rows
+// 30.4 -> 16.9, 333 rows 41.3 -> 28.9; bf16 24 rows 24.0 -> 12.3, 333 rows
+// 28.8 -> 25.4; u8 64 rows 11.5 -> 10.0, 512 rows 15.7 -> 14.8. Past that the
+// repeated loads and fill cost more than the shorter runs give (u8 and bf16,
+// one block per row from there on: bf16 2,048 rows in 1 / 2 / 3 parts
+// 82 / 98 / 113). f32 rows are long enough to stay split: fewer bytes then
+// stream at once and reach memory in better order (8,192 rows in 1 / 2 / 3 / 4
+// parts 598 / 594 / 531 / 590).
+//
+// Streaming stores leave the caches as they are written, which wins once the
+// output does not fit the 256 MB memory-side cache anyway (4,096 u8 rows 89 ->
+// 76, 2,048 bf16 rows 96 -> 82, 1,000 f32 rows 79.7 -> 74.9) and loses while it
+// fits (1,024 u8 rows 21.0 -> 24.0, 768 bf16 rows 36 -> 41, 500 f32 rows
+// 38 -> 43).
+constexpr int64_t OBS_STREAM_BYTES = 256ll << 20;
+
+struct ObsPlan {
+    int parts, stream;
+};
+
+ObsPlan obs_plan(int fmt, int nrows, int cus)
 {
-    if (cache < 0) {
-        hipFuncAttributes fa{};
-        int lds_cu = 0, per_cu = 0;
-        HIP_TRY(hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(kernel)));
-        HIP_TRY(hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, device));
-        int p = (lds_cu / 3 + lds_cu / 4) / 2 - (int)fa.sharedSizeBytes;
-        if (p > 0) {
-            HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, OBS_THREADS, p));
-            if (per_cu != 3) p = 0;
-        } else {
-            p = 0;
-        }
-        cache = p;
-    }
-    pad = cache;
-    return JQ_OK;
+    const int es = fmt == JQ_OBS_F32 ? 4 : fmt == JQ_OBS_BF16 ? 2 : 1;
+    const bool stream = (int64_t)nrows * OBS_ROW * es > OBS_STREAM_BYTES;
+    const int blocks = fmt == JQ_OBS_BF16 ? cus * 11 / 4 : cus * 4;
+    const int least = fmt == JQ_OBS_F32 ? (stream ? 3 : 2) : 1, most = fmt == JQ_OBS_U8 ? 4 : 16;
+    return {std::max(least, std::min(most, blocks / nrows)), stream ? 1 : 0};
 }
 
 // The checks of an observation request (format, buffers, tables it needs).
@@ -594,32 +637,22 @@ int jq_observe(jq_env *e, const int8_t *observer, int32_t fmt, int32_t all_seats
     if (rc) return rc;
     if ((rc = obs_args(e->rlut_ready, e->ext_on, fmt, spatial, aux, global)) != 0) return rc;
     const int nrows = all_seats ? e->S.n * 4 : e->S.n;
-    const dim3 grid(nrows), block(OBS_THREADS);
-    const float *x = e->ext_bel;
-    if (fmt == JQ_OBS_U8 && (rc = obs_u8_grid(e)) != 0) return rc;
-    int f32_pad = 0;
-    if (fmt == JQ_OBS_F32 && !e->ext_on && (rc = obs_f32_pad(k_observe<0>, e->device, e->obs_f32_pad, f32_pad)) != 0) return rc;
+    if ((rc = obs_u8_grid(e)) != 0) return rc;
     hipEvent_t t_end = e->obs_t_end;   // begin already recorded by jq_env_step
     e->obs_t_end = nullptr;
     if (!t_end && (rc = obs_timing_begin(e, stream, &t_end)) != 0) return rc;
-    switch (fmt) {
-    case JQ_OBS_F32:
-        if (e->ext_on)
-            hipLaunchKernelGGL((k_observe<0, true>), grid, block, 0, strm(stream), e->S, observer, all_seats, spatial, aux, global, nrows, x, nullptr);
-        else
-            hipLaunchKernelGGL((k_observe<0, false>), grid, block, f32_pad, strm(stream), e->S, observer, all_seats, spatial, aux, global, nrows, nullptr, nullptr);
-        break;
-    case JQ_OBS_BF16:
-        if (e->ext_on)
-            hipLaunchKernelGGL((k_observe<1, true>), grid, block, 0, strm(stream), e->S, observer, all_seats, spatial, aux, global, nrows, x, nullptr);
-        else
-            hipLaunchKernelGGL((k_observe<1, false>), grid, block, 0, strm(stream), e->S, observer, all_seats, spatial, aux, global, nrows, nullptr, nullptr);
-        break;
-    default:
+    if (fmt == JQ_OBS_U8 && !all_seats && obs_persists(e)) {
         hipLaunchKernelGGL(k_observe_u8_persist, dim3(std::min(nrows, e->obs_blocks)), dim3(OBS_THREADS), 0,
                            strm(stream), e->S, observer, all_seats, static_cast<uint8_t *>(spatial),
                            static_cast<uint8_t *>(aux), global, nrows);
-        break;
+    } else {
+        const ObsPlan p = obs_plan(fmt, nrows, e->cus);
+        auto *kernel = fmt == JQ_OBS_U8 ? &k_observe<2>
+                       : fmt == JQ_OBS_BF16 ? (e->ext_on ? &k_observe<1, true> : &k_observe<1>)
+                                            : (e->ext_on ? &k_observe<0, true> : &k_observe<0>);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nrows * p.parts), dim3(ROW_THREADS), 0, strm(stream), e->S, observer,
+                           all_seats, spatial, aux, global, nrows, p.parts, p.stream,
+                           static_cast<const float *>(e->ext_bel), nullptr);
     }
     rc = launch_check("k_observe");
     // the end event follows its begin event even when the launch failed, so no
@@ -734,7 +767,8 @@ int jq_env_step(jq_env *e, const int32_t *actions, int32_t sampler, uint64_t sam
     A.do_reset = e->S.pool ? 1 : 0; A.reset_seed = reset_seed; A.counts = counts;
     // The overlapped form moves the CSR pass, and the canonical mask with it,
     // beside the observation (below); the step kernel then skips the mask.
-    const bool overlap = spatial && obs_fmt == JQ_OBS_U8 && csr_always_fits(e, values_capacity);
+    if ((rc = obs_u8_grid(e)) != 0) return rc;
+    const bool overlap = spatial && obs_fmt == JQ_OBS_U8 && obs_persists(e) && csr_always_fits(e, values_capacity);
     A.mask_words = overlap ? nullptr : mask_words;
     // sample (unless actions are given), ply, restart from the pool and the
     // next seat's legal sets in one kernel
@@ -968,13 +1002,12 @@ static int history_rebuild(jq_history *h, const int64_t *flat, const int8_t *obs
     if (spatial || aux || global) {
         if (!spatial || !global) return fail(JQ_E_ARG, "spatial and global outputs go together");
         if ((rc = obs_args(true, false, fmt, spatial, aux, global)) != 0) return rc;
-        int pad = 0;
-        if (fmt == JQ_OBS_F32 &&
-            (rc = obs_f32_pad(k_observe<0, false, true>, h->device, h->obs_f32_pad, pad)) != 0) return rc;
+        if ((rc = device_cus(h->device, h->cus)) != 0) return rc;
+        const ObsPlan p = obs_plan(fmt, batch, h->cus);
         auto *kernel = fmt == JQ_OBS_F32 ? &k_observe<0, false, true>
                                          : fmt == JQ_OBS_BF16 ? &k_observe<1, false, true> : &k_observe<2, false, true>;
-        hipLaunchKernelGGL(kernel, dim3(batch), dim3(OBS_THREADS), pad, strm(stream), S, observer, 0, spatial, aux,
-                           global, batch, nullptr, flat);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)batch * p.parts), dim3(ROW_THREADS), 0, strm(stream), S, observer, 0,
+                           spatial, aux, global, batch, p.parts, p.stream, nullptr, flat);
         if ((rc = launch_check("k_observe")) != 0) return rc;
     }
     if (mask_words || mask_bool) {

@@ -4,7 +4,7 @@
 // Layout and values follow junqi_core/observation.py:155-232 (317 planes in the
 // observer's canonical frame, 28 globals) and its writers at :908-1651.
 //
-// Every element of a row has a u8 value code (cDECODE maps codes to floats).
+// Every element of a row has a u8 value code (ObsConsts::dec maps codes to floats).
 // Only ~1-2k of the 91,613 elements are nonzero, so a row is built sparsely in
 // LDS and then streamed densely:
 //   * `bits`: one bit per element, bit 0 of its code (all 0/1 planes), set by
@@ -25,17 +25,19 @@
 // recency planes as uint16 codes per cell, 0 for 0.0 and 1 + e for the value
 // exp(-e / tau) at elapsed step e (entry e of the recency table).
 //
-// The u8 kernel is persistent (grid = resident blocks): while a block streams
+// The u8 rows of a large batch go through a persistent kernel (grid = resident blocks): while a block streams
 // row i out, its threads already hold the gathered inputs of row i + gridDim.x
 // in registers, so the next fill only waits for the recency-table lookups.
-// f32 / bf16 rows are 2-4x wider; they run one 256-thread block per row.
+// Every other observation (f32, bf16, few u8 rows, all seats, history rows) runs
+// k_observe, whose blocks build one row or part of a row and end.
 #pragma once
 
 namespace jq {
 
 constexpr int OBS_C = 317;
 constexpr int OBS_ROW = OBS_C * NC;   // 91,613 elements
-constexpr int OBS_THREADS = 256;
+constexpr int OBS_THREADS = 256;      // persistent u8 kernel
+constexpr int ROW_THREADS = 512;      // k_observe: eight waves stream each row
 constexpr int OBS_BITS_WORDS = 2868;  // >= ceil(91613 / 32) + 1, multiple of 4
 
 // Byte-image ranges [start, end) in elements; each gets 16 zero bytes on either
@@ -70,18 +72,26 @@ constexpr uint8_t CODE_ONE = 1, CODE_NEG = 2, CODE_THIRD = 3, CODE_2THIRD = 4;
 // slot each, 160..166 the whole-plane seat flags
 constexpr int T_HIST = PID_STRIDE, T_FLAGS = T_HIST + HIST_LEN, T_END = T_FLAGS + 7;
 
+// The row-independent part of a block's LDS, built once on the host
+// (build_obs_consts) and copied in by every block.
+struct alignas(16) ObsConsts {
+    uint32_t stat[STAT_NQ * 4];   // board_static words of `bits`
+    float dec[32];                // code -> f32
+    uint32_t decb[32];            // code -> bf16 bits
+    uint8_t bval[BC_COUNT * 12 + 4];   // belief row code x type -> value code
+};
+static_assert(sizeof(ObsConsts) % 16 == 0, "copied in 16-byte words");
+__constant__ ObsConsts cOBS;
+
 struct ObsLds {
     alignas(16) uint32_t bits[OBS_BITS_WORDS];
     alignas(16) uint8_t img[IMG_BYTES];
-    alignas(16) uint32_t stat[STAT_NQ * 4];   // board_static words of `bits` (row-independent)
+    ObsConsts k;
     union {
         float rec[PID_STRIDE][4];      // recency values per pid (0 unless an enemy piece on board): f32 / bf16
         uint16_t rcode[PID_STRIDE][4]; // the same as aux codes (0 none, 1 + elapsed): u8
     };
-    float dec[32];                   // code -> f32
-    uint32_t decb[32];               // code -> bf16 bits
     int8_t cpid[CELL_STRIDE];        // canonical cell -> pid (-1 empty)
-    alignas(4) uint8_t bval[BC_COUNT * 12 + 4]; // belief row code x type -> value code
     float turnv[2];
 };
 
@@ -233,7 +243,7 @@ __device__ __forceinline__ void piece_scatter(int show_mode, int obs, int pid, i
             const int bc = P.bcode < BC_COUNT ? P.bcode : 0;
             const int c0 = rel == 1 ? 12 : rel == 2 ? 27 : 39;
             const int base = rel == 1 ? RG0_B : RG1_B, start = rel == 1 ? RG0_S : RG1_S;
-            const uint32_t *bw = reinterpret_cast<const uint32_t *>(&L.bval[bc * 12]);   // the 12 codes
+            const uint32_t *bw = reinterpret_cast<const uint32_t *>(&L.k.bval[bc * 12]);   // the 12 codes
             const uint32_t b3[3] = {bw[0], bw[1], bw[2]};
 #pragma unroll
             for (int j = 0; j < 12; ++j) {
@@ -354,38 +364,21 @@ __device__ __forceinline__ uint16_t recency_code(int mc, int last)
     return (uint16_t)(1 + el);
 }
 
-// Row-independent LDS content (tables, board_static template) of one buffer.
-// All `nthreads` threads of the block call it; it ends with a barrier.
-__device__ __forceinline__ void obs_setup(ObsLds &L, int t, int nthreads)
+// Row-independent LDS content of a block. The copy is complete after the next
+// barrier.
+__device__ __forceinline__ void obs_setup(ObsLds &L, int t)
 {
-    for (int i = t; i < BC_COUNT * 12; i += nthreads) L.bval[i] = cBVAL[i / 12][i % 12];
-    if (t < 32) {
-        const float d = t < 17 ? cDECODE[t] : 0.f;
-        L.dec[t] = d;
-        L.decb[t] = f32_to_bf16_rne(d);
-    }
-    if (t < STAT_NQ * 4) L.stat[t] = 0;
-    lds_barrier();
-    for (int k = t; k < NC; k += nthreads) {   // board_static (58-63): fixed cell classes
-        uint32_t sm = cT.statics[k];
-        while (sm) {
-            const int b = __builtin_ctz(sm);
-            sm &= sm - 1;
-            if (b < 6) {
-                const int e = (58 + b) * NC + k;
-                atomicOr(&L.stat[(e >> 5) - STAT_Q0 * 4], 1u << (e & 31));
-            }
-        }
-    }
-    lds_barrier();
+    constexpr int NQ = sizeof(ObsConsts) / 16;
+    static_assert(NQ <= OBS_THREADS && NQ <= ROW_THREADS, "one word per thread");
+    if (t < NQ) reinterpret_cast<uint4 *>(&L.k)[t] = reinterpret_cast<const uint4 *>(&cOBS)[t];
 }
 
-// Empty row: zero bits except the board_static template, zero image, no pieces.
-// Thread t of `nthreads`.
-__device__ __forceinline__ void obs_clear(ObsLds &L, int t, int nthreads)
+// Empty row: zero bits except the board_static template (`stat`), zero image,
+// no pieces. Thread t of `nthreads`.
+__device__ __forceinline__ void obs_clear(ObsLds &L, const uint32_t *stat, int t, int nthreads)
 {
     uint4 *w = reinterpret_cast<uint4 *>(L.bits);
-    const uint4 *st = reinterpret_cast<const uint4 *>(L.stat);
+    const uint4 *st = reinterpret_cast<const uint4 *>(stat);
     for (int i = t; i < OBS_BITS_WORDS / 4; i += nthreads)
         w[i] = (unsigned)(i - STAT_Q0) < (unsigned)STAT_NQ ? st[i - STAT_Q0] : make_uint4(0, 0, 0, 0);
     uint4 *b = reinterpret_cast<uint4 *>(L.img);
@@ -464,7 +457,7 @@ __device__ __forceinline__ int row_obs_prefetch(const State &S, const int8_t *ob
 }
 
 // Fill a cleared buffer with row (env, obs) from the fetched inputs, thread t
-// in [0, 256). Only the recency-table gathers are loads here. No thread reads
+// (from T_END on a thread has no part in it). Only the recency-table gathers are loads here. No thread reads
 // what another one writes, so no barrier is needed inside.
 // AUXC (the u8 format): recency as aux codes, no table lookups.
 template <bool EXT = false, bool AUXC = false>
@@ -583,7 +576,7 @@ __device__ __forceinline__ uint32_t obs_elem(const ObsLds &L, int e, int m, cons
     }
     const uint32_t code = obs_code_at(L, e, m);
     if (FMT == 2) return code;
-    return FMT == 0 ? __float_as_uint(L.dec[code]) : L.decb[code];
+    return FMT == 0 ? __float_as_uint(L.k.dec[code]) : L.k.decb[code];
 }
 
 __device__ __forceinline__ uint32_t bit_window(const ObsLds &L, int e)
@@ -612,7 +605,7 @@ __device__ __forceinline__ uint4 obs_chunk(const ObsLds &L, int e0, int off, boo
                 const int sh = (i & 1) * 16;
                 const uint32_t c0 = ((cw >> sh) & 0xFFu) | ((v >> (2 * i)) & 1u);
                 const uint32_t c1 = ((cw >> (sh + 8)) & 0xFFu) | ((v >> (2 * i + 1)) & 1u);
-                w[i] = L.decb[c0] | (L.decb[c1] << 16);
+                w[i] = L.k.decb[c0] | (L.k.decb[c1] << 16);
             }
         } else {
             for (int i = 0; i < 4; ++i) {   // 2 bits -> two bf16 halves of 0 / 1.0
@@ -623,7 +616,7 @@ __device__ __forceinline__ uint4 obs_chunk(const ObsLds &L, int e0, int off, boo
     } else {
         if (img) {
             const uint32_t cw = *reinterpret_cast<const uint32_t *>(&L.img[off]);
-            for (int i = 0; i < 4; ++i) w[i] = __float_as_uint(L.dec[((cw >> (8 * i)) & 0xFFu) | ((v >> i) & 1u)]);
+            for (int i = 0; i < 4; ++i) w[i] = __float_as_uint(L.k.dec[((cw >> (8 * i)) & 0xFFu) | ((v >> i) & 1u)]);
         } else {
             for (int i = 0; i < 4; ++i) w[i] = ((v >> i) & 1u) ? 0x3F800000u : 0u;
         }
@@ -644,23 +637,22 @@ __device__ __forceinline__ void obs_elems(const ObsLds &L, uint8_t *row, int e, 
     }
 }
 
-// A 16-byte chunk of a bf16 / f32 row. The bf16 rows go out as streaming
-// stores (1.464 -> 1.365 ms per fused bf16 step at 32,768 games); f32 rows
-// measured slower that way (2.68 -> 2.71 ms per drop-in step) and keep
-// ordinary stores.
-template <int FMT>
-__device__ __forceinline__ void row_store(uint4 *p, uint4 v)
+// A 16-byte chunk of a row, as a streaming or an ordinary store (obs_launch
+// chooses; uniform over the grid).
+__device__ __forceinline__ void row_store(uint4 *p, uint4 v, bool stream)
 {
-    if constexpr (FMT == 1) stream_store(p, v);
+    if (stream) stream_store(p, v);
     else *p = v;
 }
 
 // Stream the 91,613-element row to `row` (element phase m) in 16-byte chunks:
 // chunk q covers row bytes [16q - lead, 16q - lead + 16). A wave iteration
 // stores one whole 1 KB-aligned unit of the buffer (the row's first and last
-// units in part); each wave owns a contiguous run of units.
+// units in part); each wave owns a contiguous run of units. Part `part` of
+// `parts` equal runs of the row's units is streamed.
 template <int FMT, bool EXT = false>
-__device__ void obs_emit(const ObsLds &L, uint8_t *row, int m, const ExtLds *X = nullptr)
+__device__ void obs_emit(const ObsLds &L, uint8_t *row, int m, int part, int parts, bool stream,
+                         const ExtLds *X = nullptr)
 {
     constexpr int ES = FMT == 0 ? 4 : FMT == 1 ? 2 : 1;
     constexpr int EPC = 16 / ES;
@@ -671,13 +663,14 @@ __device__ void obs_emit(const ObsLds &L, uint8_t *row, int m, const ExtLds *X =
     const int d2 = RG2_B + 16 + ((RG2_S + m) & 15) - RG2_S, d3 = RG3_B + 16 + ((RG3_S + m) & 15) - RG3_S;
     const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    constexpr int NW = OBS_THREADS / 64;
+    constexpr int NW = ROW_THREADS / 64;
     const uint64_t gbase = (uint64_t)(uintptr_t)(row - lead) >> 4;
     const uint64_t gA = gbase + qf, gB = gbase + ql;
     const uint64_t u0 = gA >> 6, u1 = (gB + 63) >> 6;
     const int nu = (int)(u1 - u0);
-    const int per = (nu + NW - 1) / NW;
-    const int ka = min(nu, wv * per), kb = min(nu, ka + per);
+    const int pa = nu * part / parts, pb = nu * (part + 1) / parts;
+    const int per = (pb - pa + NW - 1) / NW;
+    const int ka = min(pb, pa + wv * per), kb = min(pb, ka + per);
     const bool back = wv & 1;   // odd waves walk their run from its end, as in obs_emit_u8
     for (int i = ka; i < kb; ++i) {
         const int k = back ? ka + kb - 1 - i : i;
@@ -700,7 +693,7 @@ __device__ void obs_emit(const ObsLds &L, uint8_t *row, int m, const ExtLds *X =
                                (obs_elem<FMT, EXT>(L, e0 + 2 * i + 1, m, X) << 16);
                     }
                 }
-                row_store<FMT>(reinterpret_cast<uint4 *>(dst), make_uint4(w[0], w[1], w[2], w[3]));
+                row_store(reinterpret_cast<uint4 *>(dst), make_uint4(w[0], w[1], w[2], w[3]), stream);
             }
             continue;
         }
@@ -723,11 +716,11 @@ __device__ void obs_emit(const ObsLds &L, uint8_t *row, int m, const ExtLds *X =
             if (e0 < RG3_E && e0 + EPC > RG3_S) off = e0 + d3;
             out = obs_chunk<FMT>(L, e0, off, true);
         }
-        row_store<FMT>(reinterpret_cast<uint4 *>(dst), out);
+        row_store(reinterpret_cast<uint4 *>(dst), out, stream);
     }
     // partial chunks at the two ends of the row
-    if (threadIdx.x == 0 && lead) obs_elems<FMT, EXT>(L, row, 0, EPC - m, m, X);
-    if (threadIdx.x == 64 && ((NBYTES + lead) & 15)) obs_elems<FMT, EXT>(L, row, ql * EPC - m, OBS_ROW, m, X);
+    if (threadIdx.x == 0 && part == 0 && lead) obs_elems<FMT, EXT>(L, row, 0, EPC - m, m, X);
+    if (threadIdx.x == 64 && part == parts - 1 && ((NBYTES + lead) & 15)) obs_elems<FMT, EXT>(L, row, ql * EPC - m, OBS_ROW, m, X);
 }
 
 // Image offset of the u8 chunk starting at element e0: inside the range it
@@ -782,7 +775,9 @@ __device__ __forceinline__ void obs_emit_aux_codes(const ObsLds &L, uint8_t *row
 // u8 row emission: the row's full 16-byte chunks, in 1 KB units of the output
 // buffer split into contiguous runs, one per wave. The aux row follows, spread
 // over the block.
-__device__ __forceinline__ void obs_emit_u8(const ObsLds &L, uint8_t *row, int m, uint8_t *aux, int ct)
+template <int NTHREADS>
+__device__ __forceinline__ void obs_emit_u8(const ObsLds &L, uint8_t *row, int m, uint8_t *aux, int ct,
+                                            bool stream = true, int part = 0, int parts = 1)
 {
     const int lead = m;
     const int qf = lead ? 1 : 0, ql = (OBS_ROW + lead) >> 4;   // full chunks [qf, ql)
@@ -790,7 +785,7 @@ __device__ __forceinline__ void obs_emit_u8(const ObsLds &L, uint8_t *row, int m
     const int d2 = RG2_B + 16 + ((RG2_S + m) & 15) - RG2_S, d3 = RG3_B + 16 + ((RG3_S + m) & 15) - RG3_S;
     const int wv = __builtin_amdgcn_readfirstlane(ct >> 6);
     const int lane = ct & 63;
-    constexpr int NW = OBS_THREADS / 64;
+    constexpr int NW = NTHREADS / 64;
     // chunk q covers row bytes [q*16 - m, q*16 - m + 16): a 16-byte aligned slot
     // of the output, indexed from the aligned address below the row start
     uint4 *__restrict__ slot = reinterpret_cast<uint4 *>(__builtin_assume_aligned(row - m, 16));
@@ -801,8 +796,9 @@ __device__ __forceinline__ void obs_emit_u8(const ObsLds &L, uint8_t *row, int m
     const uint64_t gA = gbase + qf, gB = gbase + ql;
     const uint64_t u0 = gA >> 6, u1 = (gB + 63) >> 6;
     const int nu = (int)(u1 - u0);
-    const int per = (nu + NW - 1) / NW;
-    const int ka = min(nu, wv * per), kb = min(nu, ka + per);
+    const int pa = nu * part / parts, pb = nu * (part + 1) / parts;
+    const int per = (pb - pa + NW - 1) / NW;
+    const int ka = min(pb, pa + wv * per), kb = min(pb, ka + per);
     // Odd waves walk their run from its end: the runs of waves 1 and 2 (and of
     // wave 3 and the next row's wave 0) start side by side and those of waves 0
     // and 1 (2 and 3) end side by side (0.7601 -> 0.7528 ms per fused step at
@@ -814,30 +810,41 @@ __device__ __forceinline__ void obs_emit_u8(const ObsLds &L, uint8_t *row, int m
         if (g >= gA && g < gB) {
             const int q = (int)(g - gbase);
             const int e0 = q * 16 - m;
-            stream_store(&slot[q], u8_chunk(L, e0, u8_img_off(e0, d0, d1, d2, d3)));
+            row_store(&slot[q], u8_chunk(L, e0, u8_img_off(e0, d0, d1, d2, d3)), stream);
         }
     }
     // partial chunks at the two ends of the row
-    if (ct == 0 && lead) obs_elems<2>(L, row, 0, 16 - m, m);
-    if (ct == 64 && ((OBS_ROW + lead) & 15)) obs_elems<2>(L, row, ql * 16 - m, OBS_ROW, m);
+    if (ct == 0 && part == 0 && lead) obs_elems<2>(L, row, 0, 16 - m, m);
+    if (ct == 64 && part == parts - 1 && ((OBS_ROW + lead) & 15)) obs_elems<2>(L, row, ql * 16 - m, OBS_ROW, m);
     if (aux) obs_emit_aux_codes(L, aux, ct);
 }
 
 // nrows = N (one row per env, observer given or the acting seat) or 4N
-// (all_seats: row = env * 4 + observer). One 256-thread block per row. EXT
-// (f32 / bf16): belief planes from ext, (N, 4, 12, 289) float32 world-cell
-// beliefs per (env, observer). HIST: row i is row flat[i] of a rollout history
-// (S = history_state) seen by observer[i]; flat values outside [0, S.n) give
-// the empty terminated game. The block reads the ~8 KB of its history row that
-// its observer uses; a gather of the whole 36 KB row into a scratch state,
-// observed from there, took 69 us more at 4,096 bf16 rows (291.8 us a minibatch
-// with it).
+// (all_seats: row = env * 4 + observer). EXT (f32 / bf16): belief planes from
+// ext, (N, 4, 12, 289) float32 world-cell beliefs per (env, observer). HIST:
+// row i is row flat[i] of a rollout history (S = history_state) seen by
+// observer[i]; flat values outside [0, S.n) give the empty terminated game. The
+// block reads the ~8 KB of its history row that its observer uses; a gather of
+// the whole 36 KB row into a scratch state, observed from there, took 69 us
+// more at 4,096 bf16 rows.
+//
+// `parts` 512-thread blocks per row (obs_launch chooses): each builds the row in
+// its LDS and streams one of `parts` equal runs of its 1 KB units. Bound: HBM
+// writes once the grid fills the chip; below that, one block's time for its
+// loads, fill and run, which is why few rows are split over many blocks (24 f32
+// rows: 41 us in 24 blocks of 256 threads, 10.9 in 384 of 512). Eight waves per
+// block in place of four: 16,384 bf16 rows 585 -> 551 us, 24 f32 rows in one
+// part 41 -> 29 us. The row's loads are issued before the block sets up and
+// clears its LDS. Waves run at issue priority 2 from the block's start through
+// its fill and 0 while streaming, so a block that has just started gets its
+// loads and LDS work issued ahead of the stores of the blocks already
+// streaming on its SIMD.
 template <int FMT, bool EXT = false, bool HIST = false>
-__global__ __launch_bounds__(OBS_THREADS) void k_observe(State S, const int8_t *__restrict__ observer, int all_seats,
+__global__ __launch_bounds__(ROW_THREADS) void k_observe(State S, const int8_t *__restrict__ observer, int all_seats,
                                                          void *__restrict__ spatial, void *__restrict__ aux,
-                                                         float *__restrict__ glob, int nrows,
-                                                         const float *__restrict__ ext = nullptr,
-                                                         const int64_t *__restrict__ flat = nullptr)
+                                                         float *__restrict__ glob, int nrows, int parts, int stream,
+                                                         const float *__restrict__ ext,
+                                                         const int64_t *__restrict__ flat)
 {
     __shared__ ObsLds L;
     ExtLds *X = nullptr;
@@ -846,7 +853,7 @@ __global__ __launch_bounds__(OBS_THREADS) void k_observe(State S, const int8_t *
         X = &XL;
     }
     constexpr int ES = FMT == 0 ? 4 : FMT == 1 ? 2 : 1;
-    const int t = threadIdx.x, row = blockIdx.x;
+    const int t = threadIdx.x, row = (int)blockIdx.x / parts, part = (int)blockIdx.x - row * parts;
     if (row >= nrows) return;
     int env, obs;
     bool stored = true;   // the row exists (always, but for HIST)
@@ -861,30 +868,24 @@ __global__ __launch_bounds__(OBS_THREADS) void k_observe(State S, const int8_t *
     }
     uint8_t *rowp = reinterpret_cast<uint8_t *>(spatial) + (size_t)row * OBS_ROW * ES;
     const int m = (int)(((uintptr_t)rowp / ES) & (16 / ES - 1));
-    // Wave issue priority 2 from the block's start through its fill, 0 while
-    // streaming: a block that has just started gets its setup, loads and fill
-    // issued ahead of the stores of the blocks already streaming on its SIMD,
-    // and starts its own stream sooner (32,768 rows, ms per launch: bf16 1.240
-    // -> 1.220 with the fill alone raised, 1.182 from the start; f32 2.229 ->
-    // 2.210 either way)
     __builtin_amdgcn_s_setprio(2);
-    obs_setup(L, t, OBS_THREADS);
-    obs_clear(L, t, OBS_THREADS);
-    if (EXT && t < PID_STRIDE) X->rel[t] = 0;
-    lds_barrier();
     RowIn R;
     if (stored) row_fetch<HIST>(S, env, obs, t, R);
     else row_empty(R);
-    row_fill<EXT, FMT == 2>(S, obs, m, t, R, L, glob ? glob + (size_t)row * 28 : nullptr,
+    obs_setup(L, t);
+    obs_clear(L, cOBS.stat, t, ROW_THREADS);
+    if (EXT && t < PID_STRIDE) X->rel[t] = 0;
+    lds_barrier();
+    row_fill<EXT, FMT == 2>(S, obs, m, t, R, L, glob && part == 0 ? glob + (size_t)row * 28 : nullptr,
                             EXT ? ext + ((size_t)env * 4 + obs) * 12 * NC : nullptr, X);
     __builtin_amdgcn_s_setprio(0);
     lds_barrier();
-    // f32 rows: a short sleep between the fill and the stores (s_sleep 1, 2 or 4:
-    // 2.271 -> 2.230-2.237 ms per launch at 32,768 rows, three alternations;
-    // 8 / 16 / 32 2.239 / 2.249 / 2.259; bf16 and u8 rows gain nothing)
-    if (FMT == 0) __builtin_amdgcn_s_sleep(2);
-    if (FMT == 2) obs_emit_u8(L, rowp, m, aux ? static_cast<uint8_t *>(aux) + (size_t)row * AUXC_ROW : nullptr, t);
-    else obs_emit<FMT, EXT>(L, rowp, m, X);
+    if (FMT == 2)
+        obs_emit_u8<ROW_THREADS>(L, rowp, m,
+                                 aux && part == 0 ? static_cast<uint8_t *>(aux) + (size_t)row * AUXC_ROW : nullptr, t,
+                                 stream != 0, part, parts);
+    else
+        obs_emit<FMT, EXT>(L, rowp, m, part, parts, stream != 0, X);
 }
 
 // u8, persistent single-buffer form: 256 threads, one LDS row. Per row: fill
@@ -897,8 +898,8 @@ __global__ __launch_bounds__(OBS_THREADS) __attribute__((amdgpu_waves_per_eu(4, 
     __shared__ ObsLds L;
     const int t = threadIdx.x, G = gridDim.x;
     if ((int)blockIdx.x >= nrows) return;   // uniform per block
-    obs_setup(L, t, OBS_THREADS);
-    obs_clear(L, t, OBS_THREADS);
+    obs_setup(L, t);
+    obs_clear(L, cOBS.stat, t, OBS_THREADS);
     RowIn R;
     int ob = row_obs(S, observer, all_seats, blockIdx.x);
     row_fetch(S, row_env(blockIdx.x, all_seats), ob, t, R);
@@ -925,7 +926,7 @@ __global__ __launch_bounds__(OBS_THREADS) __attribute__((amdgpu_waves_per_eu(4, 
             obp = row_obs_prefetch(S, observer, all_seats, row + 2 * G, nrows);
         }
         __builtin_amdgcn_s_setprio(2);
-        obs_emit_u8(L, rowp, m, aux ? aux + (size_t)row * AUXC_ROW : nullptr, t);
+        obs_emit_u8<OBS_THREADS>(L, rowp, m, aux ? aux + (size_t)row * AUXC_ROW : nullptr, t);
         __builtin_amdgcn_s_setprio(0);
         // Each wave idles after issuing its part of the row, before the block
         // clears and refills its buffer: s_sleep 56 = 56 x 64 cycles, about
@@ -935,7 +936,7 @@ __global__ __launch_bounds__(OBS_THREADS) __attribute__((amdgpu_waves_per_eu(4, 
         // 72 0.734-0.737, 80 0.740, 96 0.749, 127 0.769).
         if (row + G < nrows) __builtin_amdgcn_s_sleep(56);
         lds_barrier();
-        obs_clear(L, t, OBS_THREADS);
+        obs_clear(L, L.k.stat, t, OBS_THREADS);
         lds_barrier();
     }
 }
