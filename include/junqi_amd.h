@@ -248,8 +248,8 @@ int jq_sample_logits(jq_env *env, const int8_t *acting, const int32_t *counts, c
  * observation). hash: device uint64 (N), each env's Zobrist hash after its ply
  * and before any restart; terminated / reward as jq_step's; actions_out the
  * action taken (world id, -1 none).
- * With a u8 observation of a large batch (more than four rows per block the device holds at
- * once: 4,096 games on 256 CUs), values_capacity >= N * JQ_MAX_LEGAL and N <= 671,088 the CSR
+ * With a u8 observation of a large batch (more than 20 rows per block the device holds at
+ * once: 20,480 games on 256 CUs), values_capacity >= N * JQ_MAX_LEGAL and N <= 671,088 the CSR
  * pass, which then also writes the canonical mask words, runs on a library-owned
  * side stream beside the observation (they share no data); `stream` waits for
  * it before the call's work counts as done, so the call stays ordered on

@@ -1340,13 +1340,78 @@ __device__ __forceinline__ int select64(uint64_t x, int k)
     return pos;
 }
 
-// Write each env's ids at its offset: pieces in ascending source order, each
-// piece's destinations ascending (compact order = flat order). Two envs per
-// wave: half h (lanes 32h .. 32h + 31) takes env 2 * block + h, which fits since
-// a seat has at most 30 movable pieces. Lane j of a half produces ids j, j + 32,
-// ...: it finds its piece from the running counts, the destination by selecting
-// a bit of that piece's mask, and maps it to a flat cell through an LDS copy of
-// the compact table.
+// One env's piece of the CSR for its group of W = 32 or 64 lanes: pieces in
+// ascending source order, each piece's destinations ascending (compact order =
+// flat order). A seat has at most 30 movable pieces, so lane p of the group
+// holds piece p.
+struct EmitPiece {
+    uint64_t m0, m1, m2;   // destinations (none past the last piece)
+    int src, cnt, seat, n;
+};
+
+// Lane p's piece of env (none when !live). The record's fields do not wait for
+// its piece count: what lies past it is dropped.
+__device__ __forceinline__ EmitPiece emit_load(const State &S, int env, int p, bool live)
+{
+    EmitPiece e = {};
+    if (!live) return e;
+    const LegalRec &G = S.lg[env];
+    const int q = p < 30 ? p : 0;
+    const int src = G.src[q];
+    const uint64_t m0 = G.mask[q][0], m1 = G.mask[q][1], m2 = G.mask[q][2];
+    e.n = min((int)G.n, 30);
+    e.seat = G.seat & 3;
+    if (p < e.n) {
+        e.src = src;
+        e.m0 = m0; e.m1 = m1; e.m2 = m2;
+        e.cnt = __popcll(m0) + __popcll(m1) + __popcll(m2);
+    }
+    return e;
+}
+
+// Write the ids of each group's env at base + 0, 1, ...: lane j of a group of W
+// produces ids j, j + W, ...: it finds its piece from the running counts (start,
+// the group's 33 LDS words), the destination by selecting a bit of that piece's
+// mask, and maps it to a flat cell through an LDS copy of the compact table.
+// MASK: each id also sets its canonical bit in the group's LDS mask words (csrc:
+// the piece's canonical source, rot: world -> canonical compact).
+template <int W, bool MASK>
+__device__ __forceinline__ void emit_ids(const EmitPiece &e, int p, const int16_t *c2f, int32_t *start, int64_t base,
+                                         int32_t *__restrict__ values, int64_t cap, int csrc = 0,
+                                         const uint8_t *rot = nullptr, uint32_t *mbits = nullptr)
+{
+    int incl = e.cnt;
+    for (int o = 1; o < 32; o <<= 1) { const int v = __shfl_up(incl, o, W); if (p >= o) incl += v; }
+    if (p < e.n) start[p] = incl - e.cnt;
+    const int total = __shfl(incl, 31, W);
+    if (p == 0) start[e.n] = total;
+    wave_sync();
+    // uniform trip count (the larger group's total): every lane takes the shuffles
+    const int trips = max(__builtin_amdgcn_readlane(total, 0), __builtin_amdgcn_readlane(total, W == 32 ? 32 : 0));
+    for (int b = 0; b < trips; b += W) {
+        const int i = b + p;
+        int j = 0;   // piece of id i: the last piece whose start is <= i
+        for (int step = 16; step >= 1; step >>= 1)
+            if (j + step < e.n && start[j + step] <= i) j += step;
+        const uint64_t w0 = __shfl(e.m0, j, W), w1 = __shfl(e.m1, j, W), w2 = __shfl(e.m2, j, W);
+        const int s = __shfl(e.src, j, W), cs = MASK ? __shfl(csrc, j, W) : 0;
+        if (i < total) {
+            const int k = i - start[j];
+            const int c0 = __popcll(w0), c1 = __popcll(w1);
+            const int c = k < c0 ? select64(w0, k)
+                                 : k < c0 + c1 ? 64 + select64(w1, k - c0) : 128 + select64(w2, k - c0 - c1);
+            if (base >= 0 && base + i < cap) values[base + i] = s * NC + c2f[c];
+            if (MASK) {   // canonical bit (rotated source) * 129 + (rotated destination)
+                const int bit = cs * NONB + rot[c];
+                atomicOr(&mbits[bit >> 5], 1u << (bit & 31));
+            }
+        }
+    }
+}
+
+// The ids of every env at its scanned offset (k_scan), two envs per wave: half h
+// (lanes 32h .. 32h + 31) takes env 2 * block + h. With mask_words the canonical
+// mask of each env is built too, in LDS.
 __global__ __launch_bounds__(64) void k_emit(State S, const int32_t *__restrict__ offsets, int32_t *__restrict__ values,
                                              int64_t cap, int32_t *__restrict__ mask_words)
 {
@@ -1355,59 +1420,92 @@ __global__ __launch_bounds__(64) void k_emit(State S, const int32_t *__restrict_
     const bool live = env < S.n;
     __shared__ int16_t c2f[NONB + 3];
     __shared__ int32_t start[2][33];   // per half: first id of each piece, start[n] = total
-    // mask_words: the canonical mask of each half's env is built here, in LDS
     __shared__ uint32_t mbits[2][JQ_MASK_WORDS_PAD];
     __shared__ uint8_t rot[2][NONB + 3];   // world compact -> canonical compact of the env's acting seat
     for (int c = l; c < NONB; c += 64) c2f[c] = cT.c2f[c];
-    const int n = live ? min((int)S.lg[env].n, 30) : 0;
-    const int seat = live ? (S.lg[env].seat & 3) : 0;
-    if (mask_words) {
-        for (int w = p; w < JQ_MASK_WORDS_PAD; w += 32) mbits[h][w] = 0;
-        for (int c = p; c < NONB; c += 32) rot[h][c] = cT.rotc[seat][c];
+    const EmitPiece e = emit_load(S, env, p, live);
+    const int64_t base = live ? offsets[env] : 0;
+    if (!mask_words) {
+        emit_ids<32, false>(e, p, c2f, start[h], base, values, cap);
+        return;
     }
-    int cnt = 0, src = 0, csrc = 0;   // csrc: the source's canonical compact index
-    uint64_t m0 = 0, m1 = 0, m2 = 0;
-    if (p < n) {
-        const LegalRec &G = S.lg[env];
-        src = G.src[p];
-        m0 = G.mask[p][0]; m1 = G.mask[p][1]; m2 = G.mask[p][2];
-        cnt = __popcll(m0) + __popcll(m1) + __popcll(m2);
-        if (mask_words) csrc = cT.canc[seat][src];
-    }
-    int incl = cnt;
-    for (int o = 1; o < 32; o <<= 1) { const int v = __shfl_up(incl, o, 32); if (p >= o) incl += v; }
-    if (p < n) start[h][p] = incl - cnt;
-    const int total = __shfl(incl, 31, 32);
-    if (p == 0) start[h][n] = total;
-    const int base = live ? offsets[env] : 0;
-    __syncthreads();
-    // uniform trip count (the larger half's total): every lane takes the shuffles
-    const int trips = max(__builtin_amdgcn_readlane(total, 0), __builtin_amdgcn_readlane(total, 32));
-    for (int b = 0; b < trips; b += 32) {
-        const int i = b + p;
-        int j = 0;   // piece of id i: the last piece whose start is <= i
-        for (int step = 16; step >= 1; step >>= 1)
-            if (j + step < n && start[h][j + step] <= i) j += step;
-        const uint64_t w0 = __shfl(m0, j, 32), w1 = __shfl(m1, j, 32), w2 = __shfl(m2, j, 32);
-        const int s = __shfl(src, j, 32), cs = __shfl(csrc, j, 32);
-        if (i < total) {
-            const int k = i - start[h][j];
-            const int c0 = __popcll(w0), c1 = __popcll(w1);
-            const int c = k < c0 ? select64(w0, k)
-                                 : k < c0 + c1 ? 64 + select64(w1, k - c0) : 128 + select64(w2, k - c0 - c1);
-            if (base >= 0 && (int64_t)base + i < cap) values[base + i] = s * NC + c2f[c];
-            if (mask_words) {   // canonical bit (rotated source) * 129 + (rotated destination)
-                const int bit = cs * NONB + rot[h][c];
-                atomicOr(&mbits[h][bit >> 5], 1u << (bit & 31));
-            }
+    for (int w = p; w < JQ_MASK_WORDS_PAD; w += 32) mbits[h][w] = 0;
+    for (int c = p; c < NONB; c += 32) rot[h][c] = cT.rotc[e.seat][c];
+    const int csrc = cT.canc[e.seat][e.src];
+    emit_ids<32, true>(e, p, c2f, start[h], base, values, cap, csrc, rot[h], mbits[h]);
+    wave_sync();
+    if (live)
+        for (int w = p; w < JQ_MASK_WORDS; w += 32)
+            stream_store(mask_words + (size_t)env * JQ_MASK_WORDS + w, (int32_t)mbits[h][w]);
+}
+
+// Scan and emit in one pass of CSR_THREADS-thread blocks: a block sums the
+// counts of all envs before its own, writes its envs' offsets and then their
+// ids, one env per wave and pass. For batches whose ids always fit the buffer
+// (no total to read back).
+// Why: k_scan is one block, 6.2 us however few the envs, and k_emit waits for
+// it. The blocks read the counts again and again (n * n / (8 * passes) words in
+// all, from L2), so larger batches take more envs per block.
+constexpr int CSR_THREADS = 512, CSR_WAVES = CSR_THREADS / 64, CSR_MOST_PASSES = 4;
+struct CsrArgs {
+    const int32_t *counts;
+    int32_t *offsets, *values;
+    int64_t cap;
+    int passes;   // envs per wave
+    int blocks;   // of a launch: 0 = no CSR pass in it
+};
+
+struct CsrLds {
+    int32_t start[CSR_WAVES][33];
+    int32_t wsum[CSR_WAVES];
+    int16_t c2f[NONB + 3];
+};
+
+__device__ __forceinline__ void csr_block(const State &S, const CsrArgs &A, int block, CsrLds &L)
+{
+    const int t = threadIdx.x, l = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int envs = CSR_WAVES * A.passes, e0 = block * envs;   // wave w: envs e0 + w, e0 + w + 8, ...
+    EmitPiece e = emit_load(S, e0 + w, l, e0 + w < S.n);
+    const int own = l < envs && e0 + l < S.n ? A.counts[e0 + l] : 0;   // the block's counts, in every wave
+    int sum = 0;
+    if ((reinterpret_cast<uintptr_t>(A.counts) & 15) == 0) {
+        const int4 *c4 = reinterpret_cast<const int4 *>(A.counts);
+        for (int i = t; i < e0 / 4; i += CSR_THREADS) {
+            const int4 v = c4[i];
+            sum += (v.x + v.y) + (v.z + v.w);
         }
+    } else {
+        for (int i = t; i < e0; i += CSR_THREADS) sum += A.counts[i];
     }
-    if (mask_words) {
-        __syncthreads();
-        if (live)
-            for (int w = p; w < JQ_MASK_WORDS; w += 32)
-                stream_store(mask_words + (size_t)env * JQ_MASK_WORDS + w, (int32_t)mbits[h][w]);
+    sum = wave_sum(sum);
+    if (l == 0) L.wsum[w] = sum;
+    if (t < NONB) L.c2f[t] = cT.c2f[t];
+    lds_barrier();
+    int before = 0;
+#pragma unroll
+    for (int k = 0; k < CSR_WAVES; ++k) before += L.wsum[k];
+    int incl = own;
+    for (int o = 1; o < CSR_WAVES * CSR_MOST_PASSES; o <<= 1) { const int v = __shfl_up(incl, o); if (l >= o) incl += v; }
+    const int first = before + incl - own;   // lane j: offset of env e0 + j
+    if (w == 0 && l < envs && e0 + l < S.n) {
+        A.offsets[e0 + l] = first;
+        if (e0 + l == S.n - 1) A.offsets[S.n] = first + own;
     }
+    for (int k = 0; k < A.passes; ++k) {
+        if (k) {
+            const int env = e0 + w + CSR_WAVES * k;
+            e = emit_load(S, env, l, env < S.n);
+            wave_sync();   // the last pass's reads of `start` are done
+        }
+        const int base = __builtin_amdgcn_readlane(first, w + CSR_WAVES * k);
+        emit_ids<64, false>(e, l, L.c2f, L.start[w], base, A.values, A.cap);
+    }
+}
+
+__global__ __launch_bounds__(CSR_THREADS) void k_csr(State S, CsrArgs A)
+{
+    __shared__ CsrLds L;
+    csr_block(S, A, blockIdx.x, L);
 }
 
 // ------------------------------------------------------------------ slot mask

@@ -27,8 +27,6 @@ struct jq_env {
     State S{};
     std::vector<void *> allocs;
     bool zob_ready = false, rlut_ready = false;
-    int obs_blocks = 0;              // resident u8 observation blocks on the device
-    int cus = 0;                     // compute units of the device
     float *ext_bel = nullptr;        // uploaded (N, 4, 12, 289) beliefs, allocated on first upload
     bool ext_on = false;             // observations read the uploaded beliefs
     int8_t *pool = nullptr;          // setup pool buffer (reused while uploads fit)
@@ -50,7 +48,6 @@ struct jq_history {
     std::vector<void *> allocs;
     float *rlut = nullptr;           // recency table copied from the snapshotted handle
     bool rlut_ready = false;
-    int cus = 0;                     // compute units of the device
 };
 
 namespace {
@@ -74,8 +71,15 @@ int fail(int code, const char *fmt, ...)
         if (e_ != hipSuccess) return fail(JQ_E_HIP, "%s: %s", #expr, hipGetErrorString(e_)); \
     } while (0)
 
+// What launches need to know of a device, asked once (ensure_device_tables).
+struct DeviceInfo {
+    int cus = 0;          // compute units
+    int obs_blocks = 0;   // k_observe_u8_persist blocks the device holds at once
+};
+
 std::mutex g_tab_mu;
 bool g_tab_done[64] = {};
+DeviceInfo g_dev[64];     // written once per device under g_tab_mu, before any handle of the device exists
 Tables g_tables;
 bool g_host_tables = false;
 uint8_t g_bval[BC_COUNT][12];
@@ -155,6 +159,11 @@ int ensure_device_tables(int device)
     HIP_TRY(hipMemcpyToSymbol(HIP_SYMBOL(cT), &g_tables, sizeof g_tables));
     const ObsConsts oc = build_obs_consts();
     HIP_TRY(hipMemcpyToSymbol(HIP_SYMBOL(cOBS), &oc, sizeof oc));
+    int per_cu = 0, cus = 0;
+    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_observe_u8_persist, OBS_THREADS, 0));
+    HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+    g_dev[device].cus = std::max(1, cus);
+    g_dev[device].obs_blocks = std::max(1, per_cu) * g_dev[device].cus;
     g_tab_done[device] = true;
     return JQ_OK;
 }
@@ -250,6 +259,21 @@ bool csr_always_fits(const jq_env *e, int64_t cap)
     return bound <= (int64_t)INT32_MAX && cap >= bound;
 }
 
+// Offsets and ids in one pass (csr_block) up to CSR_SCAN_MAX envs, with more envs
+// per wave as the batch grows. us of the CSR pass in jq_legal, k_scan + k_emit /
+// 1 / 2 / 4 envs per wave: 64 envs 12.0 / 4.6 / 6.5 / 9.9, 4,096 13.1 / 6.1 /
+// 7.0 / 10.9, 8,192 14.2 / 7.6 / 8.6 / 11.3, 16,384 17.1 / 13.3 / 11.9 / 13.7,
+// 32,768 23.2 / 26.3 / 22.2 / 20.3.
+constexpr int CSR_SCAN_MAX = 32768;
+bool csr_one_pass(const jq_env *e, int64_t cap) { return e->S.n <= CSR_SCAN_MAX && csr_always_fits(e, cap); }
+
+CsrArgs csr_args(const jq_env *e, const int32_t *counts, int32_t *offsets, int32_t *values, int64_t cap)
+{
+    const int n = e->S.n;
+    const int passes = n <= 8192 ? 1 : n <= 24576 ? 2 : CSR_MOST_PASSES, envs = CSR_WAVES * passes;
+    return {counts, offsets, values, cap, passes, (n + envs - 1) / envs};
+}
+
 // CSR capacity check of jq_legal / jq_env_step: unless csr_always_fits, the
 // total (offsets[n], just scanned on `s`; -1 when it exceeds the int32 offsets)
 // is read back and must fit.
@@ -284,36 +308,13 @@ int launch_check(const char *what)
     return JQ_OK;
 }
 
-int device_cus(int device, int &cus)
-{
-    if (cus > 0) return JQ_OK;
-    int n = 0;
-    HIP_TRY(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device));
-    cus = std::max(1, n);
-    return JQ_OK;
-}
-
-// Persistent grid of the u8 observation kernel: every block the device can
-// hold at once.
-int obs_u8_grid(jq_env *e)
-{
-    if (e->obs_blocks > 0) return JQ_OK;
-    int per_cu = 0;
-    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_observe_u8_persist, OBS_THREADS, 0));
-    int rc = device_cus(e->device, e->cus);
-    if (rc) return rc;
-    e->obs_blocks = std::max(1, per_cu) * e->cus;
-    return JQ_OK;
-}
-
-// u8 rows (one per env) go through the persistent kernel from more than four
-// rows per resident block on: its prefetch of the next row's inputs hides their
+// u8 rows (one per env) go through the persistent kernel from more than 20 rows
+// per resident block on: its prefetch of the next row's inputs hides their
 // loads, which come from memory after a step's gigabytes of stores, and its tail
-// takes the CSR pass. Below that k_observe, with the CSR pass in line, is
-// faster (us per fused u8 step, persistent -> k_observe: 64 games 50.6 -> 40.3,
-// 1,024 65.4 -> 57.4, 4,096 118.4 -> 116.2, 16,384 364 -> 381, 32,768
-// 709 -> 751).
-bool obs_persists(const jq_env *e) { return e->S.n > 4 * e->obs_blocks; }
+// takes the CSR pass. Below that k_observe, with the CSR pass in its launch, is
+// faster (us per fused u8 step, persistent / k_observe: 4,096 games 118 / 105,
+// 8,192 208 / 189, 16,384 379 / 369, 24,000 517 / 537, 32,768 712 / 735).
+bool obs_persists(const jq_env *e) { return e->S.n > 20 * g_dev[e->device].obs_blocks; }
 
 // How k_observe runs `nrows` rows of format `fmt` on a device with `cus` CUs:
 // blocks per row, and streaming or ordinary stores.
@@ -604,6 +605,11 @@ int jq_legal(jq_env *e, const int8_t *acting, int32_t *counts, int32_t *offsets,
     hipLaunchKernelGGL(k_legal<>, dim3(e->S.n), dim3(64), 0, strm(stream), e->S, acting, counts, mask_words, mask_bool,
                        nullptr);
     if ((rc = launch_check("k_legal")) != 0) return rc;
+    if (values && csr_one_pass(e, values_capacity)) {
+        const CsrArgs A = csr_args(e, counts, offsets, values, values_capacity);
+        hipLaunchKernelGGL(k_csr, dim3(A.blocks), dim3(CSR_THREADS), 0, strm(stream), e->S, A);
+        return launch_check("k_csr");
+    }
     if (offsets) {
         hipLaunchKernelGGL(k_scan, dim3(1), dim3(SCAN_THREADS), 0, strm(stream), counts, offsets, e->S.n);
         if ((rc = launch_check("k_scan")) != 0) return rc;
@@ -630,35 +636,42 @@ int jq_legal_slots(jq_env *e, const int8_t *acting, uint8_t *slots, void *stream
     return launch_check("k_slots");
 }
 
-int jq_observe(jq_env *e, const int8_t *observer, int32_t fmt, int32_t all_seats, void *spatial, void *aux,
-               float *global, void *stream)
+// jq_observe; `csr` (blocks > 0, k_observe formats without uploaded beliefs):
+// the env-step's CSR pass rides in the same launch.
+static int observe(jq_env *e, const int8_t *observer, int32_t fmt, int32_t all_seats, void *spatial, void *aux,
+                   float *global, const CsrArgs &csr, void *stream)
 {
     int rc = check_env(e);
     if (rc) return rc;
     if ((rc = obs_args(e->rlut_ready, e->ext_on, fmt, spatial, aux, global)) != 0) return rc;
     const int nrows = all_seats ? e->S.n * 4 : e->S.n;
-    if ((rc = obs_u8_grid(e)) != 0) return rc;
     hipEvent_t t_end = e->obs_t_end;   // begin already recorded by jq_env_step
     e->obs_t_end = nullptr;
     if (!t_end && (rc = obs_timing_begin(e, stream, &t_end)) != 0) return rc;
-    if (fmt == JQ_OBS_U8 && !all_seats && obs_persists(e)) {
-        hipLaunchKernelGGL(k_observe_u8_persist, dim3(std::min(nrows, e->obs_blocks)), dim3(OBS_THREADS), 0,
+    if (fmt == JQ_OBS_U8 && !all_seats && !csr.blocks && obs_persists(e)) {
+        hipLaunchKernelGGL(k_observe_u8_persist, dim3(std::min(nrows, g_dev[e->device].obs_blocks)), dim3(OBS_THREADS), 0,
                            strm(stream), e->S, observer, all_seats, static_cast<uint8_t *>(spatial),
                            static_cast<uint8_t *>(aux), global, nrows);
     } else {
-        const ObsPlan p = obs_plan(fmt, nrows, e->cus);
+        const ObsPlan p = obs_plan(fmt, nrows, g_dev[e->device].cus);
         auto *kernel = fmt == JQ_OBS_U8 ? &k_observe<2>
                        : fmt == JQ_OBS_BF16 ? (e->ext_on ? &k_observe<1, true> : &k_observe<1>)
                                             : (e->ext_on ? &k_observe<0, true> : &k_observe<0>);
-        hipLaunchKernelGGL(kernel, dim3((unsigned)nrows * p.parts), dim3(ROW_THREADS), 0, strm(stream), e->S, observer,
-                           all_seats, spatial, aux, global, nrows, p.parts, p.stream,
-                           static_cast<const float *>(e->ext_bel), nullptr);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nrows * p.parts + csr.blocks), dim3(ROW_THREADS), 0, strm(stream), e->S,
+                           observer, all_seats, spatial, aux, global, nrows, p.parts, p.stream,
+                           static_cast<const float *>(e->ext_bel), nullptr, csr);
     }
     rc = launch_check("k_observe");
     // the end event follows its begin event even when the launch failed, so no
     // later launch is paired with it
     if (t_end) HIP_TRY(hipEventRecord(t_end, strm(stream)));
     return rc;
+}
+
+int jq_observe(jq_env *e, const int8_t *observer, int32_t fmt, int32_t all_seats, void *spatial, void *aux,
+               float *global, void *stream)
+{
+    return observe(e, observer, fmt, all_seats, spatial, aux, global, CsrArgs{}, stream);
 }
 
 int jq_obs_timing(jq_env *e, int32_t enable)
@@ -767,7 +780,6 @@ int jq_env_step(jq_env *e, const int32_t *actions, int32_t sampler, uint64_t sam
     A.do_reset = e->S.pool ? 1 : 0; A.reset_seed = reset_seed; A.counts = counts;
     // The overlapped form moves the CSR pass, and the canonical mask with it,
     // beside the observation (below); the step kernel then skips the mask.
-    if ((rc = obs_u8_grid(e)) != 0) return rc;
     const bool overlap = spatial && obs_fmt == JQ_OBS_U8 && obs_persists(e) && csr_always_fits(e, values_capacity);
     A.mask_words = overlap ? nullptr : mask_words;
     // sample (unless actions are given), ply, restart from the pool and the
@@ -815,6 +827,14 @@ int jq_env_step(jq_env *e, const int32_t *actions, int32_t sampler, uint64_t sam
         rc = jq_observe(e, nullptr, obs_fmt, 0, spatial, aux, global, stream);
         HIP_TRY(hipStreamWaitEvent(strm(stream), e->ev_csr, 0));   // joined even if the observation failed
         return rc;
+    }
+    if (csr_one_pass(e, values_capacity)) {
+        // in the observation's launch, or one of its own
+        const CsrArgs C = csr_args(e, counts, offsets, values, values_capacity);
+        if (spatial && !e->ext_on) return observe(e, nullptr, obs_fmt, 0, spatial, aux, global, C, stream);
+        hipLaunchKernelGGL(k_csr, dim3(C.blocks), dim3(CSR_THREADS), 0, strm(stream), e->S, C);
+        if ((rc = launch_check("k_csr")) != 0) return rc;
+        return spatial ? jq_observe(e, nullptr, obs_fmt, 0, spatial, aux, global, stream) : JQ_OK;
     }
     hipLaunchKernelGGL(k_scan, dim3(1), dim3(SCAN_THREADS), 0, strm(stream), counts, offsets, e->S.n);
     if ((rc = launch_check("k_scan")) != 0) return rc;
@@ -927,13 +947,14 @@ int jq_history_create(jq_history **out, int32_t num_envs, int32_t num_steps, int
     HIP_TRY(hipGetDeviceCount(&ndev));
     if (device < 0 || device >= ndev) return fail(JQ_E_ARG, "device %d not present (%d devices)", device, ndev);
     HIP_TRY(hipSetDevice(device));
+    int rc = ensure_device_tables(device);
+    if (rc) return rc;
     jq_history *h = new jq_history();
     h->device = device;
     h->show_mode = show_mode;
     HistState &H = h->H;
     H.steps = num_steps; H.n = num_envs;
     const size_t R = (size_t)num_steps * num_envs;
-    int rc;
 #define A(ptr, cnt) do { if ((rc = halloc(h, ptr, cnt)) != 0) { jq_history_destroy(h); return rc; } } while (0)
     A(H.cell, R * CELL_STRIDE);
     A(H.piece, R * PID_STRIDE);
@@ -1002,12 +1023,11 @@ static int history_rebuild(jq_history *h, const int64_t *flat, const int8_t *obs
     if (spatial || aux || global) {
         if (!spatial || !global) return fail(JQ_E_ARG, "spatial and global outputs go together");
         if ((rc = obs_args(true, false, fmt, spatial, aux, global)) != 0) return rc;
-        if ((rc = device_cus(h->device, h->cus)) != 0) return rc;
-        const ObsPlan p = obs_plan(fmt, batch, h->cus);
+        const ObsPlan p = obs_plan(fmt, batch, g_dev[h->device].cus);
         auto *kernel = fmt == JQ_OBS_F32 ? &k_observe<0, false, true>
                                          : fmt == JQ_OBS_BF16 ? &k_observe<1, false, true> : &k_observe<2, false, true>;
         hipLaunchKernelGGL(kernel, dim3((unsigned)batch * p.parts), dim3(ROW_THREADS), 0, strm(stream), S, observer, 0,
-                           spatial, aux, global, batch, p.parts, p.stream, nullptr, flat);
+                           spatial, aux, global, batch, p.parts, p.stream, nullptr, flat, CsrArgs{});
         if ((rc = launch_check("k_observe")) != 0) return rc;
     }
     if (mask_words || mask_bool) {

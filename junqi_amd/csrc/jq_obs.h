@@ -839,14 +839,28 @@ __device__ __forceinline__ void obs_emit_u8(const ObsLds &L, uint8_t *row, int m
 // its fill and 0 while streaming, so a block that has just started gets its
 // loads and LDS work issued ahead of the stores of the blocks already
 // streaming on its SIMD.
+// csr: an env-step's CSR pass rides in the launch as its last blocks, which run
+// while the last rows stream (us per fused step, k_csr before it / the grid's
+// first blocks / its last: u8 64 games 31.8 / 27.2 / 27.0, bf16 16,384
+// 630 / 628 / 617).
+// bf16 needs its register budget stated: it took scalar registers for 7
+// waves per SIMD, which holds 3 blocks per CU instead of 4 (16,384-game bf16 step 728 -> 650 us).
 template <int FMT, bool EXT = false, bool HIST = false>
-__global__ __launch_bounds__(ROW_THREADS) void k_observe(State S, const int8_t *__restrict__ observer, int all_seats,
+__global__ __launch_bounds__(ROW_THREADS) __attribute__((amdgpu_waves_per_eu(FMT == 1 && !EXT && !HIST ? 8 : 1))) void k_observe(State S, const int8_t *__restrict__ observer, int all_seats,
                                                          void *__restrict__ spatial, void *__restrict__ aux,
                                                          float *__restrict__ glob, int nrows, int parts, int stream,
                                                          const float *__restrict__ ext,
-                                                         const int64_t *__restrict__ flat)
+                                                         const int64_t *__restrict__ flat, CsrArgs csr)
 {
     __shared__ ObsLds L;
+    if constexpr (!EXT && !HIST) {   // an env-step's CSR pass: the grid's last blocks
+        static_assert(sizeof(CsrLds) <= sizeof(ObsLds) && CSR_THREADS == ROW_THREADS, "shares the block");
+        const int cb = (int)blockIdx.x - nrows * parts;
+        if (cb >= 0) {
+            csr_block(S, csr, cb, reinterpret_cast<CsrLds &>(L));
+            return;
+        }
+    }
     ExtLds *X = nullptr;
     if constexpr (EXT) {
         __shared__ ExtLds XL;
