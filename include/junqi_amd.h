@@ -371,7 +371,7 @@ int jq_history_reconstruct_noalloc(jq_history *hist, const int64_t *flat, const 
  * (junqi_rl/training/rollout_gpu.py:119-198). jq_mask_count: counts (device
  * int32, n) = nonzero bytes of each row of a dense (n, d) uint8 mask.
  * jq_mask_to_ids: ids (device int32, (n, k_max)) = each row's nonzero columns in
- * order, then zeros; every count must be <= k_max (check jq_mask_count first:
+ * order, then zeros; columns past the k_max-th are dropped (check jq_mask_count first:
  * _dense_mask_to_csr raises before it writes, rollout_gpu.py:119-167).
  * jq_ids_to_mask: out (device uint8, (batch, d)) = rows idx (device int64,
  * batch) of the (rows, k_max) id lists with their counts as dense rows; ids
@@ -380,6 +380,14 @@ int jq_history_reconstruct_noalloc(jq_history *hist, const int64_t *flat, const 
  * device. */
 int jq_mask_count(const uint8_t *mask, int32_t n, int32_t d, int32_t *counts, void *stream);
 int jq_mask_to_ids(const uint8_t *mask, int32_t n, int32_t d, int32_t k_max, int32_t *ids, void *stream);
+/* jq_mask_to_ids and the counts in one go, published only if every row fits:
+ * the rows are encoded into work_ids (device int32, n * k_max) and work_counts
+ * (n, 16-byte aligned); most (one int32, device or mapped host memory) gets the
+ * largest count, and when that is at most
+ * k_max ids (n, k_max) and counts (n) take the result, else they keep their
+ * contents (_dense_mask_to_csr's guard, rollout_gpu.py:119-167). n >= 1. */
+int jq_mask_encode(const uint8_t *mask, int32_t n, int32_t d, int32_t k_max, int32_t *work_ids, int32_t *work_counts,
+                   int32_t *ids, int32_t *counts, int32_t *most, void *stream);
 int jq_ids_to_mask(const int32_t *ids, const int32_t *counts, int64_t rows, int32_t k_max, const int64_t *idx,
                    int32_t batch, int32_t d, uint8_t *out, void *stream);
 

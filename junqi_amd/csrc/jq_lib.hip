@@ -1074,8 +1074,24 @@ int jq_mask_to_ids(const uint8_t *mask, int32_t n, int32_t d, int32_t k_max, int
     if (!mask || !ids) return fail(JQ_E_ARG, "null device pointer");
     if (n < 0 || d <= 0 || k_max <= 0) return fail(JQ_E_ARG, "bad shapes (n %d, d %d, k_max %d)", n, d, k_max);
     if (n == 0) return JQ_OK;
-    hipLaunchKernelGGL(k_mask_to_ids, dim3(n), dim3(64), 0, strm(stream), mask, n, d, k_max, ids);
+    hipLaunchKernelGGL(k_mask_to_ids, dim3(n), dim3(64), 0, strm(stream), mask, n, d, k_max, ids, nullptr);
     return launch_check("k_mask_to_ids");
+}
+
+int jq_mask_encode(const uint8_t *mask, int32_t n, int32_t d, int32_t k_max, int32_t *work_ids, int32_t *work_counts,
+                   int32_t *ids, int32_t *counts, int32_t *most, void *stream)
+{
+    if (!mask || !work_ids || !work_counts || !ids || !counts || !most) return fail(JQ_E_ARG, "null device pointer");
+    if (n <= 0 || d <= 0 || k_max <= 0) return fail(JQ_E_ARG, "bad shapes (n %d, d %d, k_max %d)", n, d, k_max);
+    if ((uintptr_t)work_counts % 16) return fail(JQ_E_ARG, "work_counts must be 16-byte aligned");
+    hipLaunchKernelGGL(k_mask_to_ids, dim3(n), dim3(64), 0, strm(stream), mask, n, d, k_max, work_ids, work_counts);
+    int rc = launch_check("k_mask_to_ids");
+    if (rc) return rc;
+    const int64_t quads = ((int64_t)n * k_max + 3) / 4;
+    const int blocks = (int)std::min<int64_t>(MASK_COMMIT_BLOCKS, (quads + MASK_COMMIT_THREADS - 1) / MASK_COMMIT_THREADS);
+    hipLaunchKernelGGL(k_mask_commit, dim3(blocks), dim3(MASK_COMMIT_THREADS), 0, strm(stream), work_ids, work_counts, n, k_max, ids,
+                       counts, most);
+    return launch_check("k_mask_commit");
 }
 
 int jq_ids_to_mask(const int32_t *ids, const int32_t *counts, int64_t rows, int32_t k_max, const int64_t *idx,

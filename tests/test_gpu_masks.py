@@ -89,3 +89,30 @@ def test_round_trip_of_legal_masks(masks):
     back = masks.csr_to_dense_selected(ids, cnt, torch.arange(24, device="cuda"), D)
     assert torch.equal(back, lm)
     b.close()
+
+
+@pytest.mark.parametrize("d", [1, 15, 16, 17, 1040, 9216, 9217, 16641, 20011])
+@pytest.mark.parametrize("n,k_max,shift", [(1, 5, 0), (67, 77, 1), (700, 256, 2)])
+def test_encode_row_shapes(masks, d, n, k_max, shift):
+    """Row lengths around the walk's 16-byte words, 1 KB steps and rounds, row
+    starts at every alignment, outputs off the 16-byte grid, nonzero bytes of
+    every value; then one row too many leaves the outputs as they were."""
+    rng = np.random.default_rng(d * 1000 + n)
+    m = np.zeros((n, d), np.uint8)
+    for r in range(n):
+        cnt = int(rng.integers(0, min(d, k_max) + 1))
+        m[r, rng.choice(d, cnt, replace=False)] = rng.integers(1, 256, cnt)
+    want_ids, want_counts = _np_csr(m != 0, k_max)
+    store = torch.full((n * k_max + 8,), -7, dtype=torch.int32, device="cuda")
+    ids = store[shift:shift + n * k_max].view(n, k_max)
+    counts = torch.full((n,), -7, dtype=torch.int32, device="cuda")
+    dm = torch.from_numpy(m).cuda().view(torch.bool)
+    masks.dense_mask_to_csr(dm, ids, counts)
+    assert np.array_equal(counts.cpu().numpy(), want_counts) and np.array_equal(ids.cpu().numpy(), want_ids)
+    assert (store[:shift] == -7).all() and (store[shift + n * k_max:] == -7).all()
+    if d > k_max:
+        m[n - 1] = 255
+        before = store.clone()
+        with pytest.raises(ValueError, match=f"need {d} entries"):
+            masks.dense_mask_to_csr(torch.from_numpy(m).cuda().view(torch.bool), ids, counts)
+        assert torch.equal(store, before) and np.array_equal(counts.cpu().numpy(), want_counts)
