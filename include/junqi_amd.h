@@ -165,6 +165,23 @@ int jq_step(jq_env *env, const int32_t *actions, const int8_t *acting, int32_t a
 int jq_legal(jq_env *env, const int8_t *acting, int32_t *counts, int32_t *offsets, int32_t *values,
              int64_t values_capacity, int32_t *mask_words, uint8_t *mask_bool, void *stream);
 
+/* The host-array forms of a ply and of the legal sets, for agents driven from
+ * host memory; inputs and outputs below are host pointers unless said otherwise,
+ * and each call returns when its results are in them.
+ * jq_step_host: jq_step with JQ_ACT_WORLD actions (N); any output (N each) may be
+ * NULL (MoveResultBatch, junqi_rl/gpu_rollout.py:765-778).
+ * jq_legal_dense_host: jq_legal of `acting` (N; NULL = current turn) into the
+ * device buffers counts / offsets / values, then ids (N, width) = each env's
+ * ascending ids, cut at width, -1 padded, and counts_out (N) the full counts
+ * (legal_actions_dense, junqi_rl/gpu_rollout.py:854-860).
+ * jq_env_flags_host: each env's seat to move and termination flags, any NULL;
+ * waits for the device first, as jq_get_field does. */
+int jq_step_host(jq_env *env, const int32_t *actions, uint8_t *valid, int8_t *event, uint8_t *terminated,
+                 int8_t *winner, uint8_t *draw, uint8_t *flag_captured, void *stream);
+int jq_legal_dense_host(jq_env *env, const int8_t *acting, int32_t *counts, int32_t *offsets, int32_t *values,
+                        int64_t values_capacity, int32_t width, int32_t *ids, int32_t *counts_out, void *stream);
+int jq_env_flags_host(jq_env *env, int8_t *turn, uint8_t *terminated, int8_t *winner, uint8_t *draw);
+
 /* Per-piece slot mask of `acting` (device int8 N; NULL = current turn):
  * slots: device uint8 (N, 120, 80), 16-byte aligned; slots[i][pid][s] = 1 iff
  * piece pid can take slot s. Slots 0-3 road steps (+x,-x,+y,-y), 4-7 camp

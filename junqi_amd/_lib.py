@@ -48,7 +48,7 @@ _EXPORTS = [
     "jq_sample_uniform", "jq_sample_logits",
     "jq_env_step", "jq_field_info", "jq_get_field", "jq_set_field", "jq_field_ptr", "jq_finalize_import",
     "jq_finalize_import_masked", "jq_rehash", "jq_validate_lineup",
-    "jq_sync", "jq_history_create", "jq_history_destroy", "jq_history_bytes", "jq_history_snapshot",
+    "jq_sync", "jq_step_host", "jq_legal_dense_host", "jq_env_flags_host", "jq_history_create", "jq_history_destroy", "jq_history_bytes", "jq_history_snapshot",
     "jq_history_reconstruct", "jq_history_reconstruct_noalloc", "jq_mask_count", "jq_mask_to_ids", "jq_mask_encode", "jq_ids_to_mask", "jq_upload_beliefs",
     "jq_clear_beliefs",
 ]
@@ -105,6 +105,9 @@ def bind(L: C.CDLL) -> C.CDLL:
         "jq_finalize_import": ([P, P], C.c_int), "jq_finalize_import_masked": ([P, P, P], C.c_int),
         "jq_rehash": ([P, P], C.c_int),
         "jq_sync": ([P], C.c_int),
+        "jq_step_host": ([P, P, P, P, P, P, P, P, P], C.c_int),
+        "jq_legal_dense_host": ([P, P, P, P, P, I64, I32, P, P, P], C.c_int),
+        "jq_env_flags_host": ([P, P, P, P, P], C.c_int),
         "jq_history_create": ([C.POINTER(P), I32, I32, I32, I32], C.c_int),
         "jq_history_destroy": ([P], C.c_int), "jq_history_bytes": ([P, C.POINTER(I64)], C.c_int),
         "jq_history_snapshot": ([P, P, P, I32, P], C.c_int),

@@ -144,6 +144,7 @@ class JunqiBatch:
         self.offsets = torch.zeros(self.n + 1, dtype=torch.int32, device=dev)
         self.values = torch.zeros(self.n * L.MAX_LEGAL, dtype=torch.int32, device=dev)
         self.mask_words = torch.zeros((self.n, L.MASK_WORDS), dtype=torch.int32, device=dev)
+        self._turn_view = self.field_tensor("turn")
 
     # ------------------------------------------------------------ lifetime
     def close(self) -> None:
@@ -160,6 +161,17 @@ class JunqiBatch:
     @property
     def stream(self) -> int:
         return torch.cuda.current_stream(self.device).cuda_stream
+
+    def _seats(self, t: torch.Tensor | None) -> torch.Tensor | None:
+        """Seats as the library takes them: contiguous int8 on this device, or
+        None (the current turn) for the live turn view itself, which the kernels
+        then read in the env records instead of through a copy of them."""
+        if t is None:
+            return None
+        v = self._turn_view
+        if t.dtype is torch.int8 and t.data_ptr() == v.data_ptr() and t.shape == v.shape and t.stride() == v.stride():
+            return None
+        return t.to(device=self.device, dtype=torch.int8).contiguous()
 
     @staticmethod
     def _ptr(t: torch.Tensor | None) -> int | None:
@@ -187,12 +199,10 @@ class JunqiBatch:
         a = actions.to(device=self.device, dtype=torch.int32).contiguous()
         if a.shape != (self.n,):
             raise ValueError(f"actions: expected ({self.n},), got {tuple(a.shape)}")
-        s = None
-        if acting is not None:
-            s = acting.to(device=self.device, dtype=torch.int8).contiguous()
-            if s.shape != (self.n,):
-                raise ValueError(f"acting: expected ({self.n},), got {tuple(s.shape)}")
-        if canonical and s is None:
+        s = self._seats(acting)
+        if s is not None and s.shape != (self.n,):
+            raise ValueError(f"acting: expected ({self.n},), got {tuple(s.shape)}")
+        if canonical and acting is None:
             raise ValueError("canonical actions need the acting seats")
         dev, n = self.device, self.n
         out = {
@@ -216,7 +226,7 @@ class JunqiBatch:
     # ------------------------------------------------------------ legal actions
     def legal(self, acting: torch.Tensor | None = None, *, csr: bool = True, mask_words: bool = True,
               mask_bool: bool = False) -> dict[str, torch.Tensor]:
-        s = None if acting is None else acting.to(device=self.device, dtype=torch.int8).contiguous()
+        s = self._seats(acting)
         mb = torch.empty((self.n, L.ACTION_DIM), dtype=torch.bool, device=self.device) if mask_bool else None
         p = self._ptr
         check(lib.jq_legal(self._h, p(s), self.counts.data_ptr(),
@@ -236,7 +246,7 @@ class JunqiBatch:
     def legal_slots(self, acting: torch.Tensor | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
         """(N, 120, 80) bool per-piece slot mask of the acting seats (legal_action_mask_batch,
         game_state.cu:1964-2197)."""
-        s = None if acting is None else acting.to(device=self.device, dtype=torch.int8).contiguous()
+        s = self._seats(acting)
         shape = (self.n, L.NUM_PIDS, L.SLOTS_PER_PIECE)
         if out is None:
             out = torch.empty(shape, dtype=torch.bool, device=self.device)
@@ -244,6 +254,29 @@ class JunqiBatch:
             raise ValueError(f"slot mask output must be a contiguous bool tensor of shape {shape}")
         check(lib.jq_legal_slots(self._h, self._ptr(s), out.data_ptr(), self.stream))
         return out
+
+    def legal_dense_numpy(self, acting: np.ndarray | None, width: int) -> tuple[np.ndarray, np.ndarray]:
+        """(ids (N, width) int32, counts (N,) int32) on the host for host int8
+        seats (None: the current turn); ids ascending, cut at width, -1 padded."""
+        s = None if acting is None else torch.from_numpy(acting).contiguous()
+        ids = np.empty((self.n, width), np.int32)
+        counts = np.empty(self.n, np.int32)
+        check(lib.jq_legal_dense_host(self._h, self._ptr(s), self.counts.data_ptr(), self.offsets.data_ptr(),
+                                      self.values.data_ptr(), self.values.numel(), width, ids.ctypes.data,
+                                      counts.ctypes.data, self.stream))
+        return ids, counts
+
+    def step_numpy(self, action_ids: np.ndarray) -> dict[str, np.ndarray]:
+        """One ply per env from host world ids (N,); the reference's MoveResultBatch
+        arrays on the host."""
+        a = torch.from_numpy(action_ids.astype(np.int32, copy=False)).contiguous()
+        n = self.n
+        if a.shape != (n,):
+            raise ValueError(f"actions: expected ({n},), got {tuple(a.shape)}")
+        res = {k: np.empty(n, t) for k, t in (("valid", bool), ("event", np.int8), ("terminated", bool),
+                                              ("winner_team", np.int8), ("draw", bool), ("flag_captured", bool))}
+        check(lib.jq_step_host(self._h, a.data_ptr(), *(v.ctypes.data for v in res.values()), self.stream))
+        return res
 
     def legal_csr_numpy(self, acting: torch.Tensor | None = None) -> tuple[np.ndarray, np.ndarray]:
         self.legal(acting, csr=True, mask_words=False)
@@ -266,7 +299,10 @@ class JunqiBatch:
             out_aux = torch.empty(lead + (L.AUX_BYTES,), dtype=torch.uint8, device=self.device)
         if tuple(out_spatial.shape) != lead + (L.OBS_CHANNELS, 17, 17) or out_spatial.dtype != dt:
             raise ValueError("out_spatial has the wrong shape or dtype")
-        s = None if observer is None else observer.to(device=self.device, dtype=torch.int8).contiguous()
+        if all_seats:
+            s = None if observer is None else observer.to(device=self.device, dtype=torch.int8).contiguous()
+        else:
+            s = self._seats(observer)
         check(lib.jq_observe(self._h, self._ptr(s), code, 1 if all_seats else 0, out_spatial.data_ptr(),
                              self._ptr(out_aux) if fmt == "u8" else None, out_global.data_ptr(), self.stream))
         if fmt == "u8":
@@ -313,7 +349,7 @@ class JunqiBatch:
         acting seat's legal canonical ids of the current CSR rows."""
         if out is None:
             out = torch.empty(self.n, dtype=torch.int32, device=self.device)
-        s = None if acting is None else acting.to(device=self.device, dtype=torch.int8).contiguous()
+        s = self._seats(acting)
         check(lib.jq_sample_logits(self._h, self._ptr(s), self.counts.data_ptr(), self.offsets.data_ptr(),
                                    self.values.data_ptr(), self.values.numel(), int(seed), int(ply),
                                    out.data_ptr(), self._ptr(canonical_out), self.stream))
@@ -453,7 +489,9 @@ class JunqiBatch:
     # (junqi_rl/training/gpu_collector.py:375, 538, 602-650).
     def copy_turn_to_host(self) -> np.ndarray:
         """(N,) int8 acting seat per env (py_copy_turn_to_host, bindings.cpp:186-194)."""
-        return self.get_field("turn")[:, 0].astype(np.int8)
+        turn = np.empty(self.n, np.int8)
+        check(lib.jq_env_flags_host(self._h, turn.ctypes.data, None, None, None))
+        return turn
 
     def copy_to_host(self) -> dict[str, np.ndarray]:
         """The 21 flat arrays of py_copy_to_host (bindings.cpp:117-183), keys and
@@ -543,9 +581,10 @@ class JunqiBatch:
 
     def termination(self) -> dict[str, np.ndarray]:
         """terminated / winner_team / draw on the host (copy_termination_to_host)."""
-        return {"terminated": self.get_field("terminated")[:, 0].astype(bool),
-                "winner_team": self.get_field("winner")[:, 0].astype(np.int8),
-                "draw": self.get_field("draw")[:, 0].astype(bool)}
+        n = self.n
+        out = {"terminated": np.empty(n, bool), "winner_team": np.empty(n, np.int8), "draw": np.empty(n, bool)}
+        check(lib.jq_env_flags_host(self._h, None, *(v.ctypes.data for v in out.values())))
+        return out
 
     def field_tensor(self, name: str, torch_dtype: torch.dtype | None = None) -> torch.Tensor:
         """Zero-copy (strided) device view of a per-env state field, shape (N, elems) or (N,)."""

@@ -22,8 +22,19 @@
 
 using namespace jq;
 
+// Staging of the calls that take and fill host arrays: a pinned buffer (read and
+// written by kernels and copies) and a device buffer, grown to the largest call
+// and kept with the handle. Every such call holds the lock until its stream has
+// run, so neither buffer is in use when the next one takes it.
+struct HostIo {
+    std::mutex mu;
+    uint8_t *pinned = nullptr, *dev = nullptr;
+    size_t pinned_cap = 0, dev_cap = 0;
+};
+
 struct jq_env {
     int device = 0;
+    HostIo io;
     State S{};
     std::vector<void *> allocs;
     bool zob_ready = false, rlut_ready = false;
@@ -294,6 +305,45 @@ int csr_fits(jq_env *e, const int32_t *offsets, int64_t cap, hipStream_t s)
     return JQ_OK;
 }
 
+// Room for a host call (io.mu held).
+int host_io_room(HostIo &io, size_t pinned, size_t dev)
+{
+    if (pinned > io.pinned_cap) {
+        if (io.pinned) (void)hipHostFree(io.pinned);
+        io.pinned = nullptr;
+        io.pinned_cap = 0;
+        void *q = nullptr;
+        if (hipHostMalloc(&q, pinned) != hipSuccess) return fail(JQ_E_OOM, "hipHostMalloc(%zu) failed", pinned);
+        io.pinned = static_cast<uint8_t *>(q);
+        io.pinned_cap = pinned;
+    }
+    if (dev > io.dev_cap) {
+        if (io.dev) (void)hipFree(io.dev);
+        io.dev = nullptr;
+        io.dev_cap = 0;
+        void *q = nullptr;
+        if (hipMalloc(&q, dev) != hipSuccess) return fail(JQ_E_OOM, "hipMalloc(%zu) failed", dev);
+        io.dev = static_cast<uint8_t *>(q);
+        io.dev_cap = dev;
+    }
+    return JQ_OK;
+}
+
+// `bytes` of caller input as kernels on `s` can read them: the pinned copy
+// itself while it is small (a kernel's few reads of it cost less than a copy's
+// launch), else a device copy at `dev`.
+constexpr size_t HOST_READ_MAX = 16384;
+int host_input(HostIo &io, const void *host, size_t bytes, size_t pin_off, size_t dev_off, hipStream_t s,
+               const uint8_t *&out)
+{
+    std::memcpy(io.pinned + pin_off, host, bytes);
+    out = io.pinned + pin_off;
+    if (bytes <= HOST_READ_MAX) return JQ_OK;
+    HIP_TRY(hipMemcpyAsync(io.dev + dev_off, io.pinned + pin_off, bytes, hipMemcpyHostToDevice, s));
+    out = io.dev + dev_off;
+    return JQ_OK;
+}
+
 int check_env(jq_env *e)
 {
     if (!e) return fail(JQ_E_ARG, "null handle");
@@ -446,6 +496,8 @@ int jq_destroy(jq_env *e)
     for (void *p : e->allocs) (void)hipFree(p);
     if (e->pool) (void)hipFree(e->pool);
     if (e->total_host) (void)hipHostFree(e->total_host);
+    if (e->io.pinned) (void)hipHostFree(e->io.pinned);
+    if (e->io.dev) (void)hipFree(e->io.dev);
     if (e->side) (void)hipStreamDestroy(e->side);
     if (e->ev_step) (void)hipEventDestroy(e->ev_step);
     if (e->ev_csr) (void)hipEventDestroy(e->ev_csr);
@@ -619,6 +671,103 @@ int jq_legal(jq_env *e, const int8_t *acting, int32_t *counts, int32_t *offsets,
         hipLaunchKernelGGL(k_emit, dim3((e->S.n + 1) / 2), dim3(64), 0, strm(stream), e->S, offsets, values,
                            values_capacity, nullptr);
         if ((rc = launch_check("k_emit")) != 0) return rc;
+    }
+    return JQ_OK;
+}
+
+int jq_step_host(jq_env *e, const int32_t *actions, uint8_t *valid, int8_t *event, uint8_t *terminated, int8_t *winner,
+                 uint8_t *draw, uint8_t *flag_captured, void *stream)
+{
+    int rc = check_env(e);
+    if (rc) return rc;
+    if (!actions) return fail(JQ_E_ARG, "null actions");
+    if (!e->zob_ready) return fail(JQ_E_STATE, "upload the Zobrist tables before stepping");
+    const size_t n = (size_t)e->S.n;
+    const hipStream_t s = strm(stream);
+    std::lock_guard<std::mutex> lk(e->io.mu);
+    HostIo &io = e->io;
+    if ((rc = host_io_room(io, 10 * n, 10 * n)) != 0) return rc;   // 4 bytes of action, 6 of reports per game
+    const uint8_t *a = nullptr;
+    if ((rc = host_input(io, actions, 4 * n, 0, 0, s, a)) != 0) return rc;
+    uint8_t *d = io.dev + 4 * n, *h = io.pinned + 4 * n;
+    StepOut O{};
+    O.valid = d; O.event = reinterpret_cast<int8_t *>(d + n); O.term = d + 2 * n;
+    O.winner = reinterpret_cast<int8_t *>(d + 3 * n); O.draw = d + 4 * n; O.fcap = d + 5 * n;
+    hipLaunchKernelGGL(k_step, dim3(e->S.n), dim3(64), 0, s, e->S, reinterpret_cast<const int32_t *>(a), nullptr,
+                       JQ_ACT_WORLD, O);
+    rc = launch_check("k_step");
+    if (!rc && hipMemcpyAsync(h, d, 6 * n, hipMemcpyDeviceToHost, s) != hipSuccess)
+        rc = fail(JQ_E_HIP, "copying the step's reports failed");
+    HIP_TRY(hipStreamSynchronize(s));
+    if (rc) return rc;
+    void *const out[6] = {valid, event, terminated, winner, draw, flag_captured};
+    for (int k = 0; k < 6; ++k)
+        if (out[k]) std::memcpy(out[k], h + k * n, n);
+    return JQ_OK;
+}
+
+int jq_legal_dense_host(jq_env *e, const int8_t *acting, int32_t *counts, int32_t *offsets, int32_t *values,
+                        int64_t values_capacity, int32_t width, int32_t *ids, int32_t *counts_out, void *stream)
+{
+    int rc = check_env(e);
+    if (rc) return rc;
+    if (!counts || !offsets || !values) return fail(JQ_E_ARG, "legal_dense_host needs counts, offsets and values");
+    if (!ids || !counts_out || width <= 0) return fail(JQ_E_ARG, "legal_dense_host needs host rows");
+    if (values_capacity < 0) return fail(JQ_E_ARG, "negative values capacity");
+    const size_t n = (size_t)e->S.n;
+    const hipStream_t s = strm(stream);
+    std::lock_guard<std::mutex> lk(e->io.mu);
+    HostIo &io = e->io;
+    // acting | counts | ids: the ids of an average position and half again come
+    // with the first copy, the rest (if any) with a second one
+    const size_t c_off = (n + 15) & ~(size_t)15, v_off = c_off + 4 * n;
+    const size_t guess = std::min((size_t)values_capacity, 64 * n);
+    if ((rc = host_io_room(io, v_off + 4 * guess, n)) != 0) return rc;
+    const uint8_t *a = nullptr;
+    if (acting && (rc = host_input(io, acting, n, 0, 0, s, a)) != 0) return rc;
+    rc = jq_legal(e, reinterpret_cast<const int8_t *>(a), counts, offsets, values, values_capacity, nullptr, nullptr,
+                  stream);
+    if (!rc && hipMemcpyAsync(io.pinned + c_off, counts, 4 * n, hipMemcpyDeviceToHost, s) != hipSuccess)
+        rc = fail(JQ_E_HIP, "copying the counts failed");
+    if (!rc && guess &&
+        hipMemcpyAsync(io.pinned + v_off, values, 4 * guess, hipMemcpyDeviceToHost, s) != hipSuccess)
+        rc = fail(JQ_E_HIP, "copying the ids failed");
+    HIP_TRY(hipStreamSynchronize(s));
+    if (rc) return rc;
+    std::memcpy(counts_out, io.pinned + c_off, 4 * n);
+    size_t total = 0;
+    for (size_t i = 0; i < n; ++i) total += (size_t)counts_out[i];
+    if (total > guess) {
+        if ((rc = host_io_room(io, v_off + 4 * total, n)) != 0) return rc;
+        HIP_TRY(hipMemcpyAsync(io.pinned + v_off, values, 4 * total, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+    }
+    const int32_t *v = reinterpret_cast<const int32_t *>(io.pinned + v_off);
+    for (size_t i = 0; i < n; ++i) {
+        int32_t *row = ids + i * (size_t)width;
+        const int32_t take = std::min(counts_out[i], width);
+        std::memcpy(row, v, 4 * (size_t)take);
+        std::memset(row + take, 0xFF, 4 * (size_t)(width - take));
+        v += counts_out[i];
+    }
+    return JQ_OK;
+}
+
+int jq_env_flags_host(jq_env *e, int8_t *turn, uint8_t *terminated, int8_t *winner, uint8_t *draw)
+{
+    int rc = check_env(e);
+    if (rc) return rc;
+    const size_t n = (size_t)e->S.n;
+    std::lock_guard<std::mutex> lk(e->io.mu);
+    if ((rc = host_io_room(e->io, n * sizeof(EnvRec), 0)) != 0) return rc;
+    HIP_TRY(hipDeviceSynchronize());   // of any stream, as jq_get_field
+    HIP_TRY(hipMemcpy(e->io.pinned, e->S.env, n * sizeof(EnvRec), hipMemcpyDeviceToHost));
+    const EnvRec *r = reinterpret_cast<const EnvRec *>(e->io.pinned);
+    for (size_t i = 0; i < n; ++i) {
+        if (turn) turn[i] = r[i].turn;
+        if (terminated) terminated[i] = r[i].term;
+        if (winner) winner[i] = r[i].winner;
+        if (draw) draw[i] = r[i].draw;
     }
     return JQ_OK;
 }

@@ -150,11 +150,8 @@ class GpuRollout:
         action_ids = np.asarray(action_ids)
         if action_ids.shape != (self.num_envs,):
             raise ValueError(f"action_ids shape mismatch: expected ({self.num_envs},), got {action_ids.shape}")
-        out = self._b.step(torch.from_numpy(action_ids.astype(np.int32, copy=False)).to(self.device))
-        res = {k: out[k].cpu().numpy() for k in ("valid", "event", "terminated", "winner_team", "draw",
-                                                  "flag_captured")}
-        self._last_result = res
-        return res
+        self._last_result = self._b.step_numpy(action_ids)
+        return self._last_result
 
     def step_device_torch(self, canonical_actions: torch.Tensor, acting_seats: torch.Tensor) -> dict:
         """Compact canonical ids (src_c*129 + dst_c in the acting seat's frame) →
@@ -162,10 +159,10 @@ class GpuRollout:
         (gpu_rollout.py:780-848). Move history and beliefs are updated here."""
         b, o = self._b, self._step_out
         a = canonical_actions.to(device=self.device, dtype=torch.int32).contiguous()
-        s = acting_seats.to(device=self.device, dtype=torch.int8).contiguous()
-        if a.shape != (self.num_envs,) or s.shape != (self.num_envs,):
+        s = b._seats(acting_seats)
+        if a.shape != (self.num_envs,) or (s is not None and s.shape != (self.num_envs,)):
             raise ValueError(f"expected ({self.num_envs},) actions and acting seats")
-        L.check(L.lib.jq_step(b._h, a.data_ptr(), s.data_ptr(), L.ACT_CANONICAL, None, o["event"].data_ptr(),
+        L.check(L.lib.jq_step(b._h, a.data_ptr(), b._ptr(s), L.ACT_CANONICAL, None, o["event"].data_ptr(),
                               o["terminated"].data_ptr(), o["winner_team"].data_ptr(), o["draw"].data_ptr(),
                               None, None, o["rewards"].data_ptr(), None, b.stream))
         return dict(o)
@@ -190,9 +187,7 @@ class GpuRollout:
     def legal_actions_dense(self, acting_seats: np.ndarray) -> tuple[np.ndarray, np.ndarray]:
         """(action_ids (N,512) int32, counts (N,) int32); ids ascending in each
         row, unused slots -1 (gpu_rollout.py:854-860)."""
-        s = torch.from_numpy(self._seats_np(acting_seats)).to(self.device)
-        ids, counts = _dense_from_csr(self._b, s)
-        return ids.cpu().numpy(), counts.cpu().numpy()
+        return self._b.legal_dense_numpy(self._seats_np(acting_seats), MAX_ACTIONS_PER_ENV)
 
     def legal_actions_mask(self, acting_seats: np.ndarray) -> np.ndarray:
         """(N, 120, 80) bool per-piece slot mask (gpu_rollout.py:862-869): slot
@@ -214,8 +209,8 @@ class GpuRollout:
         b = self._b
         if self._mask_bool is None:
             self._mask_bool = torch.empty((self.num_envs, FLAT_ACTION_DIM), dtype=torch.bool, device=self.device)
-        s = None if seats is None else seats.to(device=self.device, dtype=torch.int8).contiguous()
-        L.check(L.lib.jq_legal(b._h, None if s is None else s.data_ptr(), b.counts.data_ptr(), None, None, 0, None,
+        s = b._seats(seats)
+        L.check(L.lib.jq_legal(b._h, b._ptr(s), b.counts.data_ptr(), None, None, 0, None,
                                self._mask_bool.data_ptr(), b.stream))
         return self._mask_bool
 
@@ -226,8 +221,7 @@ class GpuRollout:
         if self._sp1 is None:
             self._sp1 = torch.empty((self.num_envs, OBS_CHANNELS, 17, 17), dtype=torch.float32, device=self.device)
             self._gl1 = torch.empty((self.num_envs, L.OBS_GLOBALS), dtype=torch.float32, device=self.device)
-        s = acting_seats_t.to(device=self.device, dtype=torch.int8).contiguous()
-        return self._b.observe(s, fmt="f32", out_spatial=self._sp1, out_global=self._gl1)
+        return self._b.observe(acting_seats_t, fmt="f32", out_spatial=self._sp1, out_global=self._gl1)
 
     def build_all_seat_observations_torch(self):
         """(N,4,317,17,17) and (N,4,28) f32 device views; slot k observes the seat
@@ -277,7 +271,7 @@ class GpuRollout:
 
     def turn_torch(self) -> torch.Tensor:
         """Zero-copy int8 (N,) view of the acting seats (gpu_rollout.py:1159-1169)."""
-        return self._b.field_tensor("turn")
+        return self._b._turn_view.detach()
 
     def terminated_torch(self) -> torch.Tensor:
         return self._b.field_tensor("terminated", torch.bool)
@@ -307,16 +301,3 @@ class GpuRollout:
         """The underlying JunqiBatch (all library entry points)."""
         return self._b
 
-
-def _dense_from_csr(b: JunqiBatch, seats: torch.Tensor | None) -> tuple[torch.Tensor, torch.Tensor]:
-    """(N,512) int32 ids (ascending, -1 padded) and (N,) counts from the CSR rows."""
-    b.legal(seats, csr=True, mask_words=False)
-    counts = b.counts.clone()
-    n = b.n
-    total = int(b.offsets[-1].item())
-    idx = torch.arange(MAX_ACTIONS_PER_ENV, device=b.device).unsqueeze(0)
-    take = idx < counts.clamp(max=MAX_ACTIONS_PER_ENV).unsqueeze(1)
-    dense = torch.full((n, MAX_ACTIONS_PER_ENV), -1, dtype=torch.int32, device=b.device)
-    src = b.offsets[:-1].unsqueeze(1) + idx
-    dense[take] = b.values[: max(total, 1)].gather(0, src[take].long().clamp(max=max(total - 1, 0)))
-    return dense, counts

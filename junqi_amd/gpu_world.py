@@ -13,7 +13,7 @@ import torch
 
 from . import _lib as L
 from .batch import JunqiBatch
-from .gpu_rollout import _dense_from_csr, _show_value
+from .gpu_rollout import MAX_ACTIONS_PER_ENV, _show_value
 
 
 def _pack_state_arrays(envs) -> tuple[dict, dict]:
@@ -83,8 +83,7 @@ class GpuWorld:
     def legal_actions_dense(self, acting_seats: np.ndarray) -> tuple[np.ndarray, np.ndarray]:
         """(N,512) int32 ids (ascending, -1 padded) and (N,) counts (gpu_world.py:178-188)."""
         self._validate_acting_seats(acting_seats)
-        ids, counts = _dense_from_csr(self.state, torch.from_numpy(acting_seats).to(self.device))
-        return ids.cpu().numpy(), counts.cpu().numpy()
+        return self.state.legal_dense_numpy(acting_seats, MAX_ACTIONS_PER_ENV)
 
     def legal_actions_csr(self, acting_seats: np.ndarray) -> tuple[np.ndarray, np.ndarray]:
         """(offsets (N+1,) int32, values int32): env i's ascending ids at
@@ -106,9 +105,7 @@ class GpuWorld:
         action_ids = np.asarray(action_ids)
         if action_ids.shape != (self.num_envs,):
             raise ValueError(f"action_ids: expected shape ({self.num_envs},), got {action_ids.shape}")
-        out = self.state.step(torch.from_numpy(action_ids.astype(np.int32, copy=False)).to(self.device))
-        return {k: out[k].cpu().numpy() for k in ("valid", "event", "terminated", "winner_team", "draw",
-                                                  "flag_captured")}
+        return self.state.step_numpy(action_ids)
 
     def push_termination_state(self, terminated: np.ndarray, winner_team: np.ndarray, draw: np.ndarray) -> None:
         """Overwrite terminated / winner_team / draw (gpu_world.py:255-265)."""
