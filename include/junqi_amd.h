@@ -372,6 +372,12 @@ int jq_history_reconstruct(jq_history *hist, const int64_t *flat, const int8_t *
                            void *spatial, void *aux, float *global, int32_t *mask_words, uint8_t *mask_bool,
                            void *stream);
 
+/* jq_history_reconstruct in JQ_OBS_BF16 with the globals in bfloat16 too (global:
+ * device bfloat16 (batch, 28), 4-byte aligned): a whole minibatch in the
+ * learner's dtype (junqi_rl/gpu_rollout.py:164-217, dtype=bfloat16). */
+int jq_history_reconstruct_bf16(jq_history *hist, const int64_t *flat, const int8_t *observer, int32_t batch,
+                                void *spatial, void *global, int32_t *mask_words, uint8_t *mask_bool, void *stream);
+
 /* The same rebuild for callers that cannot allocate (code under HIP graph
  * capture, serving loops, harnesses that forbid hipMalloc), at most
  * JQ_NOALLOC_MAX_ROWS rows a call. No counterpart in the reference. Neither

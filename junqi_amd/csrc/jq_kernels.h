@@ -1211,45 +1211,58 @@ __device__ __forceinline__ void legal_body(const State &S, int env, int row, int
     }
 }
 
-// HIST: block r takes row flat[r] of a rollout history (S = history_state) for
-// seat acting[r], and writes its masks as row r of the minibatch; flat values
-// outside [0, S.n) have no legal action. No counts or legal records then.
-template <bool HIST = false>
-__global__ __launch_bounds__(64) void k_legal(State S, const int8_t *__restrict__ acting,
-                                              int32_t *__restrict__ counts, int32_t *__restrict__ mask_words,
-                                              uint8_t *__restrict__ mask_bool,
-                                              const int64_t *__restrict__ flat = nullptr)
+// One wave's LDS for the legal sets of a row.
+struct LegalLds {
+    uint64_t lscr[LSCR_WORDS];
+    uint32_t bits[JQ_MASK_WORDS_PAD];
+    int8_t cell[CELL_STRIDE];
+    uint8_t rotl[NONB + 3];   // world compact -> canonical compact of the acting seat
+};
+
+// Legal sets of row `row` by one wave (lane l). HIST: history row flat[row]
+// (S = history_state) for seat acting[row], its masks as row `row` of the
+// minibatch; flat values outside [0, S.n) have no legal action. No counts or
+// legal records then.
+template <bool HIST>
+__device__ __forceinline__ void legal_row(const State &S, int row, int l, LegalLds &L, const int8_t *__restrict__ acting,
+                                          int32_t *__restrict__ counts, int32_t *__restrict__ mask_words,
+                                          uint8_t *__restrict__ mask_bool, const int64_t *__restrict__ flat)
 {
-    const int row = blockIdx.x, l = threadIdx.x;
     int env = row;
     bool stored = true;
     if constexpr (HIST) {
         const int64_t f = flat[row];
         stored = f >= 0 && f < (int64_t)S.n;
         env = stored ? (int)f : 0;
-    } else if (env >= S.n) {
-        return;
     }
-    __shared__ int8_t cell[CELL_STRIDE];
-    __shared__ uint32_t bits[JQ_MASK_WORDS_PAD];
-    __shared__ uint8_t rotl[NONB + 3];   // world compact -> canonical compact of the acting seat
-    __shared__ uint64_t lscr[LSCR_WORDS];
     const EnvRec &E = S.env[env];
     const int seat = acting ? acting[row] : E.turn;
     const bool off = !stored || E.term || seat < 0 || seat > 3 || ((E.sdead >> (seat & 3)) & 1);
-    for (int f = l; f < CELL_STRIDE; f += 64) cell[f] = f < NC ? S.cell[(size_t)env * CELL_STRIDE + f] : -1;
+    for (int f = l; f < CELL_STRIDE; f += 64) L.cell[f] = f < NC ? S.cell[(size_t)env * CELL_STRIDE + f] : -1;
     // wave issue priority 2 through the legal pass, 0 for the bool rows'
     // stores (legal_body lowers it): a wave still computing gets issue slots
     // ahead of the waves that are storing rows (drop-in step at 32,768 games:
     // 2.486 -> 2.474 ms)
     __builtin_amdgcn_s_setprio(2);
-    for (int w = l; w < JQ_MASK_WORDS_PAD; w += 64) bits[w] = 0;
+    for (int w = l; w < JQ_MASK_WORDS_PAD; w += 64) L.bits[w] = 0;
     if (mask_words || mask_bool) {
         const int s4 = seat & 3;
-        for (int c = l; c < NONB; c += 64) rotl[c] = cT.rotc[s4][c];
+        for (int c = l; c < NONB; c += 64) L.rotl[c] = cT.rotc[s4][c];
     }
-    __syncthreads();
-    legal_body<!HIST>(S, env, row, l, seat, off, cell, bits, rotl, nullptr, nullptr, lscr, counts, mask_words, mask_bool);
+    wave_sync();
+    legal_body<!HIST>(S, env, row, l, seat, off, L.cell, L.bits, L.rotl, nullptr, nullptr, L.lscr, counts, mask_words,
+                      mask_bool);
+}
+
+template <bool HIST = false>
+__global__ __launch_bounds__(64) void k_legal(State S, const int8_t *__restrict__ acting,
+                                              int32_t *__restrict__ counts, int32_t *__restrict__ mask_words,
+                                              uint8_t *__restrict__ mask_bool,
+                                              const int64_t *__restrict__ flat = nullptr)
+{
+    __shared__ LegalLds L;
+    if (!HIST && (int)blockIdx.x >= S.n) return;
+    legal_row<HIST>(S, blockIdx.x, threadIdx.x, L, acting, counts, mask_words, mask_bool, flat);
 }
 
 // Exclusive scan of counts into offsets (N+1); one 1024-thread block walks the
@@ -1453,6 +1466,14 @@ struct CsrArgs {
     int64_t cap;
     int passes;   // envs per wave
     int blocks;   // of a launch: 0 = no CSR pass in it
+};
+
+// The legal masks of a minibatch of history rows, as blocks of the launch that
+// observes them (either output may be null).
+struct MaskArgs {
+    int32_t *words;
+    uint8_t *bytes;
+    int blocks;   // 0 = no masks in the launch
 };
 
 struct CsrLds {

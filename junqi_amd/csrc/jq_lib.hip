@@ -808,7 +808,7 @@ static int observe(jq_env *e, const int8_t *observer, int32_t fmt, int32_t all_s
                                             : (e->ext_on ? &k_observe<0, true> : &k_observe<0>);
         hipLaunchKernelGGL(kernel, dim3((unsigned)nrows * p.parts + csr.blocks), dim3(ROW_THREADS), 0, strm(stream), e->S,
                            observer, all_seats, spatial, aux, global, nrows, p.parts, p.stream,
-                           static_cast<const float *>(e->ext_bel), nullptr, csr);
+                           static_cast<const float *>(e->ext_bel), nullptr, csr, MaskArgs{}, 0);
     }
     rc = launch_check("k_observe");
     // the end event follows its begin event even when the launch failed, so no
@@ -1161,28 +1161,33 @@ int jq_history_snapshot(jq_history *h, jq_env *e, const int8_t *acting, int32_t 
 // Observations and masks of `batch` history rows, straight from the history's
 // arrays: no scratch state, no allocation.
 static int history_rebuild(jq_history *h, const int64_t *flat, const int8_t *observer, int32_t batch, int32_t fmt,
-                           void *spatial, void *aux, float *global, int32_t *mask_words, uint8_t *mask_bool,
-                           void *stream)
+                           void *spatial, void *aux, void *global, int32_t global_fmt, int32_t *mask_words,
+                           uint8_t *mask_bool, void *stream)
 {
     if (!flat || !observer) return fail(JQ_E_ARG, "history reconstruction received a null device pointer");
     if (!h->rlut_ready) return fail(JQ_E_STATE, "history has no snapshot yet");
     HIP_TRY(hipSetDevice(h->device));
     int rc;
     const State S = history_state(h->H, h->rlut, h->show_mode);
+    const bool masks = mask_words || mask_bool;
     if (spatial || aux || global) {
         if (!spatial || !global) return fail(JQ_E_ARG, "spatial and global outputs go together");
-        if ((rc = obs_args(true, false, fmt, spatial, aux, global)) != 0) return rc;
+        if ((rc = obs_args(true, false, fmt, spatial, aux, static_cast<const float *>(global))) != 0) return rc;
         const ObsPlan p = obs_plan(fmt, batch, g_dev[h->device].cus);
+        // the masks ride in the observation's launch, one row per wave of its last blocks
+        constexpr int NW = ROW_THREADS / 64;
+        const MaskArgs M{mask_words, mask_bool, masks ? (batch + NW - 1) / NW : 0};
         auto *kernel = fmt == JQ_OBS_F32 ? &k_observe<0, false, true>
                                          : fmt == JQ_OBS_BF16 ? &k_observe<1, false, true> : &k_observe<2, false, true>;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)batch * p.parts), dim3(ROW_THREADS), 0, strm(stream), S, observer, 0,
-                           spatial, aux, global, batch, p.parts, p.stream, nullptr, flat, CsrArgs{});
-        if ((rc = launch_check("k_observe")) != 0) return rc;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)batch * p.parts + M.blocks), dim3(ROW_THREADS), 0, strm(stream), S,
+                           observer, 0, spatial, aux, static_cast<float *>(global), batch, p.parts, p.stream, nullptr,
+                           flat, CsrArgs{}, M, global_fmt == JQ_OBS_BF16 ? 1 : 0);
+        return launch_check("k_observe");
     }
-    if (mask_words || mask_bool) {
+    if (masks) {
         hipLaunchKernelGGL(k_legal<true>, dim3(batch), dim3(64), 0, strm(stream), S, observer, nullptr, mask_words,
                            mask_bool, flat);
-        if ((rc = launch_check("k_legal")) != 0) return rc;
+        return launch_check("k_legal");
     }
     return JQ_OK;
 }
@@ -1193,7 +1198,17 @@ int jq_history_reconstruct(jq_history *h, const int64_t *flat, const int8_t *obs
 {
     if (!h) return fail(JQ_E_ARG, "null history");
     if (batch <= 0) return fail(JQ_E_ARG, "cannot reconstruct an empty history minibatch");
-    return history_rebuild(h, flat, observer, batch, fmt, spatial, aux, global, mask_words, mask_bool, stream);
+    return history_rebuild(h, flat, observer, batch, fmt, spatial, aux, global, JQ_OBS_F32, mask_words, mask_bool,
+                           stream);
+}
+
+int jq_history_reconstruct_bf16(jq_history *h, const int64_t *flat, const int8_t *observer, int32_t batch,
+                                void *spatial, void *global, int32_t *mask_words, uint8_t *mask_bool, void *stream)
+{
+    if (!h) return fail(JQ_E_ARG, "null history");
+    if (batch <= 0) return fail(JQ_E_ARG, "cannot reconstruct an empty history minibatch");
+    return history_rebuild(h, flat, observer, batch, JQ_OBS_BF16, spatial, nullptr, global, JQ_OBS_BF16, mask_words,
+                           mask_bool, stream);
 }
 
 int jq_history_reconstruct_noalloc(jq_history *h, const int64_t *flat, const int8_t *observer, int32_t batch,
@@ -1205,7 +1220,8 @@ int jq_history_reconstruct_noalloc(jq_history *h, const int64_t *flat, const int
     if (batch > JQ_NOALLOC_MAX_ROWS)
         return fail(JQ_E_ARG, "batch %d exceeds the %d rows jq_history_reconstruct_noalloc holds", batch,
                     JQ_NOALLOC_MAX_ROWS);
-    return history_rebuild(h, flat, observer, batch, fmt, spatial, aux, global, mask_words, mask_bool, stream);
+    return history_rebuild(h, flat, observer, batch, fmt, spatial, aux, global, JQ_OBS_F32, mask_words, mask_bool,
+                           stream);
 }
 
 // ---------------------------------------------------------------- masks

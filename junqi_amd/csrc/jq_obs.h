@@ -462,7 +462,8 @@ __device__ __forceinline__ int row_obs_prefetch(const State &S, const int8_t *ob
 // AUXC (the u8 format): recency as aux codes, no table lookups.
 template <bool EXT = false, bool AUXC = false>
 __device__ __forceinline__ void row_fill(const State &S, int obs, int m, int t, const RowIn &R, ObsLds &L,
-                                         float *glob_row, const float *ext = nullptr, ExtLds *X = nullptr)
+                                         float *glob_row, const float *ext = nullptr, ExtLds *X = nullptr,
+                                         uint16_t *glob16_row = nullptr)
 {
     // env-record fields and the observer's piece types, from the fetched lanes
     const int mc = __builtin_amdgcn_readlane((int)R.ew, 2), mslc = __builtin_amdgcn_readlane((int)R.ew, 3);
@@ -518,7 +519,7 @@ __device__ __forceinline__ void row_fill(const State &S, int obs, int m, int t, 
         double mp = (double)mc / 4000.0; if (mp > 1.0) mp = 1.0;
         L.turnv[0] = (float)dp; L.turnv[1] = (float)mp;
     }
-    if (glob_row && t < 28) {   // globals (observation.py:1623-1651)
+    if ((glob_row || glob16_row) && t < 28) {   // globals (observation.py:1623-1651)
         float v;
         if (t < 24) {   // remaining counts of the left / right enemy
             const int seat = t < 12 ? (obs + 1) & 3 : (obs + 3) & 3;
@@ -526,7 +527,8 @@ __device__ __forceinline__ void row_fill(const State &S, int obs, int m, int t, 
         } else {   // flag_revealed of self, teammate, left, right
             v = (float)((sflag >> seat_rel(obs, t - 24)) & 1);
         }
-        glob_row[t] = v;
+        if (glob16_row) glob16_row[t] = f32_to_bf16_rne(v);
+        else glob_row[t] = v;
     }
 }
 
@@ -850,7 +852,8 @@ __global__ __launch_bounds__(ROW_THREADS) __attribute__((amdgpu_waves_per_eu(FMT
                                                          void *__restrict__ spatial, void *__restrict__ aux,
                                                          float *__restrict__ glob, int nrows, int parts, int stream,
                                                          const float *__restrict__ ext,
-                                                         const int64_t *__restrict__ flat, CsrArgs csr)
+                                                         const int64_t *__restrict__ flat, CsrArgs csr,
+                                                         MaskArgs masks, int glob_bf16)
 {
     __shared__ ObsLds L;
     if constexpr (!EXT && !HIST) {   // an env-step's CSR pass: the grid's last blocks
@@ -858,6 +861,18 @@ __global__ __launch_bounds__(ROW_THREADS) __attribute__((amdgpu_waves_per_eu(FMT
         const int cb = (int)blockIdx.x - nrows * parts;
         if (cb >= 0) {
             csr_block(S, csr, cb, reinterpret_cast<CsrLds &>(L));
+            return;
+        }
+    }
+    if constexpr (HIST) {   // the minibatch's legal masks, one row per wave: the grid's last blocks
+        constexpr int NW = ROW_THREADS / 64;
+        static_assert(sizeof(LegalLds) * NW <= sizeof(ObsLds), "shares the block's LDS");
+        const int mb = (int)blockIdx.x - nrows * parts;
+        if (mb >= 0) {
+            const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), r = mb * NW + w;
+            if (r < nrows)
+                legal_row<true>(S, r, threadIdx.x & 63, reinterpret_cast<LegalLds *>(&L)[w], observer, nullptr,
+                                masks.words, masks.bytes, flat);
             return;
         }
     }
@@ -890,8 +905,11 @@ __global__ __launch_bounds__(ROW_THREADS) __attribute__((amdgpu_waves_per_eu(FMT
     obs_clear(L, cOBS.stat, t, ROW_THREADS);
     if (EXT && t < PID_STRIDE) X->rel[t] = 0;
     lds_barrier();
-    row_fill<EXT, FMT == 2>(S, obs, m, t, R, L, glob && part == 0 ? glob + (size_t)row * 28 : nullptr,
-                            EXT ? ext + ((size_t)env * 4 + obs) * 12 * NC : nullptr, X);
+    const bool globals = glob && part == 0;
+    const bool g16 = HIST && FMT == 1 && glob_bf16;   // a bf16 minibatch takes its globals in bf16
+    row_fill<EXT, FMT == 2>(S, obs, m, t, R, L, globals && !g16 ? glob + (size_t)row * 28 : nullptr,
+                            EXT ? ext + ((size_t)env * 4 + obs) * 12 * NC : nullptr, X,
+                            globals && g16 ? reinterpret_cast<uint16_t *>(glob) + (size_t)row * 28 : nullptr);
     __builtin_amdgcn_s_setprio(0);
     lds_barrier();
     if (FMT == 2)

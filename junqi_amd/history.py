@@ -86,16 +86,19 @@ class GpuRolloutHistory:
         if b <= 0:
             raise ValueError("cannot reconstruct an empty history minibatch")
         dev = flat_indices.device
-        fmt, sdt = (L.OBS_BF16, torch.bfloat16) if dtype == torch.bfloat16 else (L.OBS_F32, torch.float32)
-        spatial = torch.empty((b, OBS_CHANNELS, 17, 17), dtype=sdt, device=dev)
-        glob = torch.empty((b, OBS_GLOBAL_DIMS), dtype=torch.float32, device=dev)
+        bf16 = dtype == torch.bfloat16
+        fdt = torch.bfloat16 if bf16 else torch.float32
+        spatial = torch.empty((b, OBS_CHANNELS, 17, 17), dtype=fdt, device=dev)
+        glob = torch.empty((b, OBS_GLOBAL_DIMS), dtype=fdt, device=dev)
         mask = torch.empty((b, FLAT_ACTION_DIM), dtype=torch.bool, device=dev)
         stream = torch.cuda.current_stream(dev).cuda_stream
-        check(lib.jq_history_reconstruct(self._h, flat_indices.data_ptr(), acting_seats.data_ptr(), b, fmt,
+        if bf16:
+            check(lib.jq_history_reconstruct_bf16(self._h, flat_indices.data_ptr(), acting_seats.data_ptr(), b,
+                                                  spatial.data_ptr(), glob.data_ptr(), None, mask.data_ptr(), stream))
+            return spatial, glob, mask
+        check(lib.jq_history_reconstruct(self._h, flat_indices.data_ptr(), acting_seats.data_ptr(), b, L.OBS_F32,
                                          spatial.data_ptr(), None, glob.data_ptr(), None, mask.data_ptr(), stream))
-        if spatial.dtype != dtype:
-            spatial = spatial.to(dtype)
-        return spatial, glob.to(dtype), mask
+        return spatial.to(dtype), glob.to(dtype), mask
 
     def close(self) -> None:
         if getattr(self, "_h", None) is not None and self._h.value:
