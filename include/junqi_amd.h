@@ -130,6 +130,8 @@ int jq_generate_styled(int32_t mode, int64_t seed, int32_t count, int32_t per_ga
 /* Copy of the host-built constant board tables (struct jq::Tables of
  * junqi_amd/csrc/jq_topology.h), for inspection by tests. */
 int jq_board_tables(void *host_out, int64_t nbytes);
+/* the move generator's records derived from them (struct MoveTables, same file) */
+int jq_move_tables(void *host_out, int64_t nbytes);
 
 /* Reset terminated envs from the pool, picking entry hash(env, seed) % pool_size
  * (src/env/cuda/src/game_state.cu:2936-3102). Replaces reset_terminated_envs

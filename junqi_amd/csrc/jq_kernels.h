@@ -21,6 +21,7 @@
 namespace jq {
 
 __constant__ Tables cT;
+__constant__ MoveTables cM;
 constexpr int JQ_MASK_WORDS_PAD = 528;
 constexpr int LSCR_WORDS = 12;   // legal_body's per-wave LDS scratch (u64 words)
 
@@ -175,93 +176,60 @@ __device__ __forceinline__ bool bb_has(const BB &b, int c)
     const uint64_t w = c < 64 ? b.w0 : c < 128 ? b.w1 : b.w2;
     return (w >> (c & 63)) & 1ull;
 }
-__device__ __forceinline__ BB bb_and(const BB &a, const BB &b) { return {a.w0 & b.w0, a.w1 & b.w1, a.w2 & b.w2}; }
-__device__ __forceinline__ BB bb_or(const BB &a, const BB &b) { return {a.w0 | b.w0, a.w1 | b.w1, a.w2 | b.w2}; }
-__device__ __forceinline__ bool bb_any(const BB &b) { return (b.w0 | b.w1 | b.w2) != 0; }
-__device__ __forceinline__ int bb_lowest(const BB &b)
-{
-    return b.w0 ? __builtin_ctzll(b.w0) : b.w1 ? 64 + __builtin_ctzll(b.w1) : 128 + __builtin_ctzll(b.w2);
-}
-__device__ __forceinline__ int bb_highest(const BB &b)
-{
-    return b.w2 ? 191 - __builtin_clzll(b.w2) : b.w1 ? 127 - __builtin_clzll(b.w1) : 63 - __builtin_clzll(b.w0);
-}
-__device__ __forceinline__ uint64_t lowmask(int n)
-{   // bits [0, n) of a word, n clamped to [0, 64]
-    return n <= 0 ? 0ull : n >= 64 ? ~0ull : (1ull << n) - 1ull;
-}
-__device__ __forceinline__ BB bb_below(int c) { return {lowmask(c), lowmask(c - 64), lowmask(c - 128)}; }
-__device__ __forceinline__ BB bb_above(int c) { return {~lowmask(c + 1), ~lowmask(c - 63), ~lowmask(c - 127)}; }
 
-// Number of set bits of the 289-bit flat mask m below bit f (0 <= f < 289):
-// with m = on-board cells this is f's compact index, with m = rail cells its
-// rail index. The masks are uniform, so they sit in scalar registers.
-__device__ __forceinline__ int flat_rank(const uint64_t m[5], int f)
-{
-    int n = 0;
-#pragma unroll
-    for (int k = 0; k < 5; ++k) n += __popcll(m[k] & lowmask(f - 64 * k));
-    return n;
-}
-__device__ __forceinline__ bool flat_has(const uint64_t m[5], int f)
-{
-    const int k = f >> 6;
-    const uint64_t w = k == 0 ? m[0] : k == 1 ? m[1] : k == 2 ? m[2] : k == 3 ? m[3] : m[4];
-    return (w >> (f & 63)) & 1ull;
-}
-
-// Occupied cells and cells holding an enemy of `team` that may be attacked
-// (not in a camp) of the env whose board is `cell` (flat, LDS). Uniform.
-__device__ __forceinline__ void env_boards(const int8_t *cell, int team, BB &occ, BB &ea)
+// The board of an env as uniform sets: occupied cells, cells holding an enemy of
+// `team` that may be attacked (not in a camp), and the same of the track slots
+// (MoveTables; slots without a cell count as occupied, so every curve run ends
+// inside its own path). `cell` is the board (flat, LDS), T lane l's cells.
+struct Boards {
+    BB occ, ea;
+    uint64_t tocc, tea;
+};
+__device__ __forceinline__ void env_boards(const int8_t *cell, int team, const LaneRec &T, Boards &B)
 {
     const int l = lane_id();
-    const int p0 = cell[cT.c2f[l]], p1 = cell[cT.c2f[l + 64]], p2 = l == 0 ? cell[cT.c2f[128]] : -1;
-    occ = {__ballot(p0 >= 0), __ballot(p1 >= 0), __ballot(p2 >= 0)};
+    const int p0 = cell[T.c0], p1 = cell[T.c1], p2 = l == 0 ? cell[T.c2] : -1;
+    const int pt = T.track >= 0 ? cell[T.track] : -1;
+    B.occ = {__ballot(p0 >= 0), __ballot(p1 >= 0), __ballot(p2 >= 0)};
     const BB en = {__ballot(p0 >= 0 && team_of(p0) != team), __ballot(p1 >= 0 && team_of(p1) != team),
                    __ballot(p2 >= 0 && team_of(p2) != team)};
-    ea = {en.w0 & ~cT.campm[0], en.w1 & ~cT.campm[1], en.w2 & ~cT.campm[2]};
+    B.ea = {en.w0 & ~cT.campm[0], en.w1 & ~cT.campm[1], en.w2 & ~cT.campm[2]};
+    B.tocc = __ballot(T.track < 0 || pt >= 0);
+    B.tea = __ballot(pt >= 0 && team_of(pt) != team);   // no rail cell is a camp
 }
 
-// Road steps and, for non-engineers on a rail, straight runs and curve runs of
-// the piece on compact cell sc (rail index r or -1), lane-local
-// (move_gen.py:1052-1199 parts a, b, c, e), split in two halves so two lanes
-// share one piece: half h takes road / camp neighbours 4h .. 4h + 3 of adjc,
-// the +x / -x (h = 0) or +y / -y (h = 1) straight runs, and curve run h. The
-// union of both halves is the piece's move set. land = empty or attackable.
-__device__ __forceinline__ BB piece_moves_half(int sc, int r, bool engineer, int h, const BB &occ, const BB &ea)
+// Track slots [a, b) that the piece on track slot s reaches along its curve
+// rail: up the path (half 0) or down it (half 1), to the first occupied slot,
+// that one included if attackable.
+__device__ __forceinline__ void track_run(int s, int h, const Boards &B, int &a, int &b)
 {
-    const BB land = {~occ.w0 | ea.w0, ~occ.w1 | ea.w1, (~occ.w2 | ea.w2) & 1ull};
-    // this half's road / camp neighbours that are empty or attackable
-    const uint64_t *am = cT.adjm[sc][h];
-    BB m = {am[0] & land.w0, am[1] & land.w1, am[2] & land.w2};
-    if (engineer || r < 0) return m;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {   // k = 2h + j; j = 0 runs toward higher compact indices
-        const int k = 2 * h + j;
-        const BB run = {cT.raym[r][k][0], cT.raym[r][k][1], cT.raym[r][k][2]};
-        const BB blk = bb_and(run, occ);
-        if (!bb_any(blk)) {
-            m = bb_or(m, run);
-        } else {   // cells before the first occupied one, plus that one if attackable
-            const int f = j ? bb_highest(blk) : bb_lowest(blk);
-            m = bb_or(m, bb_and(run, j ? bb_above(f) : bb_below(f)));
-            if (bb_has(ea, f)) setbit3(m.w0, m.w1, m.w2, f);
-        }
+    const uint64_t up = B.tocc >> (s + 1), down = B.tocc & ((1ull << s) - 1);
+    const int eu = s + 1 + __builtin_ctzll(up | (1ull << 63)), ed = down ? 63 - __builtin_clzll(down) : -1;
+    const int e = h ? ed : eu, hit = e >= 0 ? (int)((B.tea >> (e & 63)) & 1) : 0;
+    a = h ? e + 1 - hit : s + 1;
+    b = h ? s : e + hit;
+}
+
+// The moves of a piece's half (MoveRec M, non-engineers' rail runs included),
+// the curve run excepted: road steps and straight runs to the first occupied
+// cell, that one included if attackable (move_gen.py:1052-1199 parts a, b, c).
+// blk ^ (blk - 1) is the lowest occupied cell and all below it.
+__device__ __forceinline__ BB straight_moves_half(const MoveRec &M, bool engineer, const Boards &B)
+{
+    const uint64_t n0 = ~B.occ.w0 | B.ea.w0, n1 = ~B.occ.w1 | B.ea.w1;   // empty or attackable
+    BB m = {M.adj[0] & n0, M.adj[1] & n1, (uint64_t)M.adj2 & (~B.occ.w2 | B.ea.w2)};
+    if (engineer) return m;   // off the rails both runs are empty
+    {
+        const uint64_t b0 = M.run[0][0] & B.occ.w0, b1 = M.run[0][1] & B.occ.w1;
+        const uint64_t v0 = b0 ^ (b0 - 1), v1 = b0 ? 0ull : b1 ^ (b1 - 1);
+        m.w0 |= M.run[0][0] & n0 & v0;
+        m.w1 |= M.run[0][1] & n1 & v1;
     }
-    const uint4 q = *reinterpret_cast<const uint4 *>(cT.crayc[r][h]);
-    uint64_t qlo = ((uint64_t)q.y << 32) | q.x, qhi = ((uint64_t)q.w << 32) | q.z;   // cells in walk order
-    bool open = true;
-    // walk until every lane of the wave has met its run's end or first
-    // occupied cell (runs are short and usually blocked early)
-    for (int i = 0; i < 12 && __ballot(open) != 0; ++i) {
-        const int c = (int)(qlo & 0xFF);
-        qlo = (qlo >> 8) | (qhi << 56);
-        qhi >>= 8;
-        if (!open) continue;
-        if (c == 0xFF) { open = false; continue; }
-        if (!bb_has(occ, c)) { setbit3(m.w0, m.w1, m.w2, c); continue; }
-        if (bb_has(ea, c)) setbit3(m.w0, m.w1, m.w2, c);
-        open = false;
+    {   // the highest occupied cell and all above it
+        const uint64_t b0 = M.run[1][0] & B.occ.w0, b1 = M.run[1][1] & B.occ.w1;
+        const uint64_t v1 = ~0ull << (63 - __builtin_clzll(b1 | 1)), v0 = b1 ? 0ull : ~0ull << (63 - __builtin_clzll(b0 | 1));
+        m.w0 |= M.run[1][0] & n0 & v0;
+        m.w1 |= M.run[1][1] & n1 & v1;
     }
     return m;
 }
@@ -1083,50 +1051,46 @@ __global__ __launch_bounds__(64) void k_finalize(State S, int beliefs, const uin
 // source order (move_gen.py:1199 sorts the ids).
 // Legal sets of env `env` for `seat` by its wave (off: none): the board in LDS
 // (cell, padded to CELL_STRIDE with -1), bits cleared and, for the canonical
-// mask, rotl filled. Piece positions / types come from the LDS arrays lpos /
-// ltype when given, else from the piece records.
+// mask, rotl filled. src / t: cell and type of piece l & 31 of the seat (lanes p
+// and p + 32 share piece p < 30, one half of its moves each).
 // lscr: LSCR_WORDS words of the wave's LDS, the compact source cells of the
 // movable pieces (words 0-2) and the engineers' rail destinations (3-11).
 // The masks go to row `row` (the env's own index, or the row of a minibatch
 // rebuilt from a history); REC: the legal record of the CSR pass is written.
+//
+// Bound: one wave's chain of dependent loads and VALU work, so what a piece
+// needs of its source cell is one record, asked for before the board is
+// scanned, and its curve run is two bit scans of the track slots (MoveTables).
+// From dependent table loads and a cell-by-cell walk of the curves this part went
+// from 5,400 to 1,130 cycles of a wave alone on its SIMD (us per fused step:
+// u8 32,768 games 738 -> 722, bf16 16,384 666 -> 658, state only 4,096 33.4 -> 32.1).
 template <bool REC = true>
 __device__ __forceinline__ void legal_body(const State &S, int env, int row, int l, int seat, bool off, const int8_t *cell, uint32_t *bits,
-                           const uint8_t *rotl, const int16_t *lpos, const int8_t *ltype, uint64_t *lscr,
+                           const uint8_t *rotl, int src, int t, uint64_t *lscr,
                            int32_t *__restrict__ counts, int32_t *__restrict__ mask_words, uint8_t *__restrict__ mask_bool)
 {
     const int team = seat & 1;
     uint64_t *srcset = lscr, *edst = lscr + 3;
-    if (l < 3) srcset[l] = 0;
-    BB occ, ea;
-    env_boards(cell, team, occ, ea);
-    // lanes p and p + 32 share piece p (p < 30), one half of its moves each
+    const LaneRec T = cM.lane[l];
     const int h = l >> 5, p = l & 31;
-    bool mov = false, eng = false;
-    int src = -1, ridx = -1, sc = 0;
+    const bool own = !off && p < 30 && (unsigned)src < (unsigned)NC;
+    const MoveRec M = cM.rec[own ? src : 0][h];   // cell 0 is off the board: an empty record
+    if (l < 3) srcset[l] = 0;
+    Boards B;
+    env_boards(cell, team, T, B);
+    const int sc = (int)(M.meta & 0xFF), ridx = (int)((M.meta >> 8) & 0xFF) - 1, slot = (int)(M.meta >> 24) - 1;
+    const bool mov = own && t != T_JUNQI && t != T_DILEI && ((M.meta >> 16) & (CF_ON | CF_SH)) == CF_ON;
+    const bool eng = mov && t == T_GONGB;
     uint64_t m0 = 0, m1 = 0, m2 = 0;
-    if (!off && p < 30) {
-        const int pid = seat * 30 + p;
-        int t;
-        if (lpos) {
-            src = lpos[pid];
-            t = ltype[pid];
-        } else {
-            const PieceRec r = S.piece[pc_idx(env, pid)];
-            src = r.pos;
-            t = r.ptype;
-        }
-        // the source cell's flags, compact index and rail index: one round of
-        // independent table loads
-        const int f = (unsigned)src < (unsigned)NC ? src : 0;
-        const int fl = cT.cflags[f], fc = cT.f2c[f], fr = cT.railidx[f];
-        mov = (unsigned)src < (unsigned)NC && t != T_JUNQI && t != T_DILEI && !(fl & CF_SH);
-        if (mov) {
-            eng = t == T_GONGB;
-            sc = fc;
-            ridx = fr;
-            const BB m = piece_moves_half(sc, ridx, eng, h, occ, ea);
-            m0 = m.w0; m1 = m.w1; m2 = m.w2;
-        }
+    if (mov) {
+        const BB m = straight_moves_half(M, eng, B);
+        m0 = m.w0; m1 = m.w1; m2 = m.w2;
+    }
+    {   // curve runs: cells of track slots [ta, tb), from the lanes' prefix sets
+        int ta = 0, tb = 0;
+        if (mov && !eng && slot >= 0) track_run(slot, h, B, ta, tb);
+        m0 |= (uint64_t)(__shfl((long long)T.pre[0], tb) ^ __shfl((long long)T.pre[0], ta));
+        m1 |= (uint64_t)(__shfl((long long)T.pre[1], tb) ^ __shfl((long long)T.pre[1], ta));
     }
     m0 |= (uint64_t)__shfl_xor((long long)m0, 32);
     m1 |= (uint64_t)__shfl_xor((long long)m1, 32);
@@ -1143,7 +1107,7 @@ __device__ __forceinline__ void legal_body(const State &S, int env, int row, int
             sr[j] = lanes[j] < 64 ? __builtin_amdgcn_readlane(ridx, lanes[j]) : -1;   // uniform lane
         }
         if (l < 9) edst[l] = 0;
-        engineers_bb(ne, sr, occ, ea, edst);
+        engineers_bb(ne, sr, B.occ, B.ea, edst);
         wave_sync();
 #pragma unroll
         for (int j = 0; j < 3; ++j)
@@ -1174,8 +1138,8 @@ __device__ __forceinline__ void legal_body(const State &S, int env, int row, int
     if (mov && (mask_words || mask_bool)) {
         const int cs = rotl[sc] * NONB;
         const uint64_t half = h ? 0xAAAAAAAAAAAAAAAAull : 0x5555555555555555ull;
-        uint64_t w[3] = {m0 & half, m1 & half, m2 & half};
-        for (int q = 0; q < 3; ++q) {
+        const uint64_t w[3] = {m0 & half, m1 & half, m2 & half};
+        for (int q = 0; q < 3; ++q) {   // a loop over two words at once, two lookups in flight, took 2,500 cycles for 1,900
             uint64_t x = w[q];
             while (x) {
                 const int b = __builtin_ctzll(x) + 64 * q;
@@ -1239,6 +1203,12 @@ __device__ __forceinline__ void legal_row(const State &S, int row, int l, LegalL
     const int seat = acting ? acting[row] : E.turn;
     const bool off = !stored || E.term || seat < 0 || seat > 3 || ((E.sdead >> (seat & 3)) & 1);
     for (int f = l; f < CELL_STRIDE; f += 64) L.cell[f] = f < NC ? S.cell[(size_t)env * CELL_STRIDE + f] : -1;
+    int src = -1, t = -1;   // the seat's piece l & 31
+    if (!off && (l & 31) < 30) {
+        const PieceRec r = S.piece[pc_idx(env, seat * 30 + (l & 31))];
+        src = r.pos;
+        t = r.ptype;
+    }
     // wave issue priority 2 through the legal pass, 0 for the bool rows'
     // stores (legal_body lowers it): a wave still computing gets issue slots
     // ahead of the waves that are storing rows (drop-in step at 32,768 games:
@@ -1250,8 +1220,7 @@ __device__ __forceinline__ void legal_row(const State &S, int row, int l, LegalL
         for (int c = l; c < NONB; c += 64) L.rotl[c] = cT.rotc[s4][c];
     }
     wave_sync();
-    legal_body<!HIST>(S, env, row, l, seat, off, L.cell, L.bits, L.rotl, nullptr, nullptr, L.lscr, counts, mask_words,
-                      mask_bool);
+    legal_body<!HIST>(S, env, row, l, seat, off, L.cell, L.bits, L.rotl, src, t, L.lscr, counts, mask_words, mask_bool);
 }
 
 template <bool HIST = false>
@@ -1783,8 +1752,9 @@ __device__ __forceinline__ void env_step_wave(const State &S, int env, int l, co
         for (int c = l; c < NONB; c += 64) E.rotl[c] = cT.rotc[seat & 3][c];
     }
     wave_sync();
-    legal_body(S, env, env, l, seat, off, E.cell, E.bits, E.rotl, E.pos, E.ptype, E.lscr, A.counts, A.mask_words,
-               nullptr);
+    const int mine = !off && (l & 31) < 30 ? seat * 30 + (l & 31) : -1;   // the next seat's piece of this lane
+    legal_body(S, env, env, l, seat, off, E.cell, E.bits, E.rotl, mine >= 0 ? E.pos[mine] : -1,
+               mine >= 0 ? E.ptype[mine] : -1, E.lscr, A.counts, A.mask_words, nullptr);
     if (l == 0) write_step_res(A.O, env, E.res);   // the step's reports go out last
 }
 

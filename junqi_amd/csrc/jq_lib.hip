@@ -92,6 +92,8 @@ std::mutex g_tab_mu;
 bool g_tab_done[64] = {};
 DeviceInfo g_dev[64];     // written once per device under g_tab_mu, before any handle of the device exists
 Tables g_tables;
+MoveTables g_moves;
+bool g_moves_ok = false;
 bool g_host_tables = false;
 uint8_t g_bval[BC_COUNT][12];
 float g_decode[256];
@@ -121,6 +123,7 @@ void build_host_tables()
 {
     if (g_host_tables) return;
     build_tables(g_tables);
+    g_moves_ok = build_move_tables(g_tables, g_moves);
     std::memset(g_decode, 0, sizeof g_decode);
     g_decode[0] = 0.f; g_decode[1] = 1.f; g_decode[2] = -1.f;
     g_decode[3] = 1.0f / 3.0f; g_decode[4] = 2.0f / 3.0f;
@@ -167,7 +170,9 @@ int ensure_device_tables(int device)
     build_host_tables();
     if (device < 0 || device >= 64) return fail(JQ_E_ARG, "device %d out of range", device);
     if (g_tab_done[device]) return JQ_OK;
+    if (!g_moves_ok) return fail(JQ_E_ARG, "the board's curve rails do not fit the move tables");
     HIP_TRY(hipMemcpyToSymbol(HIP_SYMBOL(cT), &g_tables, sizeof g_tables));
+    HIP_TRY(hipMemcpyToSymbol(HIP_SYMBOL(cM), &g_moves, sizeof g_moves));
     const ObsConsts oc = build_obs_consts();
     HIP_TRY(hipMemcpyToSymbol(HIP_SYMBOL(cOBS), &oc, sizeof oc));
     int per_cu = 0, cus = 0;
@@ -603,6 +608,16 @@ int jq_board_tables(void *host_out, int64_t nbytes)
     build_host_tables();
     if (!host_out || nbytes != (int64_t)sizeof(Tables)) return fail(JQ_E_ARG, "need %zu bytes", sizeof(Tables));
     std::memcpy(host_out, &g_tables, sizeof(Tables));
+    return JQ_OK;
+}
+
+int jq_move_tables(void *host_out, int64_t nbytes)
+{
+    std::lock_guard<std::mutex> lk(g_tab_mu);
+    build_host_tables();
+    if (!host_out || nbytes != (int64_t)sizeof(MoveTables)) return fail(JQ_E_ARG, "need %zu bytes", sizeof(MoveTables));
+    if (!g_moves_ok) return fail(JQ_E_ARG, "the board's curve rails do not fit the move tables");
+    std::memcpy(host_out, &g_moves, sizeof(MoveTables));
     return JQ_OK;
 }
 

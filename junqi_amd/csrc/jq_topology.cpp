@@ -234,6 +234,72 @@ void build_tables(Tables &t)
     }
 }
 
+bool build_move_tables(const Tables &t, MoveTables &m)
+{
+    std::memset(&m, 0, sizeof m);
+    int slot_of[NRAIL];
+    int16_t cells[64];
+    std::fill(slot_of, slot_of + NRAIL, -1);
+    std::fill(cells, cells + 64, (int16_t)-1);
+    int paths = 0;
+    for (int i = 0; i < NRAIL; ++i) {   // a path starts at an end not yet taken
+        if (t.craylen[i][0] == 0 || t.craylen[i][1] != 0 || slot_of[i] >= 0) continue;
+        const int n = 1 + t.craylen[i][0];
+        if (paths == 4 || n > 15) return false;
+        for (int j = 0; j < n; ++j) {
+            const int f = j ? t.crays[i][0][j - 1] : t.railcell[i], r = t.railidx[f];
+            if (slot_of[r] >= 0) return false;
+            slot_of[r] = 16 * paths + j;
+            cells[16 * paths + j] = (int16_t)f;
+        }
+        ++paths;
+    }
+    for (int i = 0; i < NRAIL; ++i) {   // both runs of every cell follow its path
+        const int n = t.craylen[i][0] + t.craylen[i][1];
+        if (slot_of[i] < 0) {
+            if (n) return false;
+            continue;
+        }
+        for (int d = 0; d < 2; ++d)
+            for (int j = 0; j < t.craylen[i][d]; ++j) {
+                const int up = slot_of[i] + 1 + j, down = slot_of[i] - 1 - j;
+                const bool rising = slot_of[t.railidx[t.crays[i][d][0]]] > slot_of[i];
+                if (cells[rising ? up : down] != t.crays[i][d][j]) return false;
+            }
+        int len = 0;
+        for (int s = slot_of[i] & ~15; s < 64 && cells[s] >= 0; ++s) ++len;
+        if (n != len - 1) return false;
+    }
+    for (int f = 0; f < NC; ++f) {
+        const int c = t.f2c[f], r = t.railidx[f];
+        if (c < 0) continue;
+        const uint32_t slot = r >= 0 ? (uint32_t)(slot_of[r] + 1) : 0u;
+        for (int h = 0; h < 2; ++h) {
+            MoveRec &R = m.rec[f][h];
+            R.adj[0] = t.adjm[c][h][0]; R.adj[1] = t.adjm[c][h][1]; R.adj2 = (uint32_t)t.adjm[c][h][2];
+            R.meta = (uint32_t)c | (uint32_t)(r + 1) << 8 | (uint32_t)(t.cflags[f] & 0xFF) << 16 | slot << 24;
+            for (int j = 0; r >= 0 && j < 2; ++j) {
+                const uint64_t *run = t.raym[r][2 * h + j];
+                if (run[2]) return false;
+                R.run[j][0] = run[0]; R.run[j][1] = run[1];
+            }
+        }
+    }
+    uint64_t pre[2] = {0, 0};
+    for (int l = 0; l < 64; ++l) {
+        LaneRec &L = m.lane[l];
+        L.pre[0] = pre[0]; L.pre[1] = pre[1];
+        L.c0 = t.c2f[l]; L.c1 = t.c2f[l + 64]; L.c2 = t.c2f[128];
+        L.track = cells[l];
+        if (cells[l] >= 0) {
+            const int c = t.f2c[cells[l]];
+            if (c >= 128) return false;
+            pre[c >> 6] |= 1ull << (c & 63);
+        }
+    }
+    return true;
+}
+
 // ---------------------------------------------------------------- lineups
 // Mersenne Twister as CPython's random module seeds and draws it.
 namespace {

@@ -59,7 +59,39 @@ struct Tables {
     uint8_t canc[4][NC];          // world flat -> canonical compact of observer s (0xFF off board)
 };
 
+// Everything move generation asks of a source cell, for one of the two lanes
+// (half 0 / 1) that share a piece, in one 64-byte record: what it can reach on
+// an empty board, as sets over compact cells (two words; only road steps reach
+// compact cell 128).
+struct alignas(16) MoveRec {
+    uint64_t adj[2];      // this half's road / camp neighbours (Tables::adjm)
+    uint64_t run[2][2];   // straight rail runs: +x / +y (rising), -x / -y (falling); half 0 x, half 1 y
+    uint32_t meta;        // compact | (rail index + 1) << 8 | (cflags & 0xFF) << 16 | (track slot + 1) << 24
+    uint32_t adj2;        // bit 0: compact cell 128 is one of the neighbours
+    uint32_t pad[2];
+};
+static_assert(sizeof(MoveRec) == 64, "move record must be 64 bytes");
+
+// The curve rails are four simple paths of at most 15 cells: path q takes track
+// slots 16q, 16q + 1, ... in walk order, so a piece's curve run is a run of
+// slots up or down from its own. Lane l's share of the board scan.
+struct alignas(16) LaneRec {
+    uint64_t pre[2];          // cells of the track slots below l, as a compact set
+    int16_t c0, c1, c2;       // flat cells of compact cells l, l + 64 and 128
+    int16_t track;            // flat cell of track slot l, -1 none
+    uint32_t pad[2];
+};
+static_assert(sizeof(LaneRec) == 32, "lane record must be 32 bytes");
+
+struct MoveTables {
+    MoveRec rec[NC][2];       // by flat source cell (zero off board)
+    LaneRec lane[64];
+};
+
 void build_tables(Tables &t);
+// false if the curve rails are not simple paths that fit the track slots, or a
+// rail run reaches compact cell 128
+bool build_move_tables(const Tables &t, MoveTables &m);
 void seat_cell(int seat, int slot, int &x, int &y);
 
 // CPython random.Random(seed) lineup stream of junqi_core.setup.generate_random_setup
