@@ -93,6 +93,13 @@ __device__ __forceinline__ bool is_sh(int f) { return cflags(f) & CF_SH; }
 __device__ __forceinline__ int curve_of(int f) { return cflags(f) >> 8; }
 __device__ __forceinline__ int team_of(int pid) { return (pid / 30) & 1; }
 
+// Bits [base, base + 30) of the 120-bit pid set (hi:lo), i.e. the 30 pids of one seat.
+__device__ __forceinline__ uint32_t seat_bits(uint64_t lo, uint64_t hi, int base)
+{
+    const uint64_t w = base == 0 ? lo : base < 64 ? ((lo >> base) | (hi << (64 - base))) : (hi >> (base - 64));
+    return (uint32_t)w & 0x3FFFFFFFu;
+}
+
 __device__ __forceinline__ bool enemy_att(const int8_t *cell, int f, int team)
 {   // enemy piece on a non-camp cell (move_gen.py:822-867)
     const int p = cell[f];
@@ -315,39 +322,25 @@ __device__ void piece_mask_lane(const int8_t *cell, int src, int team, bool engi
 }
 
 // dst on a straight run (k < 4) or curve run of src with every earlier cell empty
-// (move_gen.py:127-171 and 384-423). Wave-uniform: table reads are scalar loads.
-// A straight move stays on src's row or column, so only the run toward dst is
-// walked; its 12 entries come in with one batch of word loads.
+// (move_gen.py:127-171 and 384-423). Uniform; every lane active. A straight move
+// stays on src's row or column, so only the run toward dst is looked at; lane i
+// takes the run's cell i (curve runs: lanes 0-10 and 16-26), all cells at once.
 __device__ __forceinline__ bool run_clear(const int8_t *cell, int src, int dst, bool curve)
 {
-    typedef const __attribute__((address_space(4))) uint32_t *const_word;
-    const int r = tab(cT.railidx, src);
+    const int r = tab(cT.railidx, src), l = lane_id();
     if (r < 0) return false;
+    int nb = -1;   // the runs are padded with -1
     if (!curve) {
         const int sx = src % 17, sy = src / 17, dx = dst % 17, dy = dst / 17;
         const int k = sy == dy ? (dx > sx ? 0 : 1) : (dy > sy ? 2 : 3);   // +x, -x, +y, -y
-        const int len = tab(&cT.raylen[r][0], k);
-        const_word rw = reinterpret_cast<const_word>(reinterpret_cast<uintptr_t>(cT.rays[r][k]));
-        uint32_t w[6];
-#pragma unroll
-        for (int j = 0; j < 6; ++j) w[j] = rw[j];
-        for (int i = 0; i < 12; ++i) {
-            if (i >= len) break;
-            const int nb = (int16_t)(w[i >> 1] >> (16 * (i & 1)));
-            if (nb == dst) return true;
-            if (__builtin_amdgcn_readfirstlane(cell[nb]) >= 0) return false;
-        }
-        return false;
+        if (l < 12) nb = cT.rays[r][k][l];
+    } else if (l < 32 && (l & 15) < 11) {
+        nb = cT.crays[r][l >> 4][l & 15];
     }
-    for (int k = 0; k < 2; ++k) {
-        const int len = tab(&cT.craylen[r][0], k);
-        for (int i = 0; i < len; ++i) {
-            const int nb = tab(&cT.crays[r][k][0], i);
-            if (nb == dst) return true;
-            if (__builtin_amdgcn_readfirstlane(cell[nb]) >= 0) break;
-        }
-    }
-    return false;
+    const uint64_t hit = __ballot(nb == dst), occ = __ballot(nb >= 0 && cell[nb >= 0 ? nb : 0] >= 0);
+    if (!hit) return false;
+    const int at = __builtin_ctzll(hit);   // a cell is on one of the two curve runs only
+    return (occ & ((1ull << at) - (1ull << (at & 48)))) == 0;
 }
 
 __device__ __forceinline__ bool engineer_reaches(const int8_t *cell, int src, int dst)
@@ -360,45 +353,29 @@ __device__ __forceinline__ bool engineer_reaches(const int8_t *cell, int src, in
     return ((t0 & r0) | (t1 & r1)) != 0;
 }
 
-// is_legal_move (move_gen.py:299-376), uniform over the wave.
-__device__ __forceinline__ bool legal_pair(const int8_t *cell, const int8_t *ptype, int seat, int src, int dst)
+// is_legal_move (move_gen.py:299-376) of the piece sp of type st on src to dst,
+// where dp stands (-1 none), and move_requires_gongb (move_gen.py:245-296) of a
+// legal engineer move. Uniform; src and dst are cells of the 17 x 17 board. A
+// straight or curve run that is clear is also a path of the engineer's closure,
+// so an engineer's closure is grown only where no run reaches dst.
+__device__ __forceinline__ bool legal_pair(const int8_t *cell, int seat, int src, int dst, int sp, int st, int dp,
+                                           bool &engineer_only)
 {
-    if (src < 0 || src >= NC || dst < 0 || dst >= NC || src == dst) return false;
-    if (!is_on(src) || !is_on(dst)) return false;
-    const int p = __builtin_amdgcn_readfirstlane(cell[src]);   // LDS reads at uniform cells: uniform values
-    if (p < 0 || p / 30 != seat) return false;
-    const int t = __builtin_amdgcn_readfirstlane(ptype[p]);
-    if (t < T_ZHADAN || t > T_GONGB) return false;   // JUNQI / DILEI never move (no other value is a piece)
-    if (is_sh(src)) return false;
-    const int q = __builtin_amdgcn_readfirstlane(cell[dst]);   // landable: empty, or an enemy outside a camp
-    if (q >= 0 && (team_of(q) == (seat & 1) || is_camp(dst))) return false;
+    engineer_only = false;
+    const uint16_t fs = cflags(src), fd = cflags(dst);
+    if (src == dst || !(fs & CF_ON) || !(fd & CF_ON)) return false;
+    if (sp < 0 || sp / 30 != seat) return false;
+    if (st < T_ZHADAN || st > T_GONGB) return false;   // JUNQI / DILEI never move (no other value is a piece)
+    if (fs & CF_SH) return false;
+    if (dp >= 0 && (team_of(dp) == (seat & 1) || (fd & CF_CAMP))) return false;   // landable: empty, or an enemy outside a camp
     const int sx = src % 17, sy = src / 17, dx = dst % 17, dy = dst / 17;
     const int adx = abs(sx - dx), ady = abs(sy - dy);
-    if (adx <= 1 && ady <= 1) {
-        if (adx == 1 && ady == 1) { if (is_camp(src) || is_camp(dst)) return true; }
-        else return true;
-    }
-    if (!(is_rail(src) && is_rail(dst))) return false;
-    if (t == T_GONGB) return engineer_reaches(cell, src, dst);
-    if (sx == dx || sy == dy) return run_clear(cell, src, dst, false);
-    if (curve_of(src) > 0 && curve_of(src) == curve_of(dst)) return run_clear(cell, src, dst, true);
-    return false;
-}
-
-// move_requires_gongb (move_gen.py:245-296) for a legal engineer move.
-__device__ __forceinline__ bool engineer_only(const int8_t *cell, int src, int dst)
-{
-    const int sx = src % 17, sy = src / 17, dx = dst % 17, dy = dst / 17;
-    const int adx = abs(sx - dx), ady = abs(sy - dy);
-    if (adx + ady == 1) return false;
-    if (adx == 1 && ady == 1 && (is_camp(src) || is_camp(dst))) return false;
-    if (!(is_rail(src) && is_rail(dst))) return false;
-    if (sx == dx || sy == dy) {
-        if (run_clear(cell, src, dst, false)) return false;
-        return engineer_reaches(cell, src, dst);
-    }
-    if (curve_of(src) > 0 && curve_of(src) == curve_of(dst) && run_clear(cell, src, dst, true)) return false;
-    return engineer_reaches(cell, src, dst);
+    if (adx <= 1 && ady <= 1 && (adx + ady == 1 || ((fs | fd) & CF_CAMP))) return true;
+    if (!(fs & fd & CF_RAIL)) return false;
+    const bool straight = sx == dx || sy == dy, curve = (fs >> 8) > 0 && (fs >> 8) == (fd >> 8);
+    if ((straight || curve) && run_clear(cell, src, dst, !straight)) return true;
+    engineer_only = st == T_GONGB && engineer_reaches(cell, src, dst);
+    return engineer_only;
 }
 
 // Does `seat` have a legal move (the Q12 test, state.py:1139-1165)?
@@ -453,13 +430,14 @@ __device__ __forceinline__ int resolve_combat(int a, int d)
 typedef const __attribute__((address_space(4))) uint64_t *KeyTable;
 __device__ __forceinline__ KeyTable keys(const uint64_t *z) { return reinterpret_cast<KeyTable>(reinterpret_cast<uintptr_t>(z)); }
 
-__device__ __forceinline__ uint64_t zp(const uint64_t *z, int pid, int t, int f)
+__device__ __forceinline__ int zp_index(int pid, int t, int f)
 {   // indexes come from state rows; out-of-range values read entry 0 instead of faulting
     pid = (unsigned)pid < 120u ? pid : 0;
     t = (unsigned)t < 14u ? t : 0;
     f = (unsigned)f < 289u ? f : 0;
-    return keys(z)[((size_t)pid * 14 + t) * 289 + f];
+    return (pid * 14 + t) * 289 + f;
 }
+__device__ __forceinline__ uint64_t zp(const uint64_t *z, int pid, int t, int f) { return keys(z)[zp_index(pid, t, f)]; }
 
 __device__ __forceinline__ int tracked(int t) { return (t >= 2 && t <= 13) ? t - 2 : -1; }
 __device__ __forceinline__ bool code_onehot(int c) { return c >= 1 && c <= 12; }
@@ -504,60 +482,44 @@ __device__ __forceinline__ void write_step_res(const StepOut &O, int env, const 
     if (O.hash) O.hash[env] = r.hash;
 }
 
-// Kill pid at its current cell (state.py:1027-1049). Uniform; lane 0 stores.
-__device__ void kill_piece(const State &S, int env, int8_t *cell, int16_t *pos, const int8_t *ptype, int pid,
-                           int reason, int loc, int step, uint64_t &zob)
-{
-    const int cur = __builtin_amdgcn_readfirstlane(pos[pid]);
-    if ((unsigned)cur >= (unsigned)NC) return;
-    zob ^= zp(S.ztab, pid, __builtin_amdgcn_readfirstlane(ptype[pid]), cur);
-    wave_sync();
-    if (lane_id() == 0) {
-        cell[cur] = -1; pos[pid] = -1;
-        PieceRec &r = S.piece[pc_idx(env, pid)];
-        r.pos = -1; r.dreason = (int8_t)reason; r.dstep = (int16_t)step; r.dloc = (int16_t)loc;
-        S.cell[(size_t)env * CELL_STRIDE + cur] = -1;
-    }
-    wave_sync();
-}
-
-__device__ void move_piece(const State &S, int env, int8_t *cell, int16_t *pos, const int8_t *ptype, int pid,
-                           int src, int dst, uint64_t &zob)
-{   // state.py:1005-1025
-    const int t = __builtin_amdgcn_readfirstlane(ptype[pid]);
-    zob ^= zp(S.ztab, pid, t, src) ^ zp(S.ztab, pid, t, dst);
-    wave_sync();
-    if (lane_id() == 0) {
-        cell[src] = -1; cell[dst] = (int8_t)pid; pos[pid] = (int16_t)dst;
-        S.cell[(size_t)env * CELL_STRIDE + src] = -1;
-        S.cell[(size_t)env * CELL_STRIDE + dst] = (int8_t)pid;
-        S.piece[pc_idx(env, pid)].pos = (int16_t)dst;
-    }
-    wave_sync();
-}
-
 // Remove every live piece of `seat` (state.py:1639-1692): KILLED_BY_ENEMY at the
-// piece's current cell. Lanes 0..29 take one pid each; Zobrist folded by XOR.
+// piece's current cell. Lanes 0..29 take one pid each and fold its key into
+// their share zacc of the Zobrist change.
 __device__ void purge_seat(const State &S, int env, int8_t *cell, int16_t *pos, const int8_t *ptype, int seat,
-                           int step, uint64_t &zob)
+                           int step, uint64_t &zacc)
 {
     const int l = lane_id();
-    uint64_t z = 0;
     wave_sync();
     if (l < 30) {
         const int pid = seat * 30 + l;
         const int cur = pos[pid];
         if ((unsigned)cur < (unsigned)NC) {
-            z = zp(S.ztab, pid, ptype[pid], cur);
+            zacc ^= zp(S.ztab, pid, ptype[pid], cur);
             cell[cur] = -1; pos[pid] = -1;
             PieceRec &r = S.piece[pc_idx(env, pid)];
             r.pos = -1; r.dreason = 0; r.dstep = (int16_t)step; r.dloc = (int16_t)cur;
             S.cell[(size_t)env * CELL_STRIDE + cur] = -1;
         }
     }
-    zob ^= wave_xor(z);
     wave_sync();
 }
+
+// The Zobrist keys a ply may XOR in, one per lane, loaded together as soon as
+// the moving pieces are known: the ply collects the lanes that count in a
+// uniform set and folds them once at its end. (As scalar loads each was waited
+// for at the wave's next LDS fence, which shares their counter.) With the kills
+// and the move in one block, one legality walk, counters from the records
+// already loaded and boards moved as words, a wave's ply went from 8,112 to
+// 6,545 lines of assembly and 23.6 k to 20.8 k cycles alone on its SIMD (us per
+// fused step: u8 32,768 games 723 -> 713, bf16 16,384 658 -> 652, state only
+// 4,096 32.1 -> 29.6, u8 64 25.2 -> 23.8).
+enum : int {
+    ZL_TURN = 0, ZL_MC0 = 4, ZL_MC1 = 5, ZL_MSLC0 = 6, ZL_MSLC1 = 7, ZL_MSLC_RESET = 8, ZL_SRC = 9, ZL_DST = 10,
+    ZL_KILL_D = 11, ZL_KILL_S = 12, ZL_TERM = 16, ZL_WIN = ZL_TERM + (ZOFF_WIN - ZOFF_TERM),
+    ZL_DRAW = ZL_TERM + (ZOFF_DRAW - ZOFF_TERM), ZL_SDEAD = ZL_TERM + (ZOFF_SDEAD - ZOFF_TERM),
+    ZL_SFLAG = ZL_TERM + (ZOFF_SFLAG - ZOFF_TERM), ZL_END = ZL_SFLAG + 4
+};
+static_assert(ZL_END <= 32, "one bit of a 32-bit set per key");
 
 // CombatMemory update for EAT / KILLED (combat_memory.py:354-569). Lane o < 4
 // handles observer o; observers never touch each other's records. K is the
@@ -624,20 +586,19 @@ __device__ __forceinline__ void cm_apply(const State &S, int env, bool is_eat, i
 }
 
 // BeliefTensor.update for the four observers (info_model.py:271-429). Entries are
-// keyed by pid so R1 migration is implicit; lane o < 4 handles observer o.
+// keyed by pid so R1 migration is implicit; lane o < 4 handles observer o, whose
+// tracked seats (trk) and codes of the two pieces are loaded by the caller.
 __device__ __forceinline__ void belief_update(const State &S, int env, const int8_t *cell, int sp, int dp, int ss, int ds,
-                              int dt, int dst, int ev, bool rsrc, bool rdst, bool fcap, int died)
+                              int dt, int dst, int ev, bool rsrc, bool rdst, bool fcap, int died, uint8_t trk,
+                              int acode, const int dcode)
 {
     const int o = lane_id();
     if (o >= 4) return;
     uint8_t *bc = S.bcode + ((size_t)env * 4 + o) * PID_STRIDE;
     int8_t *rem = S.rem + ((size_t)env * 4 + o) * 48;
-    uint8_t trk = S.env[env].remtrk[o];
     auto dec = [&](int seat, int ti) {
         if ((trk >> seat) & 1) { int8_t &c = rem[seat * 12 + ti]; if (c > 0) --c; }
     };
-    int acode = bc[sp];
-    const int dcode = dp >= 0 ? bc[dp] : 0;
     if (rsrc) dec(ss, T_SILING - 2);
     if (rdst) dec(ds, T_SILING - 2);
     if (ev == EV_EAT && dp >= 0 && dt == T_DILEI && !code_onehot(acode)) {
@@ -674,19 +635,37 @@ struct TurnAfter {
 // The board and piece records of one env, lane l's share: the loads of a ply's
 // first memory round trip, which a caller can issue early.
 struct StepLoad {
-    int8_t cv[5];
-    PieceRec r0, r1;
+    uint32_t c0, c1;   // board words l and l + 64 (l < 9)
+    uint4 r0, r1;      // records of pids l and l + 64
 };
+
+// A board is 73 words in global memory and in LDS, the three bytes past its last
+// cell -1. Lane l moves words l and l + 64.
+__device__ __forceinline__ void board_load(const State &S, int env, int l, uint32_t &c0, uint32_t &c1)
+{
+    const uint32_t *w = reinterpret_cast<const uint32_t *>(S.cell + (size_t)env * CELL_STRIDE);
+    c0 = w[l];
+    c1 = w[min(l + 64, CELL_STRIDE / 4 - 1)];
+}
+__device__ __forceinline__ void board_stage(int8_t *cell, int l, uint32_t c0, uint32_t c1)
+{
+    static_assert(CELL_STRIDE / 4 == 73 && NC == 289, "the last word holds one cell");
+    uint32_t *w = reinterpret_cast<uint32_t *>(cell);
+    w[l] = c0;
+    if (l < CELL_STRIDE / 4 - 64) w[l + 64] = l == CELL_STRIDE / 4 - 65 ? c1 | 0xFFFFFF00u : c1;
+}
 
 __device__ __forceinline__ void step_load(const State &S, int env, int l, StepLoad &P)
 {
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-        const int f = l + 64 * k;
-        P.cv[k] = f < NC ? S.cell[(size_t)env * CELL_STRIDE + f] : (int8_t)-1;
-    }
-    P.r0 = S.piece[pc_idx(env, l)];
-    P.r1 = S.piece[pc_idx(env, l + 64)];
+    board_load(S, env, l, P.c0, P.c1);
+    P.r0 = *reinterpret_cast<const uint4 *>(&S.piece[pc_idx(env, l)]);
+    P.r1 = *reinterpret_cast<const uint4 *>(&S.piece[pc_idx(env, l + 64)]);
+}
+__device__ __forceinline__ PieceRec piece_rec(const uint4 &v)
+{
+    PieceRec r;
+    __builtin_memcpy(&r, &v, sizeof r);
+    return r;
 }
 
 __device__ void step_env(const State &S, int env, int l, int32_t a, const int8_t *__restrict__ acting, int act_fmt,
@@ -701,14 +680,11 @@ __device__ void step_env(const State &S, int env, int l, int32_t a, const int8_t
     StepLoad ld;
     if (pre) ld = *pre;
     else step_load(S, env, l, ld);
-    const int8_t *cv = ld.cv;
-    const PieceRec &r0 = ld.r0, &r1 = ld.r1;
+    const PieceRec r0 = piece_rec(ld.r0), r1 = piece_rec(ld.r1);
     // the env record, read once into scalar registers before any store of the
     // ply (only this wave writes it, at the end), or handed in by the caller
     const EnvRec E = pre_rec ? *pre_rec : env_record(S, env);
-#pragma unroll
-    for (int k = 0; k < 5; ++k)
-        if (l + 64 * k < CELL_STRIDE) cell[l + 64 * k] = cv[k];
+    board_stage(cell, l, ld.c0, ld.c1);
     pos[l] = r0.pos; ptype[l] = r0.ptype;
     pos[l + 64] = r1.pos; ptype[l + 64] = r1.ptype;
     const bool was_term = E.term != 0;
@@ -734,20 +710,46 @@ __device__ void step_env(const State &S, int env, int l, int32_t a, const int8_t
     const uint8_t sdead0 = E.sdead;
     if ((sdead0 >> seat) & 1) return;
     wave_sync();
-    if (!legal_pair(cell, ptype, seat, src, dst)) return;
+    // the pieces on both cells, their types and cells: two rounds of LDS reads
+    const int sp = __builtin_amdgcn_readfirstlane(cell[src]), dp = __builtin_amdgcn_readfirstlane(cell[dst]);
+    int st = -1, dt = -1, spos = -1, dpos = -1;
+    {
+        const int a = sp >= 0 ? sp : 0, d = dp >= 0 ? dp : 0;
+        const int v0 = ptype[a], v1 = ptype[d], v2 = pos[a], v3 = pos[d];
+        st = __builtin_amdgcn_readfirstlane(v0);
+        spos = __builtin_amdgcn_readfirstlane(v2);
+        if (dp >= 0) { dt = __builtin_amdgcn_readfirstlane(v1); dpos = __builtin_amdgcn_readfirstlane(v3); }
+    }
+    bool gongb_only;
+    if (!legal_pair(cell, seat, src, dst, sp, st, dp, gongb_only)) return;
 
     const int mc0 = E.mc, mslc0 = E.mslc;
-    uint64_t zob = E.zob;
-    const KeyTable Z = keys(S.ztab);
-    zob ^= Z[ZOFF_TURN + seat] ^ Z[ZOFF_MC + (mc0 & 0xFFF)] ^ Z[ZOFF_MSLC + (mslc0 & 0x1FF)];
     const int step = mc0 + 1;
     int died = 0;
     uint8_t sdead = sdead0, sflag = E.sflag;
-    const int sp = __builtin_amdgcn_readfirstlane(cell[src]), dp = __builtin_amdgcn_readfirstlane(cell[dst]);
-    const int st = __builtin_amdgcn_readfirstlane(ptype[sp]), dt = dp >= 0 ? __builtin_amdgcn_readfirstlane(ptype[dp]) : -1;
     const int ss = sp / 30, ds = dp >= 0 ? dp / 30 : -1;
 
-    if (st == T_GONGB && engineer_only(cell, src, dst)) {
+    // loads whose values are only needed at the ply's end: the Zobrist keys
+    // (lane ZL_*) and the four observers' belief codes of the two pieces
+    int zi = l < 4 ? ZOFF_TURN + l : ZOFF_TERM + (l < ZL_END ? l - ZL_TERM : 0);
+    // the value is fixed as a scalar first, so that this is a select and not a branch
+    auto put = [&](int lane, int v) { v = __builtin_amdgcn_readfirstlane(v); zi = l == lane ? v : zi; };
+    put(ZL_MC0, ZOFF_MC + (mc0 & 0xFFF));
+    put(ZL_MC1, ZOFF_MC + ((mc0 + 1) & 0xFFF));
+    put(ZL_MSLC0, ZOFF_MSLC + (mslc0 & 0x1FF));
+    put(ZL_MSLC1, ZOFF_MSLC + ((mslc0 + 1) & 0x1FF));
+    put(ZL_MSLC_RESET, ZOFF_MSLC);
+    put(ZL_SRC, zp_index(sp, st, src));
+    put(ZL_DST, zp_index(sp, st, dst));
+    put(ZL_KILL_D, zp_index(dp, dt, dpos));
+    put(ZL_KILL_S, zp_index(sp, st, spos));
+    const uint64_t zkey = S.ztab[zi];
+    const uint8_t *bc = S.bcode + ((size_t)env * 4 + (l & 3)) * PID_STRIDE;   // every lane loads, lanes 0-3 use it
+    const int acode = bc[sp], dcode = bc[dp >= 0 ? dp : sp];                  // dcode: only with a piece on dst
+    uint64_t zm = 1u << (ZL_TURN + seat) | 1u << ZL_MC0 | 1u << ZL_MSLC0;   // the lanes whose keys count
+    uint64_t zacc = 0;                                                      // this lane's purged pieces
+
+    if (gongb_only) {
         if (l < 4) {
             S.cm[cm_idx(env, l, sp)].flags |= CMF_IS_GONGB;
             S.cmk[cm_idx(env, l, sp)] |= (uint8_t)(CMF_IS_GONGB << 2);
@@ -759,45 +761,57 @@ __device__ void step_env(const State &S, int env, int l, int32_t a, const int8_t
     if (l == 0) S.hist[(size_t)env * HIST_LEN + hhead] = src | (dst << 16);
     int ev;
     bool rsrc = false, rdst = false, fcap = false;
-    auto set_flag = [&](int s) { if (!((sflag >> s) & 1)) { sflag |= (uint8_t)(1u << s); zob ^= Z[ZOFF_SFLAG + s]; } };
-    auto set_dead = [&](int s) { if (!((sdead >> s) & 1)) { sdead |= (uint8_t)(1u << s); zob ^= Z[ZOFF_SDEAD + s]; } };
-    if (dp < 0) {
-        ev = EV_MOVE;
-        if (l == 0) S.piece[pc_idx(env, sp)].mcount += 1;
-        move_piece(S, env, cell, pos, ptype, sp, src, dst, zob);
-    } else {
-        ev = resolve_combat(st, dt);
+    auto set_flag = [&](int s) { if (!((sflag >> s) & 1)) { sflag |= (uint8_t)(1u << s); zm ^= 1u << (ZL_SFLAG + s); } };
+    auto set_dead = [&](int s) { if (!((sdead >> s) & 1)) { sdead |= (uint8_t)(1u << s); zm ^= 1u << (ZL_SDEAD + s); } };
+    ev = dp < 0 ? EV_MOVE : resolve_combat(st, dt);
+    const bool moved = ev == EV_MOVE || ev == EV_EAT;
+    const bool kill_s = (ev == EV_KILLED || ev == EV_BOMB) && (unsigned)spos < (unsigned)NC;   // a piece on no cell stays as it is
+    const bool kill_d = (ev == EV_EAT || ev == EV_BOMB) && (unsigned)dpos < (unsigned)NC;
+    if (dp >= 0) {
         rsrc = st == T_SILING && (ev == EV_KILLED || ev == EV_BOMB);
         rdst = dt == T_SILING && (ev == EV_EAT || ev == EV_BOMB);
         fcap = dt == T_JUNQI;
         if (rsrc) set_flag(ss);
         if (rdst) set_flag(ds);
-        if (ev == EV_EAT) {
-            if (l == 0) S.piece[pc_idx(env, sp)].aeat += 1;
-            kill_piece(S, env, cell, pos, ptype, dp, 0, dst, step, zob);
-            move_piece(S, env, cell, pos, ptype, sp, src, dst, zob);
-            cm_apply(S, env, true, sp, dp, ss, ds, st, dt, step);
-        } else if (ev == EV_KILLED) {
-            if (l == 0) S.piece[pc_idx(env, dp)].psurv += 1;
-            kill_piece(S, env, cell, pos, ptype, sp, (dt == T_DILEI || dt == T_ZHADAN) ? 1 : 0, dst, step, zob);
-            cm_apply(S, env, false, sp, dp, ss, ds, st, dt, step);
-        } else {
-            kill_piece(S, env, cell, pos, ptype, sp, 2, dst, step, zob);
-            kill_piece(S, env, cell, pos, ptype, dp, 2, dst, step, zob);
-        }
     }
+    if (kill_s) zm ^= 1u << ZL_KILL_S;
+    if (kill_d) zm ^= 1u << ZL_KILL_D;
+    if (moved) zm ^= 1u << ZL_SRC | 1u << ZL_DST;
+    // the counter of a move, a capture or a survived attack, by the lane that
+    // loaded the piece's record
+    const int cp = ev == EV_KILLED ? dp : sp;
+    if (ev != EV_BOMB && l == (cp & 63)) {
+        const int16_t m = cp < 64 ? r0.mcount : r1.mcount, e = cp < 64 ? r0.aeat : r1.aeat, v = cp < 64 ? r0.psurv : r1.psurv;
+        int16_t *c = &S.piece[pc_idx(env, cp)].mcount;   // mcount, aeat, psurv in a row
+        c[ev == EV_MOVE ? 0 : ev == EV_EAT ? 1 : 2] = (int16_t)((ev == EV_MOVE ? m : ev == EV_EAT ? e : v) + 1);
+    }
+    wave_sync();
+    // kills (state.py:1027-1049): lane 0 the piece on dst, lane 1 the mover
+    if (l < 2 && (l ? kill_s : kill_d)) {
+        const int pid = l ? sp : dp, cur = l ? spos : dpos;
+        const int why = ev == EV_BOMB ? 2 : (l && (dt == T_DILEI || dt == T_ZHADAN)) ? 1 : 0;
+        cell[cur] = -1; pos[pid] = -1;
+        PieceRec &r = S.piece[pc_idx(env, pid)];
+        r.pos = -1; r.dreason = (int8_t)why; r.dstep = (int16_t)step; r.dloc = (int16_t)dst;
+        S.cell[(size_t)env * CELL_STRIDE + cur] = -1;
+    }
+    if (moved && l == 0) {   // state.py:1005-1025; after lane 0's own kill on dst
+        cell[src] = -1; cell[dst] = (int8_t)sp; pos[sp] = (int16_t)dst;
+        S.cell[(size_t)env * CELL_STRIDE + src] = -1;
+        S.cell[(size_t)env * CELL_STRIDE + dst] = (int8_t)sp;
+        S.piece[pc_idx(env, sp)].pos = (int16_t)dst;
+    }
+    wave_sync();
+    if (ev == EV_EAT || ev == EV_KILLED) cm_apply(S, env, ev == EV_EAT, sp, dp, ss, ds, st, dt, step);
     if (fcap && !((sdead >> ds) & 1)) {   // state.py:864-890
         set_dead(ds); set_flag(ds);
-        purge_seat(S, env, cell, pos, ptype, ds, step, zob);
+        purge_seat(S, env, cell, pos, ptype, ds, step, zacc);
         died |= 1 << ds;
     }
     {   // dead sweep (state.py:895-901)
-        const int p0 = l, p1 = l + 64;
-        const bool a0 = pos[p0] >= 0, a1 = p1 < NP && pos[p1] >= 0;
-        for (int s = 0; s < 4; ++s) {
-            const bool has = __ballot((a0 && p0 / 30 == s) || (a1 && p1 / 30 == s)) != 0;
-            if (!((sdead >> s) & 1) && !has) { set_dead(s); died |= 1 << s; }
-        }
+        const uint64_t a0 = __ballot(pos[l] >= 0), a1 = __ballot(l + 64 < NP && pos[l + 64] >= 0);   // pids on the board
+        for (int s = 0; s < 4; ++s)
+            if (!((sdead >> s) & 1) && !seat_bits(a0, a1, s * 30)) { set_dead(s); died |= 1 << s; }
     }
     const int nmc = mc0 + 1, nmslc = ev == EV_MOVE ? mslc0 + 1 : 0;
     auto victory = [&](int &term, int &win, int &drw) {   // state.py:1695-1726
@@ -817,7 +831,7 @@ __device__ void step_env(const State &S, int env, int l, int32_t a, const int8_t
             if ((sdead >> cand) & 1) { cand = (cand + 1) & 3; continue; }
             if (seat_has_move(cell, pos, ptype, cand)) break;
             set_dead(cand);
-            purge_seat(S, env, cell, pos, ptype, cand, step, zob);
+            purge_seat(S, env, cell, pos, ptype, cand, step, zacc);
             died |= 1 << cand;
             cand = (cand + 1) & 3;
         }
@@ -827,12 +841,15 @@ __device__ void step_env(const State &S, int env, int l, int32_t a, const int8_t
         nturn = seat;
     }
     if (!term && nmc >= S.max_moves) { term = 1; drw = 1; }   // env move cap
-    zob ^= Z[ZOFF_TURN + nturn] ^ Z[ZOFF_MC + (nmc & 0xFFF)] ^ Z[ZOFF_MSLC + (nmslc & 0x1FF)];
-    if (term) zob ^= Z[ZOFF_TERM];
-    if (drw) zob ^= Z[ZOFF_DRAW];
-    if (win >= 0) zob ^= Z[ZOFF_WIN] ^ Z[ZOFF_WIN + win + 1];
+    zm ^= 1u << (ZL_TURN + nturn) | 1u << ZL_MC1;
+    zm ^= 1u << (ev == EV_MOVE ? ZL_MSLC1 : ZL_MSLC_RESET);
+    if (term) zm ^= 1u << ZL_TERM;
+    if (drw) zm ^= 1u << ZL_DRAW;
+    if (win >= 0) zm ^= 1u << ZL_WIN | 1u << (ZL_WIN + win + 1);
+    const uint64_t zob = E.zob ^ wave_xor(zacc ^ ((zm >> l) & 1 ? zkey : 0ull));
 
-    belief_update(S, env, cell, sp, dp, ss, ds, dt, dst, ev, rsrc, rdst, fcap, died);
+    const uint8_t trk = l == 0 ? E.remtrk[0] : l == 1 ? E.remtrk[1] : l == 2 ? E.remtrk[2] : E.remtrk[3];
+    belief_update(S, env, cell, sp, dp, ss, ds, dt, dst, ev, rsrc, rdst, fcap, died, trk, acode, dcode);
 
     nx.turn = nturn; nx.term = term != 0; nx.sdead = sdead;
     if (l == 0) {
@@ -852,7 +869,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) void
 {
     const int env = blockIdx.x, l = threadIdx.x;
     if (env >= S.n) return;
-    __shared__ int8_t cell[CELL_STRIDE];
+    __shared__ alignas(4) int8_t cell[CELL_STRIDE];
     __shared__ int16_t pos[PID_STRIDE];
     __shared__ int8_t ptype[PID_STRIDE];
     TurnAfter nx;
@@ -1179,7 +1196,7 @@ __device__ __forceinline__ void legal_body(const State &S, int env, int row, int
 struct LegalLds {
     uint64_t lscr[LSCR_WORDS];
     uint32_t bits[JQ_MASK_WORDS_PAD];
-    int8_t cell[CELL_STRIDE];
+    alignas(4) int8_t cell[CELL_STRIDE];
     uint8_t rotl[NONB + 3];   // world compact -> canonical compact of the acting seat
 };
 
@@ -1202,10 +1219,11 @@ __device__ __forceinline__ void legal_row(const State &S, int row, int l, LegalL
     const EnvRec &E = S.env[env];
     const int seat = acting ? acting[row] : E.turn;
     const bool off = !stored || E.term || seat < 0 || seat > 3 || ((E.sdead >> (seat & 3)) & 1);
-    for (int f = l; f < CELL_STRIDE; f += 64) L.cell[f] = f < NC ? S.cell[(size_t)env * CELL_STRIDE + f] : -1;
+    uint32_t c0, c1;
+    board_load(S, env, l, c0, c1);
     int src = -1, t = -1;   // the seat's piece l & 31
     if (!off && (l & 31) < 30) {
-        const PieceRec r = S.piece[pc_idx(env, seat * 30 + (l & 31))];
+        const PieceRec r = piece_rec(*reinterpret_cast<const uint4 *>(&S.piece[pc_idx(env, seat * 30 + (l & 31))]));
         src = r.pos;
         t = r.ptype;
     }
@@ -1215,6 +1233,7 @@ __device__ __forceinline__ void legal_row(const State &S, int row, int l, LegalL
     // 2.486 -> 2.474 ms)
     __builtin_amdgcn_s_setprio(2);
     for (int w = l; w < JQ_MASK_WORDS_PAD; w += 64) L.bits[w] = 0;
+    board_stage(L.cell, l, c0, c1);
     if (mask_words || mask_bool) {
         const int s4 = seat & 3;
         for (int c = l; c < NONB; c += 64) L.rotl[c] = cT.rotc[s4][c];
@@ -1689,7 +1708,7 @@ struct EnvLds {
     uint64_t lscr[LSCR_WORDS];
     int16_t pos[PID_STRIDE];
     int8_t ptype[PID_STRIDE];
-    int8_t cell[CELL_STRIDE];
+    alignas(4) int8_t cell[CELL_STRIDE];
     uint8_t rotl[NONB + 3];
 };
 

@@ -147,13 +147,6 @@ __device__ __forceinline__ uint16_t f32_to_bf16_rne(float f)
     return (uint16_t)(u >> 16);
 }
 
-// Bits [base, base + 30) of the 120-bit pid set (hi:lo), i.e. the 30 pids of one seat.
-__device__ __forceinline__ uint32_t seat_bits(uint64_t lo, uint64_t hi, int base)
-{
-    const uint64_t w = base == 0 ? lo : base < 64 ? ((lo >> base) | (hi << (64 - base))) : (hi >> (base - 64));
-    return (uint32_t)w & 0x3FFFFFFFu;
-}
-
 // World flat cell -> canonical flat cell of observer s (rotation.py:44-85).
 __device__ __forceinline__ int canon_cell(int s, int f)
 {
