@@ -241,11 +241,15 @@ __device__ __forceinline__ BB straight_moves_half(const MoveRec &M, bool enginee
     return m;
 }
 
-// Rail destinations of up to three engineers at once (move_gen.py:870-895): the
-// landable rail nodes adjacent to the closure of engineer j's source (rail
-// index sr[j]) through empty rail nodes, OR-ed into the wave's LDS words
+// Rail destinations of up to three engineers (move_gen.py:870-895): the
+// landable rail nodes adjacent to the closure of engineer j's source (rail index
+// sr[j]) through empty rail nodes, OR-ed into the wave's LDS words
 // dst[3j .. 3j + 2] (compact cells; zero on entry). Lane v evaluates rail nodes
-// v and v + 64 each hop; an engineer whose closure stopped growing is skipped.
+// v and v + 64. A closure is its source and the connected regions of empty nodes
+// next to it; a region is grown hop by hop (two ballots) from one node, and the
+// largest one is kept for the next engineers, who mostly stand next to the same
+// one. 8,192 positions with three engineers a seat: 39.4 -> 32.8 us for the legal
+// sets, against one closure grown per engineer.
 __device__ __forceinline__ void engineers_bb(int ne, const int sr[3], const BB &occ, const BB &ea, uint64_t *dst)
 {
     const int l = lane_id(), v1 = l + 64;
@@ -255,31 +259,34 @@ __device__ __forceinline__ void engineers_bb(int ne, const int sr[3], const BB &
     const bool l0 = e0 || bb_has(ea, c0), l1 = has1 && (e1 || bb_has(ea, c1));   // landable (empty or attackable)
     const uint64_t a0 = cT.rnbr[l][0], a1 = cT.rnbr[l][1];
     const uint64_t b0 = has1 ? cT.rnbr[v1][0] : 0ull, b1 = has1 ? cT.rnbr[v1][1] : 0ull;
-    uint64_t r0[3], r1[3];
-    bool grow[3];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        grow[j] = j < ne;
-        r0[j] = j < ne && sr[j] < 64 ? 1ull << sr[j] : 0ull;
-        r1[j] = j < ne && sr[j] >= 64 ? 1ull << (sr[j] - 64) : 0ull;
-    }
-    for (int hop = 0; hop < NRAIL && (grow[0] || grow[1] || grow[2]); ++hop) {
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            if (!grow[j]) continue;
-            const uint64_t g0 = __ballot(e0 && ((a0 & r0[j]) | (a1 & r1[j])) != 0);
-            const uint64_t g1 = __ballot(e1 && ((b0 & r0[j]) | (b1 & r1[j])) != 0) & 0x1FFull;
-            grow[j] = ((g0 & ~r0[j]) | (g1 & ~r1[j])) != 0;
-            r0[j] |= g0;
-            r1[j] |= g1;
-        }
-    }
+    uint64_t k0 = 0, k1 = 0;   // the largest region so far
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
         if (j >= ne) break;
-        if (l != sr[j] && l0 && ((a0 & r0[j]) | (a1 & r1[j])) != 0)
+        uint64_t r0 = sr[j] < 64 ? 1ull << sr[j] : 0ull, r1 = sr[j] >= 64 ? 1ull << (sr[j] - 64) : 0ull;
+        // empty neighbours of the source whose region is not in the closure yet
+        uint64_t t0 = __ballot(e0 && ((a0 & r0) | (a1 & r1)) != 0);
+        uint64_t t1 = __ballot(e1 && ((b0 & r0) | (b1 & r1)) != 0);
+        if ((t0 & k0) | (t1 & k1)) {
+            r0 |= k0; r1 |= k1;
+            t0 &= ~k0; t1 &= ~k1;
+        }
+        while (t0 | t1) {   // at most four rounds: each takes at least its own node out
+            uint64_t q0 = t0 ? t0 & (0 - t0) : 0ull, q1 = t0 ? 0ull : t1 & (0 - t1);
+            for (int hop = 0; hop < NRAIL; ++hop) {
+                const uint64_t g0 = __ballot(e0 && ((a0 & q0) | (a1 & q1)) != 0);
+                const uint64_t g1 = __ballot(e1 && ((b0 & q0) | (b1 & q1)) != 0);
+                if (!((g0 & ~q0) | (g1 & ~q1))) break;
+                q0 |= g0;
+                q1 |= g1;
+            }
+            r0 |= q0; r1 |= q1;
+            t0 &= ~q0; t1 &= ~q1;
+            if (__popcll(q0) + __popcll(q1) > __popcll(k0) + __popcll(k1)) { k0 = q0; k1 = q1; }
+        }
+        if (l != sr[j] && l0 && ((a0 & r0) | (a1 & r1)) != 0)
             atomicOr(reinterpret_cast<unsigned long long *>(&dst[3 * j + (c0 >> 6)]), 1ull << (c0 & 63));
-        if (has1 && v1 != sr[j] && l1 && ((b0 & r0[j]) | (b1 & r1[j])) != 0)
+        if (has1 && v1 != sr[j] && l1 && ((b0 & r0) | (b1 & r1)) != 0)
             atomicOr(reinterpret_cast<unsigned long long *>(&dst[3 * j + (c1 >> 6)]), 1ull << (c1 & 63));
     }
 }
@@ -1067,8 +1074,8 @@ __global__ __launch_bounds__(64) void k_finalize(State S, int beliefs, const uin
 // closures, counts, the packed canonical mask and the CSR scratch in ascending
 // source order (move_gen.py:1199 sorts the ids).
 // Legal sets of env `env` for `seat` by its wave (off: none): the board in LDS
-// (cell, padded to CELL_STRIDE with -1), bits cleared and, for the canonical
-// mask, rotl filled. src / t: cell and type of piece l & 31 of the seat (lanes p
+// (cell, padded to CELL_STRIDE with -1) and, for the canonical mask, bits
+// cleared; rotl is filled here. src / t: cell and type of piece l & 31 of the seat (lanes p
 // and p + 32 share piece p < 30, one half of its moves each).
 // lscr: LSCR_WORDS words of the wave's LDS, the compact source cells of the
 // movable pieces (words 0-2) and the engineers' rail destinations (3-11).
@@ -1083,7 +1090,7 @@ __global__ __launch_bounds__(64) void k_finalize(State S, int beliefs, const uin
 // u8 32,768 games 738 -> 722, bf16 16,384 666 -> 658, state only 4,096 33.4 -> 32.1).
 template <bool REC = true>
 __device__ __forceinline__ void legal_body(const State &S, int env, int row, int l, int seat, bool off, const int8_t *cell, uint32_t *bits,
-                           const uint8_t *rotl, int src, int t, uint64_t *lscr,
+                           uint8_t *rotl, int src, int t, uint64_t *lscr,
                            int32_t *__restrict__ counts, int32_t *__restrict__ mask_words, uint8_t *__restrict__ mask_bool)
 {
     const int team = seat & 1;
@@ -1092,6 +1099,8 @@ __device__ __forceinline__ void legal_body(const State &S, int env, int row, int
     const int h = l >> 5, p = l & 31;
     const bool own = !off && p < 30 && (unsigned)src < (unsigned)NC;
     const MoveRec M = cM.rec[own ? src : 0][h];   // cell 0 is off the board: an empty record
+    const uint8_t *rot = cT.rotc[seat & 3];   // world compact -> canonical compact of the seat
+    const uint8_t q0 = rot[l], q1 = rot[l + 64], q2 = rot[NONB - 1];
     if (l < 3) srcset[l] = 0;
     Boards B;
     env_boards(cell, team, T, B);
@@ -1136,6 +1145,7 @@ __device__ __forceinline__ void legal_body(const State &S, int env, int row, int
     // rank of this piece's source cell among the movable pieces: the movable
     // sources below it in a 129-bit set (compact order is flat order)
     if (lead) atomicOr(reinterpret_cast<unsigned long long *>(&srcset[sc >> 6]), 1ull << (sc & 63));
+    rotl[l] = q0; rotl[l + 64] = q1; rotl[NONB - 1] = q2;
     wave_sync();
     int rank = 0;
     if (lead) {
@@ -1234,10 +1244,6 @@ __device__ __forceinline__ void legal_row(const State &S, int row, int l, LegalL
     __builtin_amdgcn_s_setprio(2);
     for (int w = l; w < JQ_MASK_WORDS_PAD; w += 64) L.bits[w] = 0;
     board_stage(L.cell, l, c0, c1);
-    if (mask_words || mask_bool) {
-        const int s4 = seat & 3;
-        for (int c = l; c < NONB; c += 64) L.rotl[c] = cT.rotc[s4][c];
-    }
     wave_sync();
     legal_body<!HIST>(S, env, row, l, seat, off, L.cell, L.bits, L.rotl, src, t, L.lscr, counts, mask_words, mask_bool);
 }
@@ -1766,10 +1772,8 @@ __device__ __forceinline__ void env_step_wave(const State &S, int env, int l, co
     }
     const int seat = nx.turn;
     const bool off = nx.term || seat < 0 || seat > 3 || ((nx.sdead >> (seat & 3)) & 1);
-    if (A.mask_words) {
+    if (A.mask_words)
         for (int w = l; w < JQ_MASK_WORDS_PAD; w += 64) E.bits[w] = 0;
-        for (int c = l; c < NONB; c += 64) E.rotl[c] = cT.rotc[seat & 3][c];
-    }
     wave_sync();
     const int mine = !off && (l & 31) < 30 ? seat * 30 + (l & 31) : -1;   // the next seat's piece of this lane
     legal_body(S, env, env, l, seat, off, E.cell, E.bits, E.rotl, mine >= 0 ? E.pos[mine] : -1,
