@@ -383,7 +383,8 @@ bool obs_persists(const jq_env *e) { return e->S.n > 20 * g_dev[e->device].obs_b
 // one block per row from there on: bf16 2,048 rows in 1 / 2 / 3 parts
 // 82 / 98 / 113). f32 rows are long enough to stay split: fewer bytes then
 // stream at once and reach memory in better order (8,192 rows in 1 / 2 / 3 / 4
-// parts 598 / 594 / 531 / 590).
+// parts 598 / 594 / 531 / 590; 32,768 rows 2,310 / 2,322 / 2,149 / 2,287, in 6
+// and 8 parts 2,707 and 3,220).
 //
 // Streaming stores leave the caches as they are written, which wins once the
 // output does not fit the 256 MB memory-side cache anyway (4,096 u8 rows 89 ->

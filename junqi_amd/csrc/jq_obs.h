@@ -823,7 +823,7 @@ __device__ __forceinline__ void obs_emit_u8(const ObsLds &L, uint8_t *row, int m
 // the whole 36 KB row into a scratch state, observed from there, took 69 us
 // more at 4,096 bf16 rows.
 //
-// `parts` 512-thread blocks per row (obs_launch chooses): each builds the row in
+// `parts` 512-thread blocks per row (obs_plan chooses): each builds the row in
 // its LDS and streams one of `parts` equal runs of its 1 KB units. Bound: HBM
 // writes once the grid fills the chip; below that, one block's time for its
 // loads, fill and run, which is why few rows are split over many blocks (24 f32
