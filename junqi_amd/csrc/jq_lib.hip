@@ -381,7 +381,8 @@ bool obs_persists(const jq_env *e) { return e->S.n > 20 * g_dev[e->device].obs_b
 // 28.8 -> 25.4; u8 64 rows 11.5 -> 10.0, 512 rows 15.7 -> 14.8. Past that the
 // repeated loads and fill cost more than the shorter runs give (u8 and bf16,
 // one block per row from there on: bf16 2,048 rows in 1 / 2 / 3 parts
-// 82 / 98 / 113). f32 rows are long enough to stay split: fewer bytes then
+// 82 / 98 / 113, 16,384 rows in 1 / 2 / 3 548 / 674 / 813; u8 16,384 rows
+// 288 / 340 / 434). f32 rows are long enough to stay split: fewer bytes then
 // stream at once and reach memory in better order (8,192 rows in 1 / 2 / 3 / 4
 // parts 598 / 594 / 531 / 590; 32,768 rows 2,310 / 2,322 / 2,149 / 2,287, in 6
 // and 8 parts 2,707 and 3,220).
