@@ -256,14 +256,18 @@ class JunqiBatch:
         return out
 
     def legal_dense_numpy(self, acting: np.ndarray | None, width: int) -> tuple[np.ndarray, np.ndarray]:
-        """(ids (N, width) int32, counts (N,) int32) on the host for host int8
-        seats (None: the current turn); ids ascending, cut at width, -1 padded."""
-        s = None if acting is None else torch.from_numpy(acting).contiguous()
+        """(ids (N, width) int32, counts (N,) int32) on the host for host seats
+        (N,) (None: the current turn); ids ascending, cut at width, -1 padded."""
+        seats = None
+        if acting is not None:   # the library copies n bytes of it
+            if np.shape(acting) != (self.n,):
+                raise ValueError(f"acting: expected ({self.n},), got {np.shape(acting)}")
+            seats = np.ascontiguousarray(acting, dtype=np.int8)
         ids = np.empty((self.n, width), np.int32)
         counts = np.empty(self.n, np.int32)
-        check(lib.jq_legal_dense_host(self._h, self._ptr(s), self.counts.data_ptr(), self.offsets.data_ptr(),
-                                      self.values.data_ptr(), self.values.numel(), width, ids.ctypes.data,
-                                      counts.ctypes.data, self.stream))
+        check(lib.jq_legal_dense_host(self._h, None if seats is None else seats.ctypes.data, self.counts.data_ptr(),
+                                      self.offsets.data_ptr(), self.values.data_ptr(), self.values.numel(), width,
+                                      ids.ctypes.data, counts.ctypes.data, self.stream))
         return ids, counts
 
     def step_numpy(self, action_ids: np.ndarray) -> dict[str, np.ndarray]:

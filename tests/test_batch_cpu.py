@@ -1,0 +1,68 @@
+"""What the Python layer hands to the library, without a GPU: a JunqiBatch whose
+library calls are recorded instead of run."""
+
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from junqi_amd import _lib as jl  # noqa: E402
+from junqi_amd import batch as jb  # noqa: E402
+
+
+class _Recorder:
+    """Stands for the library: every call succeeds and is kept with its arguments;
+    `seats` are the int8 values behind a seat pointer at the time of the call."""
+
+    def __init__(self, n, seat_arg):
+        self.n, self.seat_arg, self.calls = n, seat_arg, []
+
+    def __getattr__(self, name):
+        def call(*args):
+            ptr = args[self.seat_arg.get(name, 0)] if name in self.seat_arg else None
+            seats = None if ptr is None else np.frombuffer(C.string_at(ptr, self.n), np.int8).copy()
+            self.calls.append((name, seats))
+            return 0
+        return call
+
+
+class _HostBatch(jb.JunqiBatch):
+    stream = 0
+
+    def __init__(self, n):
+        self.n, self.device, self._h = n, torch.device("cpu"), None
+        self.counts = torch.zeros(n, dtype=torch.int32)
+        self.offsets = torch.zeros(n + 1, dtype=torch.int32)
+        self.values = torch.zeros(n * jl.MAX_LEGAL, dtype=torch.int32)
+        self._turn_view = torch.zeros(n, dtype=torch.int8)
+
+
+@pytest.fixture
+def recorded(monkeypatch):
+    n = 6
+    rec = _Recorder(n, {"jq_legal_dense_host": 1})
+    monkeypatch.setattr(jb, "lib", rec)
+    return _HostBatch(n), rec
+
+
+@pytest.mark.parametrize("seats", [
+    np.array([0, 1, 2, 3, 0, 1], np.int64), np.array([0, 1, 2, 3, 0, 1], np.int32),
+    np.arange(12, dtype=np.int8)[::2] % 4, [3, 2, 1, 0, 3, 2],
+], ids=["int64", "int32", "strided", "list"])
+def test_dense_legal_seats_are_read_by_value(recorded, seats):
+    b, rec = recorded
+    b.legal_dense_numpy(seats, 8)
+    (name, got), = rec.calls
+    assert name == "jq_legal_dense_host" and np.array_equal(got, np.asarray(seats).astype(np.int8))
+
+
+@pytest.mark.parametrize("shape", [(0,), (5,), (7,), (6, 1), (1, 6), ()])
+def test_dense_legal_refuses_other_shapes(recorded, shape):
+    b, rec = recorded
+    with pytest.raises(ValueError, match="acting"):
+        b.legal_dense_numpy(np.zeros(shape, np.int8), 8)
+    assert not rec.calls
