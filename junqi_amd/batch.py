@@ -148,6 +148,7 @@ class JunqiBatch:
 
     # ------------------------------------------------------------ lifetime
     def close(self) -> None:
+        self._turn_view = None   # it looks into the library's memory
         if getattr(self, "_h", None):
             lib.jq_destroy(self._h)
             self._h = None
@@ -169,7 +170,8 @@ class JunqiBatch:
         if t is None:
             return None
         v = self._turn_view
-        if t.dtype is torch.int8 and t.data_ptr() == v.data_ptr() and t.shape == v.shape and t.stride() == v.stride():
+        if (v is not None and t.dtype is torch.int8 and t.data_ptr() == v.data_ptr() and t.shape == v.shape
+                and t.stride() == v.stride()):
             return None
         return t.to(device=self.device, dtype=torch.int8).contiguous()
 

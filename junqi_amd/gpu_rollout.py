@@ -271,7 +271,8 @@ class GpuRollout:
 
     def turn_torch(self) -> torch.Tensor:
         """Zero-copy int8 (N,) view of the acting seats (gpu_rollout.py:1159-1169)."""
-        return self._b._turn_view.detach()
+        v = self._b._turn_view
+        return self._b.field_tensor("turn") if v is None else v.detach()   # raises once closed, like the other views
 
     def terminated_torch(self) -> torch.Tensor:
         return self._b.field_tensor("terminated", torch.bool)

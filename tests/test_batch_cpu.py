@@ -66,3 +66,19 @@ def test_dense_legal_refuses_other_shapes(recorded, shape):
     with pytest.raises(ValueError, match="acting"):
         b.legal_dense_numpy(np.zeros(shape, np.int8), 8)
     assert not rec.calls
+
+
+def test_a_closed_batch_hands_out_no_view():
+    from junqi_amd.gpu_rollout import GpuRollout
+
+    r = GpuRollout.__new__(GpuRollout)
+    r._b = b = _HostBatch(6)
+    live = r.turn_torch()
+    assert b._seats(live) is None, "the live view stands for the current turn"
+    r.close()
+    for view in (r.turn_torch, r.terminated_torch, r.winner_team_torch, r.draw_torch):
+        with pytest.raises(jl.ArgumentError):
+            view()
+    assert b._seats(live) is not None, "the view of a closed batch is not the current turn"
+    with pytest.raises(jl.JunqiError):
+        b.legal_slots(torch.zeros(6, dtype=torch.int8), out=torch.empty((6, 120, 80), dtype=torch.bool))
