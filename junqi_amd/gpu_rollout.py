@@ -157,6 +157,8 @@ class GpuRollout:
         """Compact canonical ids (src_c*129 + dst_c in the acting seat's frame) →
         device dict terminated / rewards / event / draw / winner_team
         (gpu_rollout.py:780-848). Move history and beliefs are updated here."""
+        if acting_seats is None:
+            raise ValueError("canonical actions need the acting seats")
         b, o = self._b, self._step_out
         a = canonical_actions.to(device=self.device, dtype=torch.int32).contiguous()
         s = b._seats(acting_seats)
@@ -218,6 +220,8 @@ class GpuRollout:
     def build_acting_seat_observation_torch(self, acting_seats_t: torch.Tensor):
         """(N,317,17,17) f32 and (N,28) f32 device views for one observer per env
         (gpu_rollout.py:927-964)."""
+        if acting_seats_t is None:
+            raise ValueError("an acting-seat observation needs the acting seats")
         if self._sp1 is None:
             self._sp1 = torch.empty((self.num_envs, OBS_CHANNELS, 17, 17), dtype=torch.float32, device=self.device)
             self._gl1 = torch.empty((self.num_envs, L.OBS_GLOBALS), dtype=torch.float32, device=self.device)

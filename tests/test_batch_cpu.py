@@ -82,3 +82,23 @@ def test_a_closed_batch_hands_out_no_view():
     assert b._seats(live) is not None, "the view of a closed batch is not the current turn"
     with pytest.raises(jl.JunqiError):
         b.legal_slots(torch.zeros(6, dtype=torch.int8), out=torch.empty((6, 120, 80), dtype=torch.bool))
+
+
+@pytest.mark.parametrize("call", ["step_device_torch", "build_acting_seat_observation_torch"])
+def test_collector_calls_need_their_seats(recorded, monkeypatch, call):
+    from junqi_amd.gpu_rollout import GpuRollout
+
+    b, rec = recorded
+    monkeypatch.setattr(jl, "lib", rec)
+    r = GpuRollout.__new__(GpuRollout)
+    r._b, r.device, r.num_envs = b, b.device, b.n
+    r._step_out = {k: torch.zeros(b.n) for k in ("event", "terminated", "winner_team", "draw", "rewards")}
+    r._sp1 = torch.zeros((b.n, 317, 17, 17))
+    r._gl1 = torch.zeros((b.n, 28))
+    seats = torch.zeros(b.n, dtype=torch.int8)
+    args = (torch.zeros(b.n, dtype=torch.int32),) if call == "step_device_torch" else ()
+    getattr(r, call)(*args, seats)
+    assert len(rec.calls) == 1
+    with pytest.raises((ValueError, AttributeError)):
+        getattr(r, call)(*args, None)
+    assert len(rec.calls) == 1
