@@ -163,12 +163,17 @@ class JunqiBatch:
     def stream(self) -> int:
         return torch.cuda.current_stream(self.device).cuda_stream
 
-    def _seats(self, t: torch.Tensor | None) -> torch.Tensor | None:
+    def _seats(self, t: torch.Tensor | None, per_env: int = 1) -> torch.Tensor | None:
         """Seats as the library takes them: contiguous int8 on this device, or
         None (the current turn) for the live turn view itself, which the kernels
-        then read in the env records instead of through a copy of them."""
+        then read in the env records instead of through a copy of them. The
+        kernels read n * per_env of them."""
         if t is None:
             return None
+        if t.numel() < self.n * per_env:
+            raise ValueError(f"expected {self.n * per_env} seats, got {t.numel()}")
+        if per_env != 1:
+            return t.to(device=self.device, dtype=torch.int8).contiguous()
         v = self._turn_view
         if (v is not None and t.dtype is torch.int8 and t.data_ptr() == v.data_ptr() and t.shape == v.shape
                 and t.stride() == v.stride()):
@@ -305,10 +310,7 @@ class JunqiBatch:
             out_aux = torch.empty(lead + (L.AUX_BYTES,), dtype=torch.uint8, device=self.device)
         if tuple(out_spatial.shape) != lead + (L.OBS_CHANNELS, 17, 17) or out_spatial.dtype != dt:
             raise ValueError("out_spatial has the wrong shape or dtype")
-        if all_seats:
-            s = None if observer is None else observer.to(device=self.device, dtype=torch.int8).contiguous()
-        else:
-            s = self._seats(observer)
+        s = self._seats(observer, 4 if all_seats else 1)
         check(lib.jq_observe(self._h, self._ptr(s), code, 1 if all_seats else 0, out_spatial.data_ptr(),
                              self._ptr(out_aux) if fmt == "u8" else None, out_global.data_ptr(), self.stream))
         if fmt == "u8":

@@ -38,6 +38,7 @@ class _HostBatch(jb.JunqiBatch):
         self.counts = torch.zeros(n, dtype=torch.int32)
         self.offsets = torch.zeros(n + 1, dtype=torch.int32)
         self.values = torch.zeros(n * jl.MAX_LEGAL, dtype=torch.int32)
+        self.mask_words = torch.zeros((n, jl.MASK_WORDS), dtype=torch.int32)
         self._turn_view = torch.zeros(n, dtype=torch.int8)
 
 
@@ -102,3 +103,26 @@ def test_collector_calls_need_their_seats(recorded, monkeypatch, call):
     with pytest.raises((ValueError, AttributeError)):
         getattr(r, call)(*args, None)
     assert len(rec.calls) == 1
+
+
+def test_short_device_seats_are_refused(recorded):
+    """The kernels read n seats (4n for all-seat observations)."""
+    b, rec = recorded
+    n = b.n
+    seat_calls = {
+        "legal": lambda s: b.legal(s), "legal_slots": lambda s: b.legal_slots(s, out=torch.empty((n, 120, 80), dtype=torch.bool)),
+        "sample_logits": lambda s: b.sample_logits(1, 2, acting=s), "observe": lambda s: b.observe(s, fmt="u8"),
+    }
+    for name, call in seat_calls.items():
+        for ok in (torch.zeros(n, dtype=torch.int64), torch.zeros((n, 1), dtype=torch.int8), torch.zeros(n + 3, dtype=torch.int8)):
+            call(ok)
+        done = len(rec.calls)
+        for short in (torch.zeros(0, dtype=torch.int8), torch.zeros(n - 1, dtype=torch.int8)):
+            with pytest.raises(ValueError, match="seats"):
+                call(short)
+        assert len(rec.calls) == done, name
+    b.observe(torch.zeros((n, 4), dtype=torch.int8), fmt="u8", all_seats=True)
+    done = len(rec.calls)
+    with pytest.raises(ValueError, match="seats"):
+        b.observe(torch.zeros(n, dtype=torch.int8), fmt="u8", all_seats=True)
+    assert len(rec.calls) == done
