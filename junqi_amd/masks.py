@@ -36,8 +36,6 @@ def dense_mask_to_csr(mask: torch.Tensor, out_ids: torch.Tensor, out_counts: tor
     mask = mask.contiguous()
     if not out_ids.is_contiguous() or not out_counts.is_contiguous():
         raise ValueError("CSR outputs must be contiguous")
-    if n == 0:
-        return
     # the rows are encoded into scratch and published on the device if they all
     # fit; only the largest count comes back, through pinned host memory
     rows = (n * k_max + 3) // 4 * 4

@@ -116,3 +116,11 @@ def test_encode_row_shapes(masks, d, n, k_max, shift):
         with pytest.raises(ValueError, match=f"need {d} entries"):
             masks.dense_mask_to_csr(torch.from_numpy(m).cuda().view(torch.bool), ids, counts)
         assert torch.equal(store, before) and np.array_equal(counts.cpu().numpy(), want_counts)
+
+
+def test_encode_of_no_rows_is_refused(masks):
+    for d in (0, 16641):
+        mask = torch.empty((0, d), dtype=torch.bool, device="cuda")
+        with pytest.raises(ValueError):
+            masks.dense_mask_to_csr(mask, torch.empty((0, 8), dtype=torch.int32, device="cuda"),
+                                    torch.empty(0, dtype=torch.int32, device="cuda"))
