@@ -1,6 +1,7 @@
 """Legal-support storage of rollout buffers: dense bool mask rows <-> per-row id
 lists (junqi_rl/training/rollout_gpu.py:119-198), on the device through the
-jq_mask_encode / jq_ids_to_mask kernels.
+jq_mask_encode / jq_ids_to_mask kernels (jq_mask_count and jq_mask_to_ids where
+memory is short).
 
 Same arguments, shapes, dtypes and ValueError checks as the reference's
 ``_dense_mask_to_csr`` and ``_csr_to_dense_selected``; tensors must be on the
@@ -36,16 +37,28 @@ def dense_mask_to_csr(mask: torch.Tensor, out_ids: torch.Tensor, out_counts: tor
     mask = mask.contiguous()
     if not out_ids.is_contiguous() or not out_counts.is_contiguous():
         raise ValueError("CSR outputs must be contiguous")
+    s, d = _stream(mask), int(mask.shape[1])
     # the rows are encoded into scratch and published on the device if they all
     # fit; only the largest count comes back, through pinned host memory
     rows = (n * k_max + 3) // 4 * 4
-    work = torch.empty(rows + n, dtype=torch.int32, device=mask.device)
+    try:
+        work = torch.empty(rows + n, dtype=torch.int32, device=mask.device)
+    except torch.OutOfMemoryError:   # no room for a second copy of the ids: count, test, then write them in place
+        counts = torch.empty(n, dtype=torch.int32, device=mask.device)
+        check(lib.jq_mask_count(mask.data_ptr(), n, d, counts.data_ptr(), s))
+        _fits(int(counts.max()), k_max)   # synchronises
+        out_counts.copy_(counts)
+        check(lib.jq_mask_to_ids(mask.data_ptr(), n, d, k_max, out_ids.data_ptr(), s))
+        return
     most = torch.empty(1, dtype=torch.int32, pin_memory=True)   # written by the kernel itself
     p = work.data_ptr()
-    check(lib.jq_mask_encode(mask.data_ptr(), n, int(mask.shape[1]), k_max, p, p + 4 * rows, out_ids.data_ptr(),
-                             out_counts.data_ptr(), most.data_ptr(), _stream(mask)))
+    check(lib.jq_mask_encode(mask.data_ptr(), n, d, k_max, p, p + 4 * rows, out_ids.data_ptr(),
+                             out_counts.data_ptr(), most.data_ptr(), s))
     torch.cuda.current_stream(mask.device).synchronize()   # like the reference's guard
-    required = int(most)
+    _fits(int(most), k_max)
+
+
+def _fits(required: int, k_max: int) -> None:
     if required > k_max:
         raise ValueError(
             f"CSR legal-mask overflow: need {required} entries, capacity {k_max}; "

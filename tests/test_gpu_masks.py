@@ -118,6 +118,39 @@ def test_encode_row_shapes(masks, d, n, k_max, shift):
         assert torch.equal(store, before) and np.array_equal(counts.cpu().numpy(), want_counts)
 
 
+def test_encode_without_room_for_its_scratch(masks):
+    """With less device memory left than the encoded rows take, the encode still
+    runs (counting first), and an overflow still leaves the outputs as they were."""
+    rng = np.random.default_rng(5)
+    n, k = 1500, 4096                                   # 24 MB of ids
+    m = np.zeros((n, 8192), bool)
+    for r in range(n):
+        m[r, rng.choice(8192, int(rng.integers(0, 40)), replace=False)] = True
+    m[7] = np.arange(8192) < k
+    want_ids, want_counts = _np_csr(m, k)
+    dm = torch.from_numpy(m).cuda()
+    ids = torch.full((n, k), -7, dtype=torch.int32, device="cuda")
+    counts = torch.full((n,), -7, dtype=torch.int32, device="cuda")
+    over = dm.clone()
+    over[9] = torch.arange(8192, device="cuda") <= k
+    small = torch.empty(4096, dtype=torch.int32, device="cuda")   # keeps a block of small allocations around
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (8 << 20)) / total)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(n * k, dtype=torch.int32, device="cuda")
+        with pytest.raises(ValueError, match=f"need {k + 1} entries"):
+            masks.dense_mask_to_csr(over, ids, counts)
+        assert (ids.cpu() == -7).all() and (counts.cpu() == -7).all()
+        masks.dense_mask_to_csr(dm, ids, counts)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    del small
+    assert np.array_equal(counts.cpu().numpy(), want_counts) and np.array_equal(ids.cpu().numpy(), want_ids)
+
+
 def test_encode_of_no_rows_is_refused(masks):
     for d in (0, 16641):
         mask = torch.empty((0, d), dtype=torch.bool, device="cuda")
