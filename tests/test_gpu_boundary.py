@@ -9,6 +9,7 @@ from __future__ import annotations
 import ctypes
 import hashlib
 import json
+import re
 
 import numpy as np
 import pytest
@@ -164,59 +165,114 @@ def test_env_step_rejects_bad_observation_buffers_before_stepping(jq):
     b.close()
 
 
-def test_env_step_side_stream_csr(jq):
-    """jq_env_step with a u8 observation and a full-size values buffer runs the
-    CSR pass on a side stream beside the observation; with a smaller buffer it
-    runs in line (after the total is read back). Both must give the same rows,
-    masks, observations and step results, on a non-default caller stream whose
-    later work sees the joined results; the observation timing hooks count every
-    launch."""
-    print("[boundary] side-stream CSR pass", flush=True)
+def _kernels_of(call):
+    """Names of the library's kernels that one call launches, as the profiler sees
+    them (empty where it sees none)."""
+    from torch.profiler import ProfilerActivity, profile
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        call()
+        torch.cuda.synchronize()
+    return {m.group(1) for m in (re.match(r"(?:void )?jq::(k_\w+)", e.name) for e in p.events()) if m}
+
+
+def _env_step_routes(jq, n, steps, shift):
+    """jq_env_step with a u8 observation `steps` times on two batches from the same
+    seeds, one with a full-size values buffer (its CSR pass needs no total), the
+    other with a smaller one (scan, read-back of the total, emit, in line). Both
+    must give the same rows, masks, observations and step results, on a
+    non-default caller stream whose later work sees the joined results; the first
+    one's observation is timed in the first half of the steps, and its rows start
+    `shift` bytes off a 16-byte boundary. Yields after each step: the step, that
+    batch and its outputs (spatial, aux, globals, terminated, reward, hash, actions)."""
     from junqi_amd import _lib as L
-    n, steps = 3000, 24
-    side, inline = (jq.JunqiBatch(n, show_mode=2, pool_size=64) for _ in range(2))
-    for b in (side, inline):
+    full, inline = (jq.JunqiBatch(n, show_mode=2, pool_size=64) for _ in range(2))
+    for b in (full, inline):
         b.reset(31)
         b.legal()
-    dev = side.device
+    dev = full.device
     st = torch.cuda.Stream(dev)
-    mk = lambda: (torch.empty((n, 317, 17, 17), dtype=torch.uint8, device=dev),  # noqa: E731
-                  torch.empty((n, L.AUX_BYTES), dtype=torch.uint8, device=dev),
-                  torch.empty((n, 28), dtype=torch.float32, device=dev),
-                  torch.empty(n, dtype=torch.uint8, device=dev), torch.empty(n, dtype=torch.float32, device=dev),
-                  torch.empty(n, dtype=torch.int64, device=dev), torch.empty(n, dtype=torch.int32, device=dev))
-    outs = {"side": mk(), "inline": mk()}
-    caps = {"side": side.values.numel(), "inline": n * 200}
-    assert caps["inline"] < n * L.MAX_LEGAL <= caps["side"]
-    L.check(L.lib.jq_obs_timing(side._h, 1))
-    with torch.cuda.stream(st):
-        for k in range(steps):
-            snap = {}
-            for name, b in (("side", side), ("inline", inline)):
-                sp, aux, gl, te, rw, hs, ac = outs[name]
+
+    def buffers(off):
+        sp = torch.empty(n * 317 * 289 + 16, dtype=torch.uint8, device=dev)[off:off + n * 317 * 289]
+        return (sp.view(n, 317, 17, 17), torch.empty((n, L.AUX_BYTES), dtype=torch.uint8, device=dev),
+                torch.empty((n, 28), dtype=torch.float32, device=dev),
+                torch.empty(n, dtype=torch.uint8, device=dev), torch.empty(n, dtype=torch.float32, device=dev),
+                torch.empty(n, dtype=torch.int64, device=dev), torch.empty(n, dtype=torch.int32, device=dev))
+    cap = n * 200
+    runs = ((full, buffers(shift), full.values.numel()), (inline, buffers(0), cap))
+    assert cap < n * L.MAX_LEGAL <= runs[0][2]
+    torch.cuda.synchronize()   # the resets and fills above ran on the default stream
+    timed = steps // 2
+    L.check(L.lib.jq_obs_timing(full._h, 1))
+    for k in range(steps):
+        if k == timed:
+            total_ms, launches = ctypes.c_double(), ctypes.c_int64()
+            L.check(L.lib.jq_obs_timing_read(full._h, ctypes.byref(total_ms), ctypes.byref(launches)))
+            L.check(L.lib.jq_obs_timing(full._h, 0))
+            assert launches.value == timed and total_ms.value > 0.0
+        with torch.cuda.stream(st):
+            snap = []
+            for b, out, room in runs:
                 L.check(L.lib.jq_env_step(b._h, None, L.SAMPLE_LOGITS, 5, k, k, b.counts.data_ptr(),
-                                          b.offsets.data_ptr(), b.values.data_ptr(), caps[name],
-                                          b.mask_words.data_ptr(), L.OBS_U8, sp.data_ptr(), aux.data_ptr(),
-                                          gl.data_ptr(), te.data_ptr(), rw.data_ptr(), hs.data_ptr(), ac.data_ptr(),
-                                          st.cuda_stream))
+                                          b.offsets.data_ptr(), b.values.data_ptr(), room, b.mask_words.data_ptr(),
+                                          L.OBS_U8, *(t.data_ptr() for t in out), st.cuda_stream))
                 # read on the caller's stream right after the call
-                tot = b.offsets[-1].clone()
-                snap[name] = (b.counts.clone(), b.offsets.clone(), b.values[:n * 200].clone(), b.mask_words.clone(),
-                              tot, sp.clone(), aux.clone(), gl.clone(), te.clone(), rw.clone(), hs.clone(), ac.clone())
-            st.synchronize()
-            a, c = snap["side"], snap["inline"]
-            t = int(a[4])
-            assert t == int(c[4]) and t <= n * 200
-            for i, (x, y) in enumerate(zip(a, c)):
-                if i == 2:
-                    x, y = x[:t], y[:t]
+                snap.append((b.offsets[-1].clone(), b.values[:cap].clone(), b.counts, b.offsets, b.mask_words, *out))
+            tot = [int(s[0]) for s in snap]
+            assert tot[0] == tot[1] <= cap
+            for i, (x, y) in enumerate(zip(snap[0][1:], snap[1][1:])):
+                x, y = (x[:tot[0]], y[:tot[0]]) if i == 0 else (x, y)
                 assert torch.equal(x, y), f"step {k}: output {i} differs"
-    total_ms, launches = ctypes.c_double(), ctypes.c_int64()
-    L.check(L.lib.jq_obs_timing_read(side._h, ctypes.byref(total_ms), ctypes.byref(launches)))
-    L.check(L.lib.jq_obs_timing(side._h, 0))
-    assert launches.value == steps and total_ms.value > 0.0
-    side.close()
+        st.synchronize()
+        yield k, full, runs[0][1]
+    full.close()
     inline.close()
+
+
+def test_env_step_csr_in_the_observation_launch(jq):
+    """A batch too small for the persistent observation: the CSR pass rides in the
+    observation's launch, or scan and emit run before it."""
+    print("[boundary] CSR pass in the observation's launch", flush=True)
+    for _ in _env_step_routes(jq, 3000, 24, 0):
+        pass
+    b = jq.JunqiBatch(3000, show_mode=2, pool_size=64)
+    b.reset(31)
+    b.legal()
+    sp = torch.empty((b.n, 317, 17, 17), dtype=torch.uint8, device=b.device)
+    seen = _kernels_of(lambda: b.env_step(obs_fmt="u8", spatial=sp, glob=torch.empty((b.n, 28), device=b.device)))
+    assert not seen or seen == {"k_env_step", "k_observe"}, seen
+    b.close()
+
+
+def test_env_step_side_stream_csr(jq):
+    """Just past the persistent observation's threshold (20 rows per block the
+    device holds at once, 4 blocks per CU): the CSR pass and the mask run on the
+    library's side stream beside it. The row count leaves the last grid round to
+    three blocks; games of the first and last rounds are played along in the
+    oracle."""
+    from junqi_amd import _lib as L
+    grid = 4 * torch.cuda.get_device_properties(0).multi_processor_count
+    n = 20 * grid + 3
+    print(f"[boundary] side-stream CSR pass n={n}", flush=True)
+    rows = [0, 1, 2, grid - 1, grid, grid + 1, n // 2, n - grid - 1, n - grid, n - 5, n - 4, n - 3, n - 2, n - 1]
+    games = G.oracle_games_from_lineups(jq.generate_lineups(31, n)[rows], 2)
+    tables = O.tables()
+    for k, b, (sp, aux, gl, _, _, hsh, acts) in _env_step_routes(jq, n, 6, 5):
+        sel = torch.as_tensor(rows, device=b.device)
+        u8, ax, g28, mw, a, h = (t[sel].cpu().numpy() for t in (sp, aux, gl, b.mask_words, acts, hsh))
+        offs, vals = b.offsets.cpu().numpy(), b.values.cpu().numpy()
+        for j, (i, g) in enumerate(zip(rows, games)):
+            assert g.step_id(int(a[j]))[0] == 0
+            assert int(h[j]) & (2**64 - 1) == int(g.zobrist), (k, i)
+            ids = g.legal_ids()
+            assert np.array_equal(vals[offs[i]:offs[i + 1]], ids), (k, i)
+            assert np.array_equal(mw[j], G.canonical_mask_words(ids, int(g.turn), tables)), (k, i)
+            osp, ogl = g.observe(int(g.turn))
+            assert np.array_equal(jq.decode_u8(u8[j], ax[j]).view(np.uint32), osp.view(np.uint32)), (k, i)
+            assert np.array_equal(g28[j], ogl), (k, i)
+        if k == 5:
+            seen = _kernels_of(lambda: b.env_step(obs_fmt="u8", spatial=sp, aux=aux, glob=gl))
+            assert not seen or seen == {"k_env_step", "k_scan", "k_emit", "k_observe_u8_persist"}, seen
 
 
 def test_multi_tile_scan(jq):
