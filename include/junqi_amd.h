@@ -139,7 +139,8 @@ int jq_move_tables(void *host_out, int64_t nbytes);
 int jq_reset_terminated(jq_env *env, int64_t seed, void *stream);
 
 /* Apply one ply per env. actions: device int32 (N) in `action_format`; acting:
- * device int8 (N) seat per env (NULL = current turn; required for canonical ids).
+ * device int8 (N) seat per env (NULL = current turn), in whose frame canonical
+ * ids are read.
  * Outputs (device, any may be NULL): valid u8, event i8, terminated u8, winner i8,
  * draw u8, flag_captured u8, seats_died u8 bitmask, reward f32 (acting team +-1 on
  * the ply that ends the game), world_action i32.

@@ -86,11 +86,9 @@ __device__ __forceinline__ EnvRec env_record(const State &S, int env)
     __builtin_memcpy(&E, v, sizeof E);
     return E;
 }
-__device__ __forceinline__ bool is_on(int f) { return cflags(f) & CF_ON; }
 __device__ __forceinline__ bool is_rail(int f) { return cflags(f) & CF_RAIL; }
 __device__ __forceinline__ bool is_camp(int f) { return cflags(f) & CF_CAMP; }
 __device__ __forceinline__ bool is_sh(int f) { return cflags(f) & CF_SH; }
-__device__ __forceinline__ int curve_of(int f) { return cflags(f) >> 8; }
 __device__ __forceinline__ int team_of(int pid) { return (pid / 30) & 1; }
 
 // Bits [base, base + 30) of the 120-bit pid set (hi:lo), i.e. the 30 pids of one seat.
@@ -1451,7 +1449,7 @@ __global__ __launch_bounds__(64) void k_emit(State S, const int32_t *__restrict_
 // ids, one env per wave and pass. For batches whose ids always fit the buffer
 // (no total to read back).
 // Why: k_scan is one block, 6.2 us however few the envs, and k_emit waits for
-// it. The blocks read the counts again and again (n * n / (8 * passes) words in
+// it. The blocks read the counts again and again (n * n / (16 * passes) words in
 // all, from L2), so larger batches take more envs per block.
 constexpr int CSR_THREADS = 512, CSR_WAVES = CSR_THREADS / 64, CSR_MOST_PASSES = 4;
 struct CsrArgs {

@@ -336,7 +336,11 @@ int host_io_room(HostIo &io, size_t pinned, size_t dev)
 
 // `bytes` of caller input as kernels on `s` can read them: the pinned copy
 // itself while it is small (a kernel's few reads of it cost less than a copy's
-// launch), else a device copy at `dev`.
+// launch), else a device copy at `dev`. us of jq_step_host's whole call, copied /
+// read in place (4 bytes a game): 64 games 26.2 / 24.7, 1,024 26.3 / 24.9, 4,096
+// 34.3 / 34.3, 8,192 40.8 / 38.7, 16,384 47.4 / 53.0, 65,536 83 / 125; a game's
+// one byte of seats makes no difference at any of these (legal_dense_host at
+// 256 games 47.4 / 46.9, at 65,536 6,279 / 6,306).
 constexpr size_t HOST_READ_MAX = 16384;
 int host_input(HostIo &io, const void *host, size_t bytes, size_t pin_off, size_t dev_off, hipStream_t s,
                const uint8_t *&out)
@@ -368,7 +372,12 @@ int launch_check(const char *what)
 // loads, which come from memory after a step's gigabytes of stores, and its tail
 // takes the CSR pass. Below that k_observe, with the CSR pass in its launch, is
 // faster (us per fused u8 step, persistent / k_observe: 4,096 games 118 / 105,
-// 8,192 208 / 189, 16,384 379 / 369, 24,000 517 / 537, 32,768 712 / 735).
+// 8,192 208 / 189, 16,384 379 / 369, 24,000 517 / 537, 32,768 712 / 735). Rows
+// of all four seats never take it: k_observe is faster for them at any size (us
+// per observation alone, persistent / k_observe: 20,484 rows 400 / 374, 24,000
+// 465 / 436, 32,768 633 / 592, 65,536 1,278 / 1,076). One seat's rows observed
+// alone would gain too (20,481 402 / 362, 32,768 614 / 584, 50,000 967 / 947);
+// they follow the fused step, which is where such batches are observed.
 bool obs_persists(const jq_env *e) { return e->S.n > 20 * g_dev[e->device].obs_blocks; }
 
 // How k_observe runs `nrows` rows of format `fmt` on a device with `cus` CUs:
@@ -735,8 +744,12 @@ int jq_legal_dense_host(jq_env *e, const int8_t *acting, int32_t *counts, int32_
     const hipStream_t s = strm(stream);
     std::lock_guard<std::mutex> lk(e->io.mu);
     HostIo &io = e->io;
-    // acting | counts | ids: the ids of an average position and half again come
-    // with the first copy, the rest (if any) with a second one
+    // acting | counts | ids: the ids of an average position (42 to 45 in play) and
+    // half again come with the first copy, the rest (if any) with a second one,
+    // which costs its own wait. us of the call at a mean of 44 ids, share 32 / 48 /
+    // 64 / 96 / 128: 64 games 46 / 34 / 34 / 41 / 41, 1,024 76 / 65 / 66 / 68 / 70,
+    // 8,192 260 / 235 / 244 / 263 / 281; 48 would fall short as soon as a batch's
+    // mean passes it.
     const size_t c_off = (n + 15) & ~(size_t)15, v_off = c_off + 4 * n;
     const size_t guess = std::min((size_t)values_capacity, 64 * n);
     if ((rc = host_io_room(io, v_off + 4 * guess, n)) != 0) return rc;
@@ -1235,7 +1248,7 @@ int jq_history_reconstruct_noalloc(jq_history *h, const int64_t *flat, const int
     if (!h) return fail(JQ_E_ARG, "null history");
     if (batch <= 0) return fail(JQ_E_ARG, "cannot reconstruct an empty history minibatch");
     if (batch > JQ_NOALLOC_MAX_ROWS)
-        return fail(JQ_E_ARG, "batch %d exceeds the %d rows jq_history_reconstruct_noalloc holds", batch,
+        return fail(JQ_E_ARG, "batch %d exceeds the %d rows jq_history_reconstruct_noalloc takes", batch,
                     JQ_NOALLOC_MAX_ROWS);
     return history_rebuild(h, flat, observer, batch, fmt, spatial, aux, global, JQ_OBS_F32, mask_words, mask_bool,
                            stream);

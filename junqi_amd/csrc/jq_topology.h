@@ -45,7 +45,10 @@ struct Tables {
     int8_t localidx[NC];          // slot index in the owner's rectangle or -1
     // compact-cell forms for bitboard move generation (129-bit sets, bit c =
     // compact cell c; compact order is flat order, so a straight run's cells
-    // rise (+x, +y) or fall (-x, -y) in compact index)
+    // rise (+x, +y) or fall (-x, -y) in compact index). On the device only railc
+    // and campm are read; MoveTables is derived from adjm, raym and the curve
+    // runs on the host, and adjc, crayc, railidxc, onm, railm and shm serve
+    // inspection
     alignas(8) uint8_t adjc[NONB][8];     // road neighbours then camp diagonals, compact (0xFF none)
     uint64_t adjm[NONB][2][3];            // adjc[c][4h .. 4h + 3] as a 129-bit set, h = 0, 1
     uint64_t raym[NRAIL][4][3];           // straight runs (+x, -x, +y, -y) as compact masks

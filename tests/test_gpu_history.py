@@ -83,7 +83,7 @@ def test_history_reconstructs_observations_and_masks(jq):
     for b, p in enumerate(picks):
         assert np.array_equal(sb[b].view(torch.int16).cpu().numpy().view(np.uint16), _bf16_rne(want[p][0])), p
     assert np.array_equal(mb.cpu().numpy(), mask)
-    # a smaller batch after a larger one reuses the scratch rows
+    # a smaller batch after a larger one
     s2, g2, m2 = hist.reconstruct(flat[:3].flip(0), obs[:3].flip(0), dtype=torch.float32)
     for b, p in enumerate(reversed(picks[:3])):
         assert np.array_equal(s2[b].cpu().numpy().view(np.uint32), want[p][0].view(np.uint32)), p
