@@ -162,7 +162,8 @@ def cpu_baseline(envs: int, seconds: float, sampler: int, obs: bool, seed: int) 
 OBS_TIMED_EVERY = 8   # observation launches timed with events: every 8th step of the timed region
 
 # device kernel that writes the observation rows, per output format
-OBS_KERNEL = {"f32": "jq::k_observe<0, false>", "bf16": "jq::k_observe<1, false>", "u8": "jq::k_observe_u8_persist"}
+OBS_KERNEL = {"f32": "jq::k_observe<0, false, false>", "bf16": "jq::k_observe<1, false, false>",
+              "u8": "jq::k_observe_u8_persist"}
 
 
 def measured_traffic(kernel: str, games: int):
